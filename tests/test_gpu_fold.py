@@ -1,0 +1,106 @@
+"""GPU parity of the reflection-folded FP64 form at the edges of its tiles.
+
+The folded kernel has an instance per row count of a parity (q and dimension),
+two tile widths and unequal parities for odd q.  Values are random, so nothing
+but the symmetry that the form relies on holds; the sizes are the smallest and
+largest of each instance and those past the last one (the general form).
+
+Tolerance: FP64 sums of at most 27 x 1024 products against FP64 sums of the
+same products in another order; their rounding is about
+sqrt(27648) * 1.1e-16 = 2e-14 of the result's size and 3e-12 at the very worst,
+so 1e-12 as for the other FP64 tests.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import list1_ref, orbit_ref
+from tests.gpu_helpers import adaptive, rel_errors
+from tests.test_gpu_plan import _sub_tree
+from volumential_amd import orbit, tree as vtree
+from volumential_amd.kernels import HelmholtzKernel, LaplaceKernel
+from volumential_amd.table import NearFieldInteractionTable
+from volumential_amd.wrangler import NearFieldWrangler
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-12
+
+
+def _table(dim, q, cplx, extent=2.0):
+    m = orbit.build_case_metadata(dim, q)
+    reps = orbit.enumerate_representatives(m)
+    rng = np.random.default_rng(100 * dim + q)
+    v = rng.standard_normal(reps.size)
+    if cplx:
+        v = v + 1j * rng.standard_normal(reps.size)
+    kernel = HelmholtzKernel(dim, 3.0) if cplx else LaplaceKernel(dim)
+    t = NearFieldInteractionTable(q, dim, kernel, source_box_extent=extent)
+    t.build_normalizer_table()
+    t.set_reduced_table_data(reps, v)
+    return t
+
+
+def _case(dim, q, cplx, uniform_level, n_rhs, seed):
+    """Tree with permuted node ids of which every third box is no target."""
+    extent = 2.0
+    if uniform_level is None:
+        tr = adaptive(dim, q, max_level=3)
+    else:
+        tr = vtree.uniform_tree(dim, q, uniform_level)
+        if cplx:
+            extent = tr.root_extent / 2**uniform_level
+    rng = np.random.default_rng(seed)
+    tr.local_ids = np.concatenate(
+        [rng.permutation(tr.n_q_points) for _ in range(tr.nboxes)]).astype(np.int32)
+    n_tgt = np.asarray(tr.target_boxes).size
+    tr = _sub_tree(tr, np.flatnonzero(np.arange(n_tgt) % 3 != 1))
+    f = rng.standard_normal((n_rhs, tr.n_points))
+    if cplx:
+        f = f + 1j * rng.standard_normal(f.shape)
+    return tr, _table(dim, q, cplx, extent), f
+
+
+def _check(tr, table, f, cplx, pick):
+    w = NearFieldWrangler(tr, table)
+    pot, _ = w.eval_direct_plan(tr.target_boxes, tr.neighbor_source_boxes_starts,
+                                tr.neighbor_source_boxes_lists, torch.as_tensor(f, device="cuda"),
+                                form="f64")
+    got = pot[0].cpu().numpy()[pick]
+    meta = orbit_ref.case_metadata(tr.dim, tr.quad_order)
+    nm = np.stack([table.mode_normalizers])
+    tsl = int(round(np.log2(tr.root_extent / table.source_box_extent)))
+    ref = list1_ref.near_field_from_tree(
+        tr, np.stack([table.compact_values()]), nm.astype(np.complex128) if cplx else nm, meta,
+        f[pick], mode="fixed" if cplx else "canonical", scaling_power=0 if cplx else 2,
+        log_displacement=tr.dim == 2 and not cplx, table_root_extent=table.source_box_extent,
+        table_starting_level=tsl)
+    l2, linf = rel_errors(got, ref)
+    assert l2 <= TOL and linf <= TOL, (l2, linf)
+
+
+@pytest.mark.parametrize("n_rhs", [1, 5])
+@pytest.mark.parametrize("dim,q", [(2, q) for q in (2, 3, 4, 5, 8, 10, 11)] +
+                         [(3, q) for q in (2, 3, 4, 5, 7, 8)])
+def test_fold_graded(cuda, dim, q, n_rhs):
+    print(f"case: fold graded {dim}D q={q} R={n_rhs}", flush=True)
+    tr, table, f = _case(dim, q, False, None, n_rhs, q)
+    _check(tr, table, f, False, list(range(n_rhs)))
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("dim,q", [(2, 2), (2, 5), (2, 8), (3, 2), (3, 3), (3, 5), (3, 6)])
+def test_fold_many_densities(cuda, dim, q, cplx):
+    """Enough tiles for the wide ones; 192 densities are three passes of 64."""
+    print(f"case: fold {dim}D q={q} R=192 {'complex' if cplx else 'real'}", flush=True)
+    tr, table, f = _case(dim, q, cplx, 4 if dim == 2 else 2, 192, q)
+    _check(tr, table, f, cplx, [0, 63, 64, 191])
+
+
+@pytest.mark.parametrize("n_rhs", [7, 33])
+def test_fold_ragged_densities(cuda, n_rhs):
+    """Tiles whose columns are not all in use (2D q = 3, 1024 boxes)."""
+    print(f"case: fold 2D q=3 R={n_rhs}", flush=True)
+    tr, table, f = _case(2, 3, False, 5, n_rhs, 3)
+    _check(tr, table, f, False, list(range(n_rhs)))

@@ -45,7 +45,7 @@ def _hipcc() -> str:
     return exe
 
 
-def build(verbose: bool = False, jobs: int = 4) -> Path:
+def build(verbose: bool = False, jobs: int = 8) -> Path:
     hipcc = _hipcc()
     OBJ.mkdir(exist_ok=True)
     sources = sorted(CSRC.glob("*.hip"))

@@ -26,12 +26,15 @@
 #include <cmath>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <numeric>
 #include <string>
 #include <type_traits>
+#include <unordered_map>
 #include <vector>
 
+#include "fold.h"
 #include "internal.h"
 #include "split_series.h"
 
@@ -1155,6 +1158,13 @@ struct TileSchedule {
   int64_t n_steps = 0;
 };
 
+// Tiles of the folded FP64 form: B boxes each, steps = list-1 classes (fold.h).
+struct FoldSchedule {
+  int B = 0, n_tiles = 0;
+  int64_t n_steps = 0;
+  DevBuf tile_step_start, tile_chunk_start, tile_boxes, chunks, step_src;
+};
+
 // The dynamic-LDS limit of a tile kernel is raised to the full 160 KiB (less
 // the kernel's static LDS, the phase word's) once per device (bit d of
 // `done`), so later launches -- including ones recorded into a HIP graph --
@@ -1252,6 +1262,9 @@ struct vl1_plan {
   DevBuf pt_class, alpha_lut;
   bool stream_colmax = false;
   std::map<int, TileSchedule*> schedules;  // by 2 Rc + (Morton-only order)
+  FoldPlan* fold = nullptr;                // folded FP64 form (null: the dense one)
+  std::map<int, FoldSchedule*> fold_schedules;  // by 2 B + (Morton-only order)
+  int fold_rc = 1;  // densities per 64 columns of the first folded evaluation (statistics)
   std::map<int, int> tuned;                 // variant by (form, slices, Rc), from vl1_plan_tune
   int forced_variant = -1;                  // candidate under test in vl1_plan_tune
   // staging buffers (grown on demand).  A buffer that is outgrown is
@@ -1263,6 +1276,8 @@ struct vl1_plan {
   int staged_form = -1, staged_rhs = 0, staged_slices = -1;
   ~vl1_plan() {
     for (auto& kv : schedules) delete kv.second;
+    for (auto& kv : fold_schedules) delete kv.second;
+    delete fold;
     for (auto& kv : A_by_slices) delete kv.second;
     for (auto& kv : A8_by_slices) delete kv.second;
     for (DevBuf* b : retired) delete b;
@@ -1402,6 +1417,162 @@ static int build_schedule(vl1_plan* pl, int Rc, bool morton_only, TileSchedule**
   return VL1_OK;
 }
 
+// Each target's classes; a repeated source of one class slot counts once, as
+// in the dense form's schedule.
+static void fold_targets(vl1_plan* pl) {
+  FoldPlan& f = *pl->fold;
+  if (!f.start.empty()) return;
+  const int np = f.d.np;
+  std::vector<std::pair<int, int64_t>> ent;  // (class x np + slot, pair)
+  f.start.assign(pl->n_tgt + 1, 0);
+  int64_t k = 0;
+  for (int t = 0; t < pl->n_tgt; ++t) {
+    ent.clear();
+    for (; k < pl->n_pairs && pl->pair_tgt[k] == t; ++k) {
+      const int b = pl->pair_block[k];
+      ent.push_back({f.key_cls[b] * np + f.key_slot[b], k});
+    }
+    std::sort(ent.begin(), ent.end());
+    int last = -1;
+    for (const auto& e : ent) {
+      const int c = e.first / np, j = e.first % np;
+      if (c != last) {
+        f.cls.push_back(c);
+        f.src.resize(f.src.size() + np, -1);
+        last = c;
+      }
+      int32_t& slot = f.src[f.src.size() - np + j];
+      if (slot < 0) slot = pl->pair_src[e.second];
+    }
+    f.start[t + 1] = (int32_t)f.cls.size();
+  }
+}
+
+// Tiles of the folded form: targets in the order of their class lists (then
+// Morton), so that a tile's union of classes, and with it its chunks, stays
+// near each box's own -- graded 3D tree of 14246 boxes, 380 different lists,
+// tiles of 32: 20893 chunks and 127 in the longest tile, against 31106 and 271
+// with the lists in hash order.  Tiles are then dealt out longest first, runs of
+// equal length in eighths to the XCDs (workgroup i runs on XCD i % 8), which
+// keeps neighbours in one L2.
+static int build_fold_schedule(vl1_plan* pl, int B, bool morton_only, FoldSchedule** out,
+                               hipStream_t s) {
+  const int key = B * 2 + (morton_only ? 1 : 0);
+  auto it = pl->fold_schedules.find(key);
+  if (it != pl->fold_schedules.end()) {
+    *out = it->second;
+    return VL1_OK;
+  }
+  fold_targets(pl);
+  const FoldPlan& fp = *pl->fold;
+  const int np = fp.d.np;
+  std::vector<int> rank(pl->n_tgt, 0);  // of a target's class list among the different ones
+  if (B > 1 && !morton_only) {
+    std::unordered_map<uint64_t, int> group_of;
+    std::vector<int> first;  // a target with the group's list
+    for (int i = 0; i < pl->n_tgt; ++i) {
+      uint64_t h = 1469598103934665603ull;  // FNV-1a over the class ids
+      for (int e = fp.start[i]; e < fp.start[i + 1]; ++e) {
+        h ^= (uint64_t)(uint32_t)fp.cls[e];
+        h *= 1099511628211ull;
+      }
+      const auto g = group_of.emplace(h, (int)first.size());
+      if (g.second) first.push_back(i);
+      rank[i] = g.first->second;
+    }
+    std::vector<int> by(first.size()), pos(first.size());
+    std::iota(by.begin(), by.end(), 0);
+    std::sort(by.begin(), by.end(), [&](int a, int b) {
+      const int32_t* c = fp.cls.data();
+      const int s0 = fp.start[first[a]], e0 = fp.start[first[a] + 1];
+      const int s1 = fp.start[first[b]], e1 = fp.start[first[b] + 1];
+      return std::lexicographical_compare(c + s0, c + e0, c + s1, c + e1);
+    });
+    for (size_t k = 0; k < by.size(); ++k) pos[by[k]] = (int)k;
+    for (int& r : rank) r = pos[r];
+  }
+  std::vector<int> order(pl->n_tgt);
+  std::iota(order.begin(), order.end(), 0);
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+    if (rank[a] != rank[b]) return rank[a] < rank[b];
+    return pl->tgt_morton[a] < pl->tgt_morton[b];
+  });
+  auto sch = new FoldSchedule();
+  sch->B = B;
+  sch->n_tiles = (pl->n_tgt + B - 1) / B;
+  // classes and chunks of the tiles, then their places
+  std::vector<int32_t> classes;
+  std::vector<size_t> cls_at(sch->n_tiles + 1, 0);
+  std::vector<int> n_chunks(sch->n_tiles, 0), place(sch->n_tiles), by_len(sch->n_tiles);
+  for (int t = 0; t < sch->n_tiles; ++t) {
+    const size_t c0 = classes.size();
+    for (int b = t * B; b < std::min((t + 1) * B, pl->n_tgt); ++b)
+      classes.insert(classes.end(), fp.cls.begin() + fp.start[order[b]],
+                     fp.cls.begin() + fp.start[order[b] + 1]);
+    std::sort(classes.begin() + c0, classes.end());
+    classes.erase(std::unique(classes.begin() + c0, classes.end()), classes.end());
+    cls_at[t + 1] = classes.size();
+    for (size_t k = c0; k < classes.size(); ++k)
+      n_chunks[t] += fold_chunks(fp.d, __builtin_popcount(fp.zmask[classes[k]]));
+    by_len[t] = t;
+  }
+  std::stable_sort(by_len.begin(), by_len.end(),
+                   [&](int a, int b) { return n_chunks[a] > n_chunks[b]; });
+  for (int i = 0; i < sch->n_tiles;) {
+    int j = i;
+    while (j < sch->n_tiles && n_chunks[by_len[j]] == n_chunks[by_len[i]]) ++j;
+    int k = i;
+    for (int x = 0; x < 8; ++x)  // the places of [i, j) on XCD x
+      for (int at = i + (x - i % 8 + 8) % 8; at < j; at += 8) place[at] = by_len[k++];
+    i = j;
+  }
+  std::vector<int32_t> tss(sch->n_tiles + 1, 0), tcs(sch->n_tiles + 1, 0);
+  std::vector<int32_t> tboxes((size_t)sch->n_tiles * B, -1), src;
+  std::vector<uint32_t> words;
+  src.reserve(classes.size() * B * np + (size_t)kFoldPad * B * np);
+  for (int t = 0; t < sch->n_tiles; ++t) {
+    const int first = place[t] * B, n = std::min(B, pl->n_tgt - first);
+    const int32_t* cl = classes.data() + cls_at[place[t]];
+    const size_t n_cl = cls_at[place[t] + 1] - cls_at[place[t]];
+    const size_t base = src.size();
+    src.resize(base + n_cl * B * np, pl->nboxes);  // nboxes: the zero box
+    for (int b = 0; b < n; ++b) {
+      const int tg = order[first + b];
+      tboxes[(size_t)t * B + b] = pl->tgt_boxes[tg];
+      size_t k = 0;
+      for (int e = fp.start[tg]; e < fp.start[tg + 1]; ++e) {
+        while (cl[k] != fp.cls[e]) ++k;
+        int32_t* q = src.data() + base + (k * B + b) * np;
+        for (int j = 0; j < np; ++j)
+          if (fp.src[(size_t)e * np + j] >= 0) q[j] = fp.src[(size_t)e * np + j];
+      }
+    }
+    for (size_t i = 0; i < n_cl; ++i) {
+      const int z = fp.zmask[cl[i]], m = __builtin_popcount(z);
+      for (int k = 0; k < fold_chunks(fp.d, m); ++k)
+        words.push_back(fold_chunk_word(cl[i], z, m, k, k == 0));
+    }
+    tss[t + 1] = tss[t] + (int32_t)n_cl;
+    tcs[t + 1] = (int32_t)words.size();
+  }
+  sch->n_steps = tss.back();
+  // the kernel prefetches past a tile's end
+  words.resize(words.size() + kFoldPad, fold_chunk_word(0, 0, 0, 0, true));
+  src.resize(src.size() + (size_t)kFoldPad * B * np, pl->nboxes);
+  hipError_t e = upload(sch->tile_step_start, tss.data(), tss.size() * 4, s);
+  if (e == hipSuccess) e = upload(sch->tile_boxes, tboxes.data(), tboxes.size() * 4, s);
+  if (e == hipSuccess) e = upload(sch->tile_chunk_start, tcs.data(), tcs.size() * 4, s);
+  if (e == hipSuccess) e = upload(sch->chunks, words.data(), words.size() * 4, s);
+  if (e == hipSuccess) e = upload(sch->step_src, src.data(), src.size() * 4, s);
+  if (e != hipSuccess) {
+    delete sch;
+    return fail(VL1_E_HIP, std::string("plan schedule upload: ") + hipGetErrorString(e));
+  }
+  pl->fold_schedules[key] = sch;
+  *out = sch;
+  return VL1_OK;
+}
+
 static int ensure_A(vl1_plan* pl, int S, hipStream_t s) {
   if (pl->A(S)) return VL1_OK;
   auto A = new DevBuf();
@@ -1469,6 +1640,190 @@ static int ensure_A8(vl1_plan* pl, int S, hipStream_t s) {
   }
   pl->A8_by_slices[S] = A;
   return VL1_OK;
+}
+
+// (case, table level) blocks to expand; alpha, disp, h: Helmholtz split only.
+struct BlockList {
+  std::vector<int32_t> cse, lev;
+  std::vector<double> alpha, disp, h;
+};
+
+// M [blocks x n_rg][MP][KP] of the listed blocks.
+static hipError_t expand_plan_blocks(const vl1_payload* pay, const vl1_plan* pl,
+                                     const vl1_helmholtz_split_blocks* sp, double H,
+                                     const BlockList& bl, int MP, int KP, int n_rg, int rg_size,
+                                     DevBuf& M, hipStream_t s) {
+  const int dim = pl->dim, n = pl->n, n_keys = (int)bl.cse.size(), n_blocks = n_keys * n_rg;
+  DevBuf dcase, dlev, dperm, dsign, dgroup;
+  hipError_t e = upload(dcase, bl.cse.data(), bl.cse.size() * 4, s);
+  if (e == hipSuccess) e = upload(dlev, bl.lev.data(), bl.lev.size() * 4, s);
+  if (e == hipSuccess) e = upload(dperm, pay->perm.data(), pay->perm.size(), s);
+  if (e == hipSuccess) e = upload(dsign, pay->sign.data(), pay->sign.size(), s);
+  if (e == hipSuccess) e = upload(dgroup, pay->group.data(), pay->group.size(), s);
+  if (e == hipSuccess) e = M.alloc((size_t)n_blocks * MP * KP * sizeof(double));
+  if (e == hipSuccess && sp) {
+    std::vector<int32_t> vecs((size_t)pay->n_cases * dim);
+    for (size_t k = 0; k < vecs.size(); ++k) vecs[k] = sp->case_vecs[k];
+    const bool deriv = sp->deriv_kind != VL1_SPLIT_DERIV_NONE;
+    const std::complex<double> kk(sp->k_re, sp->k_im);
+    const int order = sp->split_order < 1 ? 1 : sp->split_order;
+    std::vector<double> coef = deriv ? split_derivative_coefficients(dim, kk, sp->series_nmax, order)
+                                     : split_coefficients(dim, kk, sp->series_nmax, order);
+    if (coef.empty()) coef.assign(2, 0.0);  // 3D derivative with one term: R' = 0
+    DevBuf dal, ddi, dh, dvec, dun, duw, dco, dext;
+    e = upload(dal, bl.alpha.data(), bl.alpha.size() * 8, s);
+    if (e == hipSuccess) e = upload(ddi, bl.disp.data(), bl.disp.size() * 8, s);
+    if (e == hipSuccess) e = upload(dh, bl.h.data(), bl.h.size() * 8, s);
+    if (e == hipSuccess) e = upload(dvec, vecs.data(), vecs.size() * 4, s);
+    if (e == hipSuccess) e = upload(dun, sp->unit_nodes, (size_t)pay->q * 8, s);
+    if (e == hipSuccess) e = upload(duw, sp->unit_weights, (size_t)pay->q * 8, s);
+    if (e == hipSuccess) e = upload(dco, coef.data(), coef.size() * 8, s);
+    if (e == hipSuccess && (order > 1 || sp->smooth_order > 0)) {
+      // per (case, level) block -- n_keys of them, before the cut into
+      // row groups -- and (target, source) the remainder of order m, the
+      // terms' tables and the 2D log parts, complex
+      DevBuf dtt, dtp, dtl, dtc, dsn, dsw, dsi;
+      const int nt = sp->n_terms, ms = sp->smooth_order;
+      e = dext.alloc((size_t)n_keys * n * n * sizeof(double2));
+      if (e == hipSuccess && nt > 0) {
+        e = upload(dtt, sp->term_tables, (size_t)nt * pay->n_entries * 8, s);
+        if (e == hipSuccess) e = upload(dtp, sp->term_powers, (size_t)nt * 4, s);
+        if (e == hipSuccess) e = upload(dtl, sp->term_logs, (size_t)nt * 4, s);
+        if (e == hipSuccess) e = upload(dtc, sp->term_coefs, (size_t)nt * 16, s);
+      }
+      if (e == hipSuccess && ms > 0) {
+        e = upload(dsn, sp->smooth_nodes, (size_t)ms * 8, s);
+        if (e == hipSuccess) e = upload(dsw, sp->smooth_weights, (size_t)ms * 8, s);
+        if (e == hipSuccess) e = upload(dsi, sp->smooth_interp, (size_t)ms * pay->q * 8, s);
+      }
+      if (e == hipSuccess) {
+        const int64_t total = (int64_t)n_keys * n * n;
+        const int grid = (int)std::min<int64_t>((total + 255) / 256, 65536);
+        auto kern = dim == 2 ? split_extra_kernel<2> : split_extra_kernel<3>;
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, s, pay->q, n, n_keys,
+                           dcase.as<int32_t>(), dh.as<double>(), H, dvec.as<int32_t>(),
+                           dperm.as<uint8_t>(), dsign.as<int8_t>(), dgroup.as<uint8_t>(),
+                           pay->ranks.as<uint16_t>(), pay->offs.as<int32_t>(), pay->n_entries,
+                           dun.as<double>(), duw.as<double>(), dco.as<double>(),
+                           sp->series_nmax, ms, dsn.as<double>(), dsw.as<double>(),
+                           dsi.as<double>(), nt, dtt.as<double>(), dtp.as<int32_t>(),
+                           dtl.as<int32_t>(), dtc.as<double>(), deriv ? sp->deriv_axis : -1,
+                           sp->deriv_kind == VL1_SPLIT_DERIV_SOURCE ? -1.0 : 1.0,
+                           pay->sign_mask, dext.as<double2>());
+        e = hipGetLastError();
+      }
+      if (e == hipSuccess) e = hipStreamSynchronize(s);  // before the uploads are freed
+    }
+    if (e == hipSuccess) {
+      const int64_t total = (int64_t)n_blocks * MP * KP;
+      const int grid = (int)std::min<int64_t>((total + 255) / 256, 65536);
+      hipLaunchKernelGGL(expand_split_blocks_kernel, dim3(grid), dim3(256), 0, s, dim, pay->q, n,
+                         pay->sign_mask, deriv ? sp->deriv_axis : -1,
+                         sp->deriv_kind == VL1_SPLIT_DERIV_SOURCE ? -1.0 : 1.0, MP, KP,
+                         n_blocks, n_rg, rg_size, dcase.as<int32_t>(),
+                         dlev.as<int32_t>(), pay->n_entries, dal.as<double>(),
+                         ddi.as<double>(), dh.as<double>(), dvec.as<int32_t>(),
+                         dperm.as<uint8_t>(), dsign.as<int8_t>(), dgroup.as<uint8_t>(),
+                         pay->ranks.as<uint16_t>(), pay->offs.as<int32_t>(),
+                         pay->table.as<double>(), pay->nmlz.as<double>(), dun.as<double>(),
+                         duw.as<double>(), dco.as<double>(), sp->series_nmax,
+                         dext.ptr ? dext.as<double2>() : nullptr, M.as<double>());
+      e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(s);  // before the uploads are freed
+  } else if (e == hipSuccess && pay->dense_kind) {
+    const int64_t total = (int64_t)n_blocks * MP * KP;
+    const int grid = (int)std::min<int64_t>((total + 255) / 256, 65536);
+    hipLaunchKernelGGL(expand_dense_blocks_kernel, dim3(grid), dim3(256), 0, s, n, pay->n_cases,
+                       pl->cplx, MP, KP, n_blocks, n_rg, rg_size,
+                       dcase.as<int32_t>(), dlev.as<int32_t>(), pay->dense.as<double>(),
+                       M.as<double>());
+    e = hipGetLastError();
+  } else if (e == hipSuccess) {
+    const int64_t total = (int64_t)n_blocks * MP * KP;
+    const int grid = (int)std::min<int64_t>((total + 255) / 256, 65536);
+    hipLaunchKernelGGL(expand_blocks_kernel, dim3(grid), dim3(256), 0, s, dim, pay->q, n, pl->cplx,
+                       pay->sign_mask, MP, KP, n_blocks, n_rg, rg_size,
+                       dcase.as<int32_t>(), dlev.as<int32_t>(),
+                       dperm.as<uint8_t>(), dsign.as<int8_t>(), dgroup.as<uint8_t>(),
+                       pay->ranks.as<uint16_t>(), pay->offs.as<int32_t>(), pay->table.as<double>(),
+                       pay->n_entries, M.as<double>());
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) e = hipStreamSynchronize(s);  // before the uploads are freed
+  return e;
+}
+
+// Folded FP64 form of a plan over an arithmetic-orbit payload, first half:
+// the classes of the plan's keys under reflections of the folded axes.  A class
+// representative (all folded components positive) that is no key itself is
+// appended to `keys`.  Null for boxes the tile kernel does not take and trees
+// beyond its 32-bit byte offsets: the dense form runs.
+static std::unique_ptr<FoldPlan> fold_classes(const vl1_plan* pl, const vl1_payload* pay, bool split,
+                                              const std::vector<int64_t>& key_vid, BlockList& keys) {
+  const int dim = pl->dim;
+  auto f = std::unique_ptr<FoldPlan>(new FoldPlan());
+  if (!fold_layout(*f, dim, pay->q, pl->cplx, (uint32_t)pay->sign_mask)) return nullptr;
+  if ((double)(pl->nboxes + 1) * f->d.kg * 32.0 >= 4294967296.0) return nullptr;
+  // blocks of a level: the table level, or the split's source level
+  auto level_key = [&](int k) {
+    int64_t l = keys.lev[k];
+    if (split) std::memcpy(&l, &keys.h[k], sizeof(l));
+    return l;
+  };
+  std::map<std::pair<int64_t, int64_t>, int> cls_of, key_of;
+  for (int k = 0; k < pl->n_keys; ++k) key_of[{key_vid[k], level_key(k)}] = k;
+  for (int k = 0; k < pl->n_keys; ++k) {
+    int64_t code = key_vid[k], rep = 0, unit = 1;
+    int flips = 0, zmask = 0;
+    for (int a = dim - 1; a >= 0; --a, unit *= 13, code /= 13) {
+      int v = (int)(code % 13) - 6;
+      if (a < f->d.nf && v != 0) {
+        zmask |= 1 << a;
+        if (v < 0) flips |= 1 << a;
+        v = std::abs(v);
+      }
+      rep += (v + 6) * unit;
+    }
+    auto ins = cls_of.insert({{rep, level_key(k)}, f->n_cls});
+    if (ins.second) {
+      auto at = key_of.find({rep, level_key(k)});
+      int blk = at != key_of.end() ? at->second : (int)keys.cse.size();
+      if (at == key_of.end()) {
+        const int64_t cid = pay->case_indices[rep];
+        if (cid < 0 || cid >= pay->n_cases) return nullptr;
+        keys.cse.push_back((int32_t)cid);
+        keys.lev.push_back(keys.lev[k]);
+        if (split) {
+          keys.alpha.push_back(keys.alpha[k]);
+          keys.disp.push_back(keys.disp[k]);
+          keys.h.push_back(keys.h[k]);
+        }
+      }
+      f->rep_blk.push_back(blk);
+      f->zmask.push_back((uint8_t)zmask);
+      ++f->n_cls;
+    }
+    f->key_cls.push_back(ins.first->second);
+    f->key_flips.push_back(flips);
+    int slot = 0, bit = 0;  // the sign bits of the nonzero axes, compressed
+    for (int a = 0; a < f->d.nf; ++a)
+      if ((zmask >> a) & 1) slot |= ((flips >> a) & 1) << bit++;
+    f->key_slot.push_back(slot);
+  }
+  return f;
+}
+
+// Second half, after the blocks are expanded: the representatives' blocks in
+// the folded basis, kept unless a block is not the reflection of its class's
+// representative (descriptors without the reflection symmetry of a list-1
+// table).
+static hipError_t fold_tables(vl1_plan* pl, std::unique_ptr<FoldPlan> f, int q, hipStream_t s) {
+  int32_t flag = 0;
+  const hipError_t e = fold_build_launch(*f, pl->dim, q, pl->M.as<double>(), pl->MP, pl->KP, pl->n_rg,
+                                         pl->rg_size, &flag, s);
+  if (e == hipSuccess && !flag) pl->fold = f.release();
+  return e;
 }
 
 static int plan_create(vl1_plan** out, const vl1_payload* pay, const vl1_plan_desc* d,
@@ -1646,6 +2001,8 @@ static int plan_create(vl1_plan** out, const vl1_payload* pay, const vl1_plan_de
   const int64_t n_pairs = d->nbr_starts[d->n_tgt_boxes];
   pl->n_pairs = n_pairs;
   std::map<std::pair<int, int>, int> blk_of;
+  std::vector<int64_t> key_vid;  // per key the case code of its pairs
+  bool one_vid = true;           // ... which all pairs of the key share
   const double H = d->table_root_extent;
   {
     double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
@@ -1718,6 +2075,7 @@ static int plan_create(vl1_plan** out, const vl1_payload* pay, const vl1_plan_de
       if (f == blk_of.end()) {
         blk = (int)pl->blk_case.size();
         blk_of[key] = blk;
+        key_vid.push_back(vid);
         pl->blk_case.push_back(cid);
         pl->blk_lev.push_back(lev);
         if (split) {
@@ -1727,6 +2085,7 @@ static int plan_create(vl1_plan** out, const vl1_payload* pay, const vl1_plan_de
         }
       } else {
         blk = f->second;
+        one_vid = one_vid && key_vid[blk] == vid;
       }
       pl->pair_tgt.push_back(i);
       pl->pair_src.push_back(sb);
@@ -1801,105 +2160,14 @@ static int plan_create(vl1_plan** out, const vl1_payload* pay, const vl1_plan_de
   if (e == hipSuccess) e = upload(pl->box_starts, bstarts.data(), bstarts.size() * 4, s);
   if (e == hipSuccess) e = upload(pl->box_alpha, balpha.data(), balpha.size() * 8, s);
   if (e == hipSuccess) e = upload(pl->box_disp, bdisp.data(), bdisp.size() * 8, s);
-  DevBuf dcase, dlev, dperm, dsign, dgroup;
   if (e == hipSuccess && pl->n_blocks > 0) {
-    e = upload(dcase, pl->blk_case.data(), pl->blk_case.size() * 4, s);
-    if (e == hipSuccess) e = upload(dlev, pl->blk_lev.data(), pl->blk_lev.size() * 4, s);
-    if (e == hipSuccess) e = upload(dperm, pay->perm.data(), pay->perm.size(), s);
-    if (e == hipSuccess) e = upload(dsign, pay->sign.data(), pay->sign.size(), s);
-    if (e == hipSuccess) e = upload(dgroup, pay->group.data(), pay->group.size(), s);
-    if (e == hipSuccess) e = pl->M.alloc((size_t)pl->n_blocks * pl->MP * pl->KP * sizeof(double));
-    if (e == hipSuccess && split) {
-      std::vector<int32_t> vecs((size_t)pay->n_cases * dim);
-      for (size_t k = 0; k < vecs.size(); ++k) vecs[k] = sp->case_vecs[k];
-      const bool deriv = sp->deriv_kind != VL1_SPLIT_DERIV_NONE;
-      const std::complex<double> kk(sp->k_re, sp->k_im);
-      const int order = sp->split_order < 1 ? 1 : sp->split_order;
-      std::vector<double> coef = deriv ? split_derivative_coefficients(dim, kk, sp->series_nmax, order)
-                                       : split_coefficients(dim, kk, sp->series_nmax, order);
-      if (coef.empty()) coef.assign(2, 0.0);  // 3D derivative with one term: R' = 0
-      DevBuf dal, ddi, dh, dvec, dun, duw, dco, dext;
-      e = upload(dal, pl->blk_alpha.data(), pl->blk_alpha.size() * 8, s);
-      if (e == hipSuccess) e = upload(ddi, pl->blk_disp.data(), pl->blk_disp.size() * 8, s);
-      if (e == hipSuccess) e = upload(dh, pl->blk_h.data(), pl->blk_h.size() * 8, s);
-      if (e == hipSuccess) e = upload(dvec, vecs.data(), vecs.size() * 4, s);
-      if (e == hipSuccess) e = upload(dun, sp->unit_nodes, (size_t)pay->q * 8, s);
-      if (e == hipSuccess) e = upload(duw, sp->unit_weights, (size_t)pay->q * 8, s);
-      if (e == hipSuccess) e = upload(dco, coef.data(), coef.size() * 8, s);
-      if (e == hipSuccess && (order > 1 || sp->smooth_order > 0)) {
-        // per (case, level) block -- n_keys of them, before the cut into
-        // row groups -- and (target, source) the remainder of order m, the
-        // terms' tables and the 2D log parts, complex
-        DevBuf dtt, dtp, dtl, dtc, dsn, dsw, dsi;
-        const int nt = sp->n_terms, ms = sp->smooth_order;
-        e = dext.alloc((size_t)pl->n_keys * n * n * sizeof(double2));
-        if (e == hipSuccess && nt > 0) {
-          e = upload(dtt, sp->term_tables, (size_t)nt * pay->n_entries * 8, s);
-          if (e == hipSuccess) e = upload(dtp, sp->term_powers, (size_t)nt * 4, s);
-          if (e == hipSuccess) e = upload(dtl, sp->term_logs, (size_t)nt * 4, s);
-          if (e == hipSuccess) e = upload(dtc, sp->term_coefs, (size_t)nt * 16, s);
-        }
-        if (e == hipSuccess && ms > 0) {
-          e = upload(dsn, sp->smooth_nodes, (size_t)ms * 8, s);
-          if (e == hipSuccess) e = upload(dsw, sp->smooth_weights, (size_t)ms * 8, s);
-          if (e == hipSuccess) e = upload(dsi, sp->smooth_interp, (size_t)ms * pay->q * 8, s);
-        }
-        if (e == hipSuccess) {
-          const int64_t total = (int64_t)pl->n_keys * n * n;
-          const int grid = (int)std::min<int64_t>((total + 255) / 256, 65536);
-          auto kern = dim == 2 ? split_extra_kernel<2> : split_extra_kernel<3>;
-          hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, s, pay->q, n, pl->n_keys,
-                             dcase.as<int32_t>(), dh.as<double>(), H, dvec.as<int32_t>(),
-                             dperm.as<uint8_t>(), dsign.as<int8_t>(), dgroup.as<uint8_t>(),
-                             pay->ranks.as<uint16_t>(), pay->offs.as<int32_t>(), pay->n_entries,
-                             dun.as<double>(), duw.as<double>(), dco.as<double>(),
-                             sp->series_nmax, ms, dsn.as<double>(), dsw.as<double>(),
-                             dsi.as<double>(), nt, dtt.as<double>(), dtp.as<int32_t>(),
-                             dtl.as<int32_t>(), dtc.as<double>(), deriv ? sp->deriv_axis : -1,
-                             sp->deriv_kind == VL1_SPLIT_DERIV_SOURCE ? -1.0 : 1.0,
-                             pay->sign_mask, dext.as<double2>());
-          e = hipGetLastError();
-        }
-        if (e == hipSuccess) e = hipStreamSynchronize(s);  // before the uploads are freed
-      }
-      if (e == hipSuccess) {
-        const int64_t total = (int64_t)pl->n_blocks * pl->MP * pl->KP;
-        const int grid = (int)std::min<int64_t>((total + 255) / 256, 65536);
-        hipLaunchKernelGGL(expand_split_blocks_kernel, dim3(grid), dim3(256), 0, s, dim, pay->q, n,
-                           pay->sign_mask, deriv ? sp->deriv_axis : -1,
-                           sp->deriv_kind == VL1_SPLIT_DERIV_SOURCE ? -1.0 : 1.0, pl->MP, pl->KP,
-                           pl->n_blocks, pl->n_rg, pl->rg_size, dcase.as<int32_t>(),
-                           dlev.as<int32_t>(), pay->n_entries, dal.as<double>(),
-                           ddi.as<double>(), dh.as<double>(), dvec.as<int32_t>(),
-                           dperm.as<uint8_t>(), dsign.as<int8_t>(), dgroup.as<uint8_t>(),
-                           pay->ranks.as<uint16_t>(), pay->offs.as<int32_t>(),
-                           pay->table.as<double>(), pay->nmlz.as<double>(), dun.as<double>(),
-                           duw.as<double>(), dco.as<double>(), sp->series_nmax,
-                           dext.ptr ? dext.as<double2>() : nullptr, pl->M.as<double>());
-        e = hipGetLastError();
-      }
-      if (e == hipSuccess) e = hipStreamSynchronize(s);  // before the uploads are freed
-    } else if (e == hipSuccess && pay->dense_kind) {
-      const int64_t total = (int64_t)pl->n_blocks * pl->MP * pl->KP;
-      const int grid = (int)std::min<int64_t>((total + 255) / 256, 65536);
-      hipLaunchKernelGGL(expand_dense_blocks_kernel, dim3(grid), dim3(256), 0, s, n, pay->n_cases,
-                         pl->cplx, pl->MP, pl->KP, pl->n_blocks, pl->n_rg, pl->rg_size,
-                         dcase.as<int32_t>(), dlev.as<int32_t>(), pay->dense.as<double>(),
-                         pl->M.as<double>());
-      e = hipGetLastError();
-    } else if (e == hipSuccess) {
-      const int64_t total = (int64_t)pl->n_blocks * pl->MP * pl->KP;
-      const int grid = (int)std::min<int64_t>((total + 255) / 256, 65536);
-      hipLaunchKernelGGL(expand_blocks_kernel, dim3(grid), dim3(256), 0, s, dim, pay->q, n, pl->cplx,
-                         pay->sign_mask, pl->MP, pl->KP, pl->n_blocks, pl->n_rg, pl->rg_size,
-                         dcase.as<int32_t>(), dlev.as<int32_t>(),
-                         dperm.as<uint8_t>(), dsign.as<int8_t>(), dgroup.as<uint8_t>(),
-                         pay->ranks.as<uint16_t>(), pay->offs.as<int32_t>(), pay->table.as<double>(),
-                         pay->n_entries, pl->M.as<double>());
-      e = hipGetLastError();
-    }
-    if (e == hipSuccess) e = pl->MF.alloc(pl->M.bytes);
-    if (e == hipSuccess) {
+    BlockList keys{pl->blk_case, pl->blk_lev, pl->blk_alpha, pl->blk_disp, pl->blk_h};
+    std::unique_ptr<FoldPlan> fold;
+    if (one_vid && !pay->dense_kind) fold = fold_classes(pl, pay, split, key_vid, keys);
+    e = expand_plan_blocks(pay, pl, sp, H, keys, pl->MP, pl->KP, pl->n_rg, pl->rg_size, pl->M, s);
+    if (e == hipSuccess && fold) e = fold_tables(pl, std::move(fold), pay->q, s);
+    if (e == hipSuccess && !pl->fold) e = pl->MF.alloc(pl->M.bytes);
+    if (e == hipSuccess && !pl->fold) {
       const int64_t total = (int64_t)pl->n_blocks * pl->MP * pl->KP;
       const int grid = (int)std::min<int64_t>((total + 255) / 256, 65536);
       hipLaunchKernelGGL(frag_f64_kernel, dim3(grid), dim3(256), 0, s, pl->MP, pl->KP, pl->n_blocks,
@@ -2020,13 +2288,30 @@ static int i8_check_range(const vl1_plan* pl, const TileSchedule* sch, int S) {
   return VL1_OK;
 }
 
+// What one evaluation runs on: the slice count and tile schedule, or the
+// folded form's tiles.
+struct Prepared {
+  int S = 0;
+  TileSchedule* sch = nullptr;
+  FoldSchedule* fold = nullptr;
+  FoldTile tile;
+};
+
+static bool uses_fold(const vl1_plan* pl, int form) { return form == VL1_FORM_F64 && pl->fold; }
+
 // Checks, then builds (allocating) the slice set and tile schedule this
 // evaluation needs if the plan does not hold them yet.
 static int plan_prepare(vl1_plan* pl, int form, int n_rhs, const vl1_split_opts* opts,
-                        hipStream_t s, int* S_out, TileSchedule** sch_out) {
+                        hipStream_t s, Prepared* out) {
   int S = 0;
   int rc = plan_check(pl, form, n_rhs, opts, &S);
   if (rc != VL1_OK) return rc;
+  if (uses_fold(pl, form)) {
+    out->tile = fold_tile(pl->fold->d, pl->n_tgt, n_rhs);
+    const bool morton = (plan_variant(pl, form, S, std::min(n_rhs, kCols)) & kVarMorton) != 0;
+    if (pl->fold_schedules.empty()) pl->fold_rc = std::min(n_rhs, kCols);
+    return build_fold_schedule(pl, out->tile.B, morton, &out->fold, s);
+  }
   if (form == VL1_FORM_SPLIT_BF16) {
     rc = ensure_A(pl, S, s);
     if (rc != VL1_OK) return rc;
@@ -2034,10 +2319,10 @@ static int plan_prepare(vl1_plan* pl, int form, int n_rhs, const vl1_split_opts*
     rc = ensure_A8(pl, S, s);
     if (rc != VL1_OK) return rc;
   }
-  *S_out = S;
+  out->S = S;
   const int Rc = std::min(n_rhs, kCols);
-  rc = build_schedule(pl, Rc, (plan_variant(pl, form, S, Rc) & kVarMorton) != 0, sch_out, s);
-  if (rc == VL1_OK && form == VL1_FORM_SPLIT_I8) rc = i8_check_range(pl, *sch_out, S);
+  rc = build_schedule(pl, Rc, (plan_variant(pl, form, S, Rc) & kVarMorton) != 0, &out->sch, s);
+  if (rc == VL1_OK && form == VL1_FORM_SPLIT_I8) rc = i8_check_range(pl, out->sch, S);
   return rc;
 }
 
@@ -2054,13 +2339,22 @@ struct Staging {
 };
 
 // Bytes of staging for (form, S, R) laid out in one region, each part
-// 256-byte aligned: split X | colscale | nmdot, FP64 XF | nmdot.
+// 256-byte aligned: split X | colscale | nmdot, FP64 XF | nmdot (folded: X | dl
+// with `tile`).
 static size_t staging_layout(const vl1_plan* pl, int form, int S, int R, int n_tiles, char* base,
-                             Staging* st) {
+                             Staging* st, const FoldTile* tile = nullptr) {
   auto al = [](size_t b) { return (b + 255) / 256 * 256; };
   const size_t cols = (size_t)pl->nboxes * R;
   size_t off = 0;
   Staging t;
+  if (tile) {
+    t.XF = reinterpret_cast<double*>(base);
+    off = al(fold_x_size(pl->fold->d, *tile, pl->nboxes, R) * 8);
+    t.nmdot = reinterpret_cast<double*>(base + off);
+    off += al(fold_dl_size(*tile, pl->nboxes, R) * 8);
+    if (st) *st = t;
+    return off;
+  }
   if (form == VL1_FORM_SPLIT_I8) {
     t.X8 = reinterpret_cast<int8_t*>(base + off);
     off += al((size_t)pl->nboxes * S * R * pl->KP);
@@ -2083,6 +2377,50 @@ static size_t staging_layout(const vl1_plan* pl, int form, int S, int R, int n_t
   off += al(cols * 8);
   if (st) *st = t;
   return off;
+}
+
+static int fold_stage(vl1_plan* pl, const FoldTile& tile, const double* f, int64_t ldf, int R,
+                      const Staging& st, hipStream_t s) {
+  const hipError_t e = fold_stage_launch(
+      *pl->fold, tile, pl->nboxes, R, f, ldf, pl->mode_point.as<int32_t>(),
+      pl->box_starts.as<int32_t>(), pl->box_alpha.as<double>(), pl->box_disp.as<double>(),
+      pl->payload->nmlz.as<double>(), pl->log_disp, st.XF, st.nmdot, s);
+  if (e != hipSuccess) return fail(VL1_E_HIP, std::string("staging launch: ") + hipGetErrorString(e));
+  return VL1_OK;
+}
+
+static int fold_contract(vl1_plan* pl, const Prepared& pr, int R, double* y, int64_t ldy,
+                         const Staging& st, hipStream_t s) {
+  const FoldPlan& f = *pl->fold;
+  FoldParams p{};
+  p.d = f.d;
+  p.B = pr.tile.B;
+  p.Rc = pr.tile.Rc;
+  p.R = R;
+  p.nb = pl->nboxes;
+  p.n_box_tiles = pr.fold->n_tiles;
+  p.nm = f.nm;
+  p.cplx = f.cplx;
+  p.rows = f.rows;
+  p.tile_step_start = pr.fold->tile_step_start.as<int32_t>();
+  p.tile_boxes = pr.fold->tile_boxes.as<int32_t>();
+  p.tile_chunk_start = pr.fold->tile_chunk_start.as<int32_t>();
+  p.chunks = pr.fold->chunks.as<uint32_t>();
+  p.lut_u = f.u_lut;
+  p.lut_l = f.l_lut;
+  p.maxc = f.maxc;
+  p.step_src = pr.fold->step_src.as<int32_t>();
+  p.A = f.A.as<double>();
+  p.cls_stride = f.cls_stride;
+  p.X = st.XF;
+  p.dl = pl->log_disp ? st.nmdot : nullptr;
+  p.out = f.out_lut;
+  p.mode_point = pl->mode_point.as<int32_t>();
+  p.y = y;
+  p.ldy = ldy;
+  const hipError_t e = fold_contract_launch(p, pr.tile, s);
+  if (e != hipSuccess) return fail(VL1_E_HIP, std::string("folded tile launch: ") + hipGetErrorString(e));
+  return VL1_OK;
 }
 
 // Launch the staging kernel of `form` into `st`.
@@ -2274,11 +2612,11 @@ int vl1_plan_stage(vl1_plan* pl, int form, const double* f, int64_t ldf, int n_r
     return fail(VL1_E_ARG, "vl1_plan_stage: bad leading dimension");
   if (pl->n_tgt == 0 || pl->n_blocks == 0) return VL1_OK;
   hipStream_t s = (hipStream_t)stream;
-  int S = 0;
-  TileSchedule* sch = nullptr;
-  int rc = plan_prepare(pl, form, n_rhs, opts, s, &S, &sch);
+  Prepared pr;
+  int rc = plan_prepare(pl, form, n_rhs, opts, s, &pr);
   if (rc != VL1_OK) return rc;
-  const int R = n_rhs;
+  const int R = n_rhs, S = pr.S;
+  TileSchedule* sch = pr.sch;
   const size_t ncolumns = (size_t)pl->nboxes * R;
   hipError_t e = hipSuccess;
   // the largest buffer first: a failed allocation then leaves the others
@@ -2293,13 +2631,18 @@ int vl1_plan_stage(vl1_plan* pl, int form, const double* f, int64_t ldf, int n_r
     e = pl->grow(pl->X, (size_t)pl->nboxes * S * R * pl->KP * 2);
     if (e == hipSuccess) e = pl->grow(pl->nmdot, ncolumns * 8);
     if (e == hipSuccess) e = pl->grow(pl->colscale, ncolumns * 8);
+  } else if (pr.fold) {
+    e = pl->grow(pl->XF, fold_x_size(pl->fold->d, pr.tile, pl->nboxes, R) * 8);
+    if (e == hipSuccess && pl->log_disp)
+      e = pl->grow(pl->nmdot, fold_dl_size(pr.tile, pl->nboxes, R) * 8);
   } else {
     e = pl->grow(pl->XF, (size_t)pl->nboxes * R * pl->KP * 8);
     if (e == hipSuccess) e = pl->grow(pl->nmdot, ncolumns * 8);
   }
   if (e != hipSuccess) return fail(VL1_E_HIP, std::string("vl1_plan_stage alloc: ") + hipGetErrorString(e));
   const Staging st = plan_staging(pl);
-  rc = stage_launch(pl, form, S, f, ldf, R, st, s);
+  rc = pr.fold ? fold_stage(pl, pr.tile, f, ldf, R, st, s)
+               : stage_launch(pl, form, S, f, ldf, R, st, s);
   if (rc != VL1_OK) return rc;
   pl->staged_form = form;
   pl->staged_rhs = R;
@@ -2315,13 +2658,13 @@ int vl1_plan_contract(vl1_plan* pl, int form, int n_rhs, double* y, int64_t ldy,
     return fail(VL1_E_ARG, "vl1_plan_contract: bad leading dimension");
   if (pl->n_tgt == 0 || pl->n_blocks == 0) return VL1_OK;
   hipStream_t s = (hipStream_t)stream;
-  int S = 0;
-  TileSchedule* sch = nullptr;
-  int rc = plan_prepare(pl, form, n_rhs, opts, s, &S, &sch);
+  Prepared pr;
+  int rc = plan_prepare(pl, form, n_rhs, opts, s, &pr);
   if (rc != VL1_OK) return rc;
-  if (pl->staged_form != form || pl->staged_rhs != n_rhs || pl->staged_slices != S)
+  if (pl->staged_form != form || pl->staged_rhs != n_rhs || pl->staged_slices != pr.S)
     return fail(VL1_E_ARG, "vl1_plan_contract: densities were not staged for this form/RHS/slices");
-  return contract_launch(pl, form, S, sch, n_rhs, y, ldy, plan_staging(pl), s,
+  if (pr.fold) return fold_contract(pl, pr, n_rhs, y, ldy, plan_staging(pl), s);
+  return contract_launch(pl, form, pr.S, pr.sch, n_rhs, y, ldy, plan_staging(pl), s,
                          form == VL1_FORM_SPLIT_I8 && opts ? opts->error_est : nullptr);
 }
 
@@ -2331,8 +2674,13 @@ int vl1_plan_contract(vl1_plan* pl, int form, int n_rhs, double* y, int64_t ldy,
 // `scratch` itself to a kernel (on the host it only names the symbol): the
 // device address comes from hipGetSymbolAddress, looked up once per device
 // with that device current.
+// Staging is accepted up to kScratchBytes by the plain layouts; the folded
+// FP64 layout of the same call pads its parities to 4 and its densities to
+// whole tiles (at most 1.125 x 1.08 of the plain one beyond a few boxes), which
+// the array holds too.
 constexpr size_t kScratchBytes = (size_t)64 << 20;
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+constexpr size_t kScratchArray = (size_t)80 << 20;
+static __device__ __align__(256) unsigned char scratch[kScratchArray];
 
 constexpr int kMaxDevices = 64;
 static std::mutex scratch_mu;
@@ -2370,17 +2718,27 @@ int vl1_plan_eval_noalloc(vl1_plan* pl, int form, const double* f, int64_t ldf, 
   // allocates (one vl1_plan_eval with this form, slice count and RHS count
   // per tile builds both)
   const int Rc = std::min(n_rhs, kCols);
-  const int key = Rc * 2 + ((plan_variant(pl, form, S, Rc) & kVarMorton) ? 1 : 0);
-  auto it = pl->schedules.find(key);
-  if ((form != VL1_FORM_F64 && !pl->slices(form, S)) || it == pl->schedules.end())
+  const bool morton = (plan_variant(pl, form, S, Rc) & kVarMorton) != 0;
+  Prepared pr;
+  pr.S = S;
+  if (uses_fold(pl, form)) {
+    pr.tile = fold_tile(pl->fold->d, pl->n_tgt, n_rhs);
+    auto it = pl->fold_schedules.find(pr.tile.B * 2 + (morton ? 1 : 0));
+    if (it != pl->fold_schedules.end()) pr.fold = it->second;
+  } else {
+    auto it = pl->schedules.find(Rc * 2 + (morton ? 1 : 0));
+    if (it != pl->schedules.end()) pr.sch = it->second;
+  }
+  if ((form != VL1_FORM_F64 && !pl->slices(form, S)) || (!pr.sch && !pr.fold))
     return fail(VL1_E_UNSUPPORTED,
                 "vl1_plan_eval_noalloc: the plan is not prepared for this form / slice count / "
                 "RHS count (evaluate it once with vl1_plan_eval first)");
   if (form == VL1_FORM_SPLIT_I8) {
-    rc = i8_check_range(pl, it->second, S);
+    rc = i8_check_range(pl, pr.sch, S);
     if (rc != VL1_OK) return rc;
   }
-  const size_t need = staging_layout(pl, form, S, n_rhs, it->second->n_tiles, nullptr, nullptr);
+  const int n_tiles = pr.sch ? pr.sch->n_tiles : 0;
+  const size_t need = staging_layout(pl, form, S, n_rhs, n_tiles, nullptr, nullptr);
   if (need > kScratchBytes)
     return fail(VL1_E_UNSUPPORTED, "vl1_plan_eval_noalloc: staging needs " + std::to_string(need) +
                                        " bytes, above the fixed " + std::to_string(kScratchBytes) +
@@ -2389,13 +2747,28 @@ int vl1_plan_eval_noalloc(vl1_plan* pl, int form, const double* f, int64_t ldf, 
   rc = scratch_address(&base);
   if (rc != VL1_OK) return rc;
   Staging st;
-  staging_layout(pl, form, S, n_rhs, it->second->n_tiles, static_cast<char*>(base), &st);
   hipStream_t s = (hipStream_t)stream;
+  if (pr.fold) {
+    // as many densities at a time as the array holds (all of them but for
+    // trees of a few boxes with very many densities)
+    int step = n_rhs;
+    while (step > 64 && staging_layout(pl, form, S, step, 0, nullptr, nullptr, &pr.tile) > kScratchArray)
+      step = (step / 2 + 63) / 64 * 64;
+    if (staging_layout(pl, form, S, step, 0, static_cast<char*>(base), &st, &pr.tile) > kScratchArray)
+      return fail(VL1_E_UNSUPPORTED, "vl1_plan_eval_noalloc: staging exceeds the scratch array");
+    for (int r = 0; r < n_rhs && rc == VL1_OK; r += step) {
+      const int nr = std::min(step, n_rhs - r);
+      rc = fold_stage(pl, pr.tile, f + r * ldf, ldf, nr, st, s);
+      if (rc == VL1_OK) rc = fold_contract(pl, pr, nr, y + r * ldy, ldy, st, s);
+    }
+    return rc;
+  }
+  staging_layout(pl, form, S, n_rhs, n_tiles, static_cast<char*>(base), &st);
   // every word the contraction reads is written by the staging kernel
   // (padding rows included), so nothing needs clearing between calls
   rc = stage_launch(pl, form, S, f, ldf, n_rhs, st, s);
   if (rc != VL1_OK) return rc;
-  return contract_launch(pl, form, S, it->second, n_rhs, y, ldy, st, s,
+  return contract_launch(pl, form, S, pr.sch, n_rhs, y, ldy, st, s,
                          form == VL1_FORM_SPLIT_I8 && opts ? opts->error_est : nullptr);
 }
 
@@ -2495,13 +2868,19 @@ int vl1_plan_stats(const vl1_plan* pl, int64_t* out5) {
     const TileSchedule* sch = pl->schedules.begin()->second;
     tiles = sch->n_tiles;
     steps = sch->n_steps;
+  } else if (!pl->fold_schedules.empty()) {
+    // in the other forms' units: 64-column tiles of at most kMaxTileRows rows;
+    // the folded form takes all rows of a tile and one step per class
+    const int B = std::max(1, kCols / pl->fold_rc);
+    tiles = (int64_t)((pl->n_tgt + B - 1) / B) * pl->n_rg;
+    steps = pl->fold_schedules.begin()->second->n_steps;
   }
   out5[1] = tiles;
   out5[2] = steps;
   out5[3] = pl->n_keys;
   int64_t bytes = (int64_t)(pl->M.bytes + pl->MF.bytes + pl->rowscale.bytes + pl->X.bytes +
                             pl->XF.bytes + pl->colscale.bytes + pl->nmdot.bytes +
-                            pl->mode_point.bytes);
+                            pl->mode_point.bytes + (pl->fold ? pl->fold->A.bytes : 0));
   for (auto& kv : pl->A_by_slices) bytes += (int64_t)kv.second->bytes;
   for (const DevBuf* b : pl->retired) bytes += (int64_t)b->bytes;
   out5[4] = bytes;

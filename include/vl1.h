@@ -263,7 +263,10 @@ typedef struct vl1_split_opts {
    * receives per RHS the estimated relative error of the result over the
    * plan's targets, [0] max |error| / max |y| (Linf) and [1]
    * ||error||_2 / ||y||_2 (L2).  The estimate is 4/254 of the last slice
-   * diagonal kept, the size of the first diagonal dropped, per output. */
+   * diagonal kept, the size of the first diagonal dropped, per output; 2^-52
+   * where nothing is dropped (5 and 6 slices of a plan with
+   * reflection-symmetric blocks run on the FP64 form's folded kernel, which is
+   * faster there).  FP64 rounding itself is not part of it. */
   double* error_est;
 } vl1_split_opts;
 

@@ -18,8 +18,9 @@ import torch
 from oracle import list1_ref, orbit_ref
 from tests.gpu_helpers import adaptive, rel_errors
 from tests.test_gpu_plan import _sub_tree
-from volumential_amd import orbit, tree as vtree
+from volumential_amd import _capi, orbit, tree as vtree
 from volumential_amd.kernels import HelmholtzKernel, LaplaceKernel
+from volumential_amd.plan import FORMS
 from volumential_amd.table import NearFieldInteractionTable
 from volumential_amd.wrangler import NearFieldWrangler
 
@@ -104,3 +105,39 @@ def test_fold_ragged_densities(cuda, n_rhs):
     print(f"case: fold 2D q=3 R={n_rhs}", flush=True)
     tr, table, f = _case(2, 3, False, 5, n_rhs, 3)
     _check(tr, table, f, False, list(range(n_rhs)))
+
+
+@pytest.mark.parametrize("form", ["split", "split_i8"])
+@pytest.mark.parametrize("dim,level,n_rhs", [(2, 4, 3), (3, 2, 64)])
+def test_split_forms_on_fold(cuda, dim, level, n_rhs, form):
+    """Five and more slices run on the folded kernel: the FP64 form's result
+    (the same launches), an estimate at the size of FP64 rounding, and the
+    same through the allocation-free entry, also at a density count that was
+    prepared at another multiple of 64.  Fewer slices keep their own error."""
+    print(f"case: {form} on the folded kernel {dim}D R={n_rhs}", flush=True)
+    tr, table, f = _case(dim, 4, False, level, n_rhs, 7)
+    w = NearFieldWrangler(tr, table)
+    plan = w.get_plan(w.target_kernels[0], tr.target_boxes, tr.neighbor_source_boxes_starts,
+                      tr.neighbor_source_boxes_lists)
+    fd = torch.as_tensor(f, device="cuda")
+    est = torch.full((n_rhs, 2), -1.0, dtype=torch.float64, device="cuda")
+    ref = plan.eval(fd, form="f64")
+    low = plan.eval(fd, form=form, n_slices=4)
+    i8 = form == "split_i8"
+    for S in (5, 6):
+        got = plan.eval(fd, form=form, n_slices=S, error_est=est if i8 else None)
+        assert torch.equal(got, ref)
+        if i8:
+            assert bool(((est > 0) & (est <= 1e-15)).all())
+    lo = (low - ref).abs().max() / ref.abs().max()
+    assert 1e-13 < float(lo) < 1e-5
+    for F in (fd, torch.cat([fd, fd]) if n_rhs == 64 else fd):
+        y = torch.full_like(F, float("nan"))
+        opts = _capi.SplitOpts(n_slices=5, n_products=0)
+        _capi.check(_capi.lib().vl1_plan_eval_noalloc(
+            plan.handle, FORMS[form], F.data_ptr(), F.shape[1], F.shape[0], y.data_ptr(),
+            y.shape[1], opts, _capi.stream_handle(None)), "vl1_plan_eval_noalloc")
+        targets = ~torch.isnan(y[0])
+        want = torch.cat([ref, ref]) if F.shape[0] > n_rhs else ref
+        scale = ref.abs().max()
+        assert float((y[:, targets] - want[:, targets]).abs().max() / scale) <= 1e-13

@@ -100,7 +100,6 @@ inline int fold_chunks(const FoldDims& d, int m) {
   return (d.rounds + (kFoldUnits >> m) - 1) / (kFoldUnits >> m);
 }
 
-// Tile shape for R densities over n_tgt boxes.
 struct FoldTile {
   int nct = 0, Rc = 0, B = 0;  // 16-column tiles; densities and boxes per tile
 };
@@ -132,7 +131,8 @@ struct FoldPlan {
 // Folded basis of q^dim nodes (2 values per node if complex); false: sizes
 // the kernel does not take.
 bool fold_layout(FoldPlan& f, int dim, int q, int cplx, uint32_t sign_mask);
-FoldTile fold_tile(const FoldDims& d, int n_tgt, int R);
+// Tile shape for R densities over n_tgt boxes (16 nct columns; 0: choose).
+FoldTile fold_tile(int n_tgt, int R, int nct = 0);
 // X and dl sizes in doubles for one evaluation.
 size_t fold_x_size(const FoldDims& d, const FoldTile& t, int nb, int R);
 size_t fold_dl_size(const FoldTile& t, int nb, int R);

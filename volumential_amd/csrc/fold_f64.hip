@@ -175,7 +175,7 @@ bool fold_layout(FoldPlan& f, int dim, int q, int cplx, uint32_t sign_mask) {
 // them best (R = 24 over 64 columns: 3 x 8 densities of 8 boxes, all columns
 // in use; 59: 15 x 4), the largest up to 8 among equals -- neighbouring boxes
 // in a tile share their sources' cache lines.
-FoldTile fold_tile(const FoldDims& d, int n_tgt, int R) {
+FoldTile fold_tile(int n_tgt, int R, int nct) {
   const int Rq = std::min(R, 64);  // larger counts are whole multiples of 64
   auto pick = [&](int nct) {
     const int cols = 16 * nct;
@@ -195,6 +195,7 @@ FoldTile fold_tile(const FoldDims& d, int n_tgt, int R) {
     }
     return t;
   };
+  if (nct) return pick(nct);
   // 32 columns, unless that leaves some of the 256 CUs at one workgroup or
   // none; then 16 (q = 4, 4096 boxes, one density: three calls 141 us with 32,
   // 122 us with 16; graded q = 5, 446 tiles: 477 us with 32, 563 us with 16)

@@ -31,6 +31,7 @@
 #include <numeric>
 #include <string>
 #include <type_traits>
+#include <set>
 #include <unordered_map>
 #include <vector>
 
@@ -1264,6 +1265,10 @@ struct vl1_plan {
   std::map<int, TileSchedule*> schedules;  // by 2 Rc + (Morton-only order)
   FoldPlan* fold = nullptr;                // folded FP64 form (null: the dense one)
   std::map<int, FoldSchedule*> fold_schedules;  // by 2 B + (Morton-only order)
+  uint32_t fold_ready = 0;  // fold_bit of the calls prepared on it
+  int max_sources = 0;      // list-1 sources of a target
+  bool unfolded = false;    // a call ran on the general kernels
+  std::set<int> prepared_rhs;  // densities per tile of the calls prepared so far
   int fold_rc = 1;  // densities per 64 columns of the first folded evaluation (statistics)
   std::map<int, int> tuned;                 // variant by (form, slices, Rc), from vl1_plan_tune
   int forced_variant = -1;                  // candidate under test in vl1_plan_tune
@@ -2029,6 +2034,7 @@ static int plan_create(vl1_plan** out, const vl1_payload* pay, const vl1_plan_de
   for (int i = 0; i < d->n_tgt_boxes; ++i) {
     const int tb = d->target_boxes[i];
     pl->tgt_boxes.push_back(tb);
+    pl->max_sources = std::max(pl->max_sources, (int)(d->nbr_starts[i + 1] - d->nbr_starts[i]));
     for (int64_t k = d->nbr_starts[i]; k < d->nbr_starts[i + 1]; ++k) {
       const int sb = d->nbr_lists[k];
       const int lvl = d->box_levels[sb];
@@ -2211,6 +2217,9 @@ int vl1_plan_destroy(vl1_plan* plan) {
 // boxes per tile); kVarNoPhase = no XCD phase alignment of the step order.
 constexpr int kVarOneRow = 1, kVarMorton = 2, kVarNoPhase = 4;
 
+// (form, slices) that have been prepared on the folded kernel
+static uint32_t fold_bit(int form, int S) { return 1u << (form * 8 + S); }
+
 static int tune_key(int form, int S, int Rc) { return (form * 8 + S) * 1024 + Rc; }
 
 static int default_variant(const vl1_plan* pl, int form) {
@@ -2279,9 +2288,11 @@ static int i8_ring_slots(int S, int waves) {
 // The int8 form sums a tile's digit products exactly in int32: the largest
 // diagonal (S products per K column, |d| <= 127) over all K columns of all
 // the tile's steps must stay below 2^31.
+static bool i8_sums_fit(double steps, int KP, int S) {
+  return steps * KP * S * 127.0 * 127.0 < 2147483647.0;
+}
 static int i8_check_range(const vl1_plan* pl, const TileSchedule* sch, int S) {
-  const double worst = (double)sch->max_steps * pl->KP * S * 127.0 * 127.0;
-  if (worst >= 2147483647.0)
+  if (!i8_sums_fit(sch->max_steps, pl->KP, S))
     return fail(VL1_E_UNSUPPORTED, "vl1_plan: int8 split form: " + std::to_string(sch->max_steps) +
                                        " steps per tile could overflow the exact int32 sums; "
                                        "use the BF16 split or FP64 form");
@@ -2297,7 +2308,25 @@ struct Prepared {
   FoldTile tile;
 };
 
-static bool uses_fold(const vl1_plan* pl, int form) { return form == VL1_FORM_F64 && pl->fold; }
+// The folded FP64 kernel takes the FP64 form, and the split forms at the slice
+// counts that aim at the 1e-10 bar: a folded block costs 1/8 (3D) or 1/4 (2D)
+// of the products, a split one S (S + 1) / 2 times them on faster units.
+// Measured at S = 5, split against folded, us per call: int8 3D q = 6, 32768
+// boxes, 64 densities 29651 / 22939; int8 2D q = 6 complex per-level, 12919
+// boxes, 16 densities 1323 / 468; int8 fused Helmholtz split, 16384 boxes, 16
+// densities 647 / 513; BF16 3D q = 4, 4096 boxes, 20 densities 1023 / 244.
+// Below 5 slices a caller asks for the split itself, its error included.
+// Calls whose int8 sums might leave int32 stay with the int8 form, which
+// refuses them by its own schedule (i8_check_range).
+constexpr int kFoldSlices = 5;
+static bool uses_fold(const vl1_plan* pl, int form, int S, int n_rhs) {
+  if (!pl->fold) return false;
+  if (form == VL1_FORM_F64) return true;
+  if (S < kFoldSlices) return false;
+  const int B = std::max(1, kCols / std::min(n_rhs, kCols));  // boxes per int8 tile
+  const double steps = std::min((double)pl->n_keys, (double)B * pl->max_sources);
+  return form != VL1_FORM_SPLIT_I8 || i8_sums_fit(steps, pl->KP, S);
+}
 
 // Checks, then builds (allocating) the slice set and tile schedule this
 // evaluation needs if the plan does not hold them yet.
@@ -2306,24 +2335,39 @@ static int plan_prepare(vl1_plan* pl, int form, int n_rhs, const vl1_split_opts*
   int S = 0;
   int rc = plan_check(pl, form, n_rhs, opts, &S);
   if (rc != VL1_OK) return rc;
-  if (uses_fold(pl, form)) {
-    out->tile = fold_tile(pl->fold->d, pl->n_tgt, n_rhs);
-    const bool morton = (plan_variant(pl, form, S, std::min(n_rhs, kCols)) & kVarMorton) != 0;
-    if (pl->fold_schedules.empty()) pl->fold_rc = std::min(n_rhs, kCols);
-    return build_fold_schedule(pl, out->tile.B, morton, &out->fold, s);
-  }
-  if (form == VL1_FORM_SPLIT_BF16) {
+  out->S = S;
+  const int Rc = std::min(n_rhs, kCols);
+  const bool morton = (plan_variant(pl, form, S, Rc) & kVarMorton) != 0;
+  const bool fold = uses_fold(pl, form, S, n_rhs);
+  if (!fold && form == VL1_FORM_SPLIT_BF16) {
     rc = ensure_A(pl, S, s);
     if (rc != VL1_OK) return rc;
-  } else if (form == VL1_FORM_SPLIT_I8) {
+  } else if (!fold && form == VL1_FORM_SPLIT_I8) {
     rc = ensure_A8(pl, S, s);
     if (rc != VL1_OK) return rc;
   }
-  out->S = S;
-  const int Rc = std::min(n_rhs, kCols);
-  rc = build_schedule(pl, Rc, (plan_variant(pl, form, S, Rc) & kVarMorton) != 0, &out->sch, s);
-  if (rc == VL1_OK && form == VL1_FORM_SPLIT_I8) rc = i8_check_range(pl, out->sch, S);
-  return rc;
+  if (fold) {
+    pl->fold_ready |= fold_bit(form, S);
+    out->tile = fold_tile(pl->n_tgt, n_rhs);
+    if (pl->fold_schedules.empty()) pl->fold_rc = Rc;
+    rc = build_fold_schedule(pl, out->tile.B, morton, &out->fold, s);
+  } else {
+    pl->unfolded = true;
+    rc = build_schedule(pl, Rc, morton, &out->sch, s);
+    if (rc == VL1_OK && form == VL1_FORM_SPLIT_I8) rc = i8_check_range(pl, out->sch, S);
+  }
+  // a plan that serves both kernels keeps the tiles of every density count for
+  // both: an allocation-free call takes any prepared form at any prepared count
+  pl->prepared_rhs.insert(Rc);
+  if (rc != VL1_OK || !pl->fold || !pl->unfolded) return rc;
+  for (int R : pl->prepared_rhs) {
+    FoldSchedule* fs = nullptr;
+    TileSchedule* ts = nullptr;
+    rc = build_fold_schedule(pl, fold_tile(pl->n_tgt, R).B, false, &fs, s);
+    if (rc == VL1_OK) rc = build_schedule(pl, R, false, &ts, s);
+    if (rc != VL1_OK) return rc;
+  }
+  return VL1_OK;
 }
 
 // Per-evaluation staging: density slices, column scales and the 2D log-term
@@ -2389,8 +2433,13 @@ static int fold_stage(vl1_plan* pl, const FoldTile& tile, const double* f, int64
   return VL1_OK;
 }
 
+static __global__ void fold_est_kernel(int n, double* __restrict__ est) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) est[i] = 0x1p-52;
+}
+
 static int fold_contract(vl1_plan* pl, const Prepared& pr, int R, double* y, int64_t ldy,
-                         const Staging& st, hipStream_t s) {
+                         const Staging& st, hipStream_t s, double* est) {
   const FoldPlan& f = *pl->fold;
   FoldParams p{};
   p.d = f.d;
@@ -2418,7 +2467,12 @@ static int fold_contract(vl1_plan* pl, const Prepared& pr, int R, double* y, int
   p.mode_point = pl->mode_point.as<int32_t>();
   p.y = y;
   p.ldy = ldy;
-  const hipError_t e = fold_contract_launch(p, pr.tile, s);
+  hipError_t e = fold_contract_launch(p, pr.tile, s);
+  if (e == hipSuccess && est) {
+    // no product is cut: what is left is FP64 rounding, which the estimate does not cover
+    hipLaunchKernelGGL(fold_est_kernel, dim3((2 * R + 255) / 256), dim3(256), 0, s, 2 * R, est);
+    e = hipGetLastError();
+  }
   if (e != hipSuccess) return fail(VL1_E_HIP, std::string("folded tile launch: ") + hipGetErrorString(e));
   return VL1_OK;
 }
@@ -2621,7 +2675,11 @@ int vl1_plan_stage(vl1_plan* pl, int form, const double* f, int64_t ldf, int n_r
   hipError_t e = hipSuccess;
   // the largest buffer first: a failed allocation then leaves the others
   // untouched
-  if (form == VL1_FORM_SPLIT_I8) {
+  if (pr.fold) {
+    e = pl->grow(pl->XF, fold_x_size(pl->fold->d, pr.tile, pl->nboxes, R) * 8);
+    if (e == hipSuccess && pl->log_disp)
+      e = pl->grow(pl->nmdot, fold_dl_size(pr.tile, pl->nboxes, R) * 8);
+  } else if (form == VL1_FORM_SPLIT_I8) {
     e = pl->grow(pl->X8, (size_t)pl->nboxes * S * R * pl->KP);
     if (e == hipSuccess) e = pl->grow(pl->nmdot, ncolumns * 8);
     if (e == hipSuccess) e = pl->grow(pl->colscale, ncolumns * 8);
@@ -2631,10 +2689,6 @@ int vl1_plan_stage(vl1_plan* pl, int form, const double* f, int64_t ldf, int n_r
     e = pl->grow(pl->X, (size_t)pl->nboxes * S * R * pl->KP * 2);
     if (e == hipSuccess) e = pl->grow(pl->nmdot, ncolumns * 8);
     if (e == hipSuccess) e = pl->grow(pl->colscale, ncolumns * 8);
-  } else if (pr.fold) {
-    e = pl->grow(pl->XF, fold_x_size(pl->fold->d, pr.tile, pl->nboxes, R) * 8);
-    if (e == hipSuccess && pl->log_disp)
-      e = pl->grow(pl->nmdot, fold_dl_size(pr.tile, pl->nboxes, R) * 8);
   } else {
     e = pl->grow(pl->XF, (size_t)pl->nboxes * R * pl->KP * 8);
     if (e == hipSuccess) e = pl->grow(pl->nmdot, ncolumns * 8);
@@ -2663,9 +2717,9 @@ int vl1_plan_contract(vl1_plan* pl, int form, int n_rhs, double* y, int64_t ldy,
   if (rc != VL1_OK) return rc;
   if (pl->staged_form != form || pl->staged_rhs != n_rhs || pl->staged_slices != pr.S)
     return fail(VL1_E_ARG, "vl1_plan_contract: densities were not staged for this form/RHS/slices");
-  if (pr.fold) return fold_contract(pl, pr, n_rhs, y, ldy, plan_staging(pl), s);
-  return contract_launch(pl, form, pr.S, pr.sch, n_rhs, y, ldy, plan_staging(pl), s,
-                         form == VL1_FORM_SPLIT_I8 && opts ? opts->error_est : nullptr);
+  double* est = form == VL1_FORM_SPLIT_I8 && opts ? opts->error_est : nullptr;
+  if (pr.fold) return fold_contract(pl, pr, n_rhs, y, ldy, plan_staging(pl), s, est);
+  return contract_launch(pl, form, pr.S, pr.sch, n_rhs, y, ldy, plan_staging(pl), s, est);
 }
 
 // ------------------------------------------------ allocation-free evaluation
@@ -2675,11 +2729,11 @@ int vl1_plan_contract(vl1_plan* pl, int form, int n_rhs, double* y, int64_t ldy,
 // device address comes from hipGetSymbolAddress, looked up once per device
 // with that device current.
 // Staging is accepted up to kScratchBytes by the plain layouts; the folded
-// FP64 layout of the same call pads its parities to 4 and its densities to
-// whole tiles (at most 1.125 x 1.08 of the plain one beyond a few boxes), which
-// the array holds too.
+// layout of the same call pads its parities to 4 and its densities to whole
+// tiles, and holds 8 bytes where 5 int8 slices take 5 (at most 1.64 x 1.08 of
+// the plain layout beyond a few boxes, 3D q = 3), which the array holds too.
 constexpr size_t kScratchBytes = (size_t)64 << 20;
-constexpr size_t kScratchArray = (size_t)80 << 20;
+constexpr size_t kScratchArray = (size_t)128 << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchArray];
 
 constexpr int kMaxDevices = 64;
@@ -2721,23 +2775,32 @@ int vl1_plan_eval_noalloc(vl1_plan* pl, int form, const double* f, int64_t ldf, 
   const bool morton = (plan_variant(pl, form, S, Rc) & kVarMorton) != 0;
   Prepared pr;
   pr.S = S;
-  if (uses_fold(pl, form)) {
-    pr.tile = fold_tile(pl->fold->d, pl->n_tgt, n_rhs);
-    auto it = pl->fold_schedules.find(pr.tile.B * 2 + (morton ? 1 : 0));
-    if (it != pl->fold_schedules.end()) pr.fold = it->second;
+  const bool fold = uses_fold(pl, form, S, n_rhs);
+  if (fold) {
+    // either tile width serves: a count prepared at another multiple of 64
+    // may have taken the other one
+    pr.tile = fold_tile(pl->n_tgt, n_rhs);
+    for (int k = 0; k < 2 && !pr.fold; ++k) {
+      if (k) pr.tile = fold_tile(pl->n_tgt, n_rhs, 3 - pr.tile.nct);
+      auto it = pl->fold_schedules.find(pr.tile.B * 2 + (morton ? 1 : 0));
+      if (it != pl->fold_schedules.end()) pr.fold = it->second;
+    }
   } else {
     auto it = pl->schedules.find(Rc * 2 + (morton ? 1 : 0));
     if (it != pl->schedules.end()) pr.sch = it->second;
   }
-  if ((form != VL1_FORM_F64 && !pl->slices(form, S)) || (!pr.sch && !pr.fold))
+  const bool ready = form == VL1_FORM_F64 ||
+                     (fold ? (pl->fold_ready & fold_bit(form, S)) != 0 : pl->slices(form, S) != nullptr);
+  if (!ready || (!pr.sch && !pr.fold))
     return fail(VL1_E_UNSUPPORTED,
                 "vl1_plan_eval_noalloc: the plan is not prepared for this form / slice count / "
                 "RHS count (evaluate it once with vl1_plan_eval first)");
-  if (form == VL1_FORM_SPLIT_I8) {
+  if (form == VL1_FORM_SPLIT_I8 && !fold) {
     rc = i8_check_range(pl, pr.sch, S);
     if (rc != VL1_OK) return rc;
   }
-  const int n_tiles = pr.sch ? pr.sch->n_tiles : 0;
+  const int B = std::max(1, kCols / Rc);
+  const int n_tiles = pr.sch ? pr.sch->n_tiles : (pl->n_tgt + B - 1) / B * pl->n_rg;
   const size_t need = staging_layout(pl, form, S, n_rhs, n_tiles, nullptr, nullptr);
   if (need > kScratchBytes)
     return fail(VL1_E_UNSUPPORTED, "vl1_plan_eval_noalloc: staging needs " + std::to_string(need) +
@@ -2748,6 +2811,7 @@ int vl1_plan_eval_noalloc(vl1_plan* pl, int form, const double* f, int64_t ldf, 
   if (rc != VL1_OK) return rc;
   Staging st;
   hipStream_t s = (hipStream_t)stream;
+  double* est = form == VL1_FORM_SPLIT_I8 && opts ? opts->error_est : nullptr;
   if (pr.fold) {
     // as many densities at a time as the array holds (all of them but for
     // trees of a few boxes with very many densities)
@@ -2759,7 +2823,7 @@ int vl1_plan_eval_noalloc(vl1_plan* pl, int form, const double* f, int64_t ldf, 
     for (int r = 0; r < n_rhs && rc == VL1_OK; r += step) {
       const int nr = std::min(step, n_rhs - r);
       rc = fold_stage(pl, pr.tile, f + r * ldf, ldf, nr, st, s);
-      if (rc == VL1_OK) rc = fold_contract(pl, pr, nr, y + r * ldy, ldy, st, s);
+      if (rc == VL1_OK) rc = fold_contract(pl, pr, nr, y + r * ldy, ldy, st, s, est ? est + 2 * r : est);
     }
     return rc;
   }
@@ -2768,8 +2832,7 @@ int vl1_plan_eval_noalloc(vl1_plan* pl, int form, const double* f, int64_t ldf, 
   // (padding rows included), so nothing needs clearing between calls
   rc = stage_launch(pl, form, S, f, ldf, n_rhs, st, s);
   if (rc != VL1_OK) return rc;
-  return contract_launch(pl, form, S, pr.sch, n_rhs, y, ldy, st, s,
-                         form == VL1_FORM_SPLIT_I8 && opts ? opts->error_est : nullptr);
+  return contract_launch(pl, form, S, pr.sch, n_rhs, y, ldy, st, s, est);
 }
 
 int vl1_plan_eval(vl1_plan* pl, int form, const double* f, int64_t ldf, int n_rhs, double* y,

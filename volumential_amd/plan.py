@@ -12,6 +12,10 @@ the per-case dense blocks, and then evaluates many densities per call
   operand (default 6), exact int32 sums over all of a tile's list-1 boxes,
   one FP64 recombination per output, and an error estimate per density.
 
+At 5 and 6 slices both split forms run on the FP64 form's folded kernel where
+the plan has one (tables with the reflection symmetry): faster there, and exact
+to FP64 rounding.
+
 This is the batched counterpart of the per-RHS ``eval_direct`` loop of
 ``volume_fmm.py:983-1031``.
 """

@@ -32,6 +32,7 @@ struct vl1_payload {
   // built at creation for the dense kind, where a quiet NaN marks an entry
   // without data
   mutable vl1::DevBuf dense;
+  mutable int dense_finite = 0;  // every entry of an expanded row-map table is finite
   int64_t device_bytes() const {
     return (int64_t)(table.bytes + nmlz.bytes + case_idx.bytes + ranks.bytes + offs.bytes +
                      rowmap.bytes + dense.bytes);

@@ -249,7 +249,7 @@ __global__ void __launch_bounds__(kNFBlock) near_field_f64_kernel(const NFParams
 
 // ------------------------------------------------------------------------
 // FP64-MFMA form of the same evaluation (real tables, boxes of at most 256
-// nodes): per target box and group of 64 densities, every list-1 pair is a
+// nodes): per target box and group of 16 NC densities, every list-1 pair is a
 // product Y[tid][r] += sum_sid A[tid][sid] X[sid][r] with
 //   A[tid][sid] = D[lev][case][mode(sid)][mode(tid)]  (expanded blocks),
 //   X[sid][r]   = scaling * f[r][sbeg + sid],
@@ -257,16 +257,22 @@ __global__ void __launch_bounds__(kNFBlock) near_field_f64_kernel(const NFParams
 // the pair, so ragged boxes, permuted, repeated or invalid mode ids keep the
 // semantics of the scalar kernel above: an invalid id (or a missing entry,
 // NaN in the expanded blocks) gives A = 0.  v_mfma_f64_16x16x4f64 tiles:
-// wave w owns row tiles w, w + 8 (16 rows each) and all four 16-column
-// tiles; K advances in chunks of 32 source particles.  A chunk's densities
-// go through a two-slot LDS ring and its table fragments through
-// registers, both loaded one chunk ahead; a pair's source modes (and its
-// descriptor) are prepared one pair ahead.  The 2D log displacement is the
+// wave w owns row tiles w, w + 8 (16 rows each) and all NC 16-column tiles
+// (the fewest of 1, 2, 4 for the densities: fewer columns are computed than
+// asked for only past the last density).  K advances in chunks of KC source
+// particles; a chunk's densities go through a two-slot LDS ring and its table
+// fragments through registers, both loaded one chunk ahead, and a pair's source
+// modes two pairs ahead.  Pair descriptors (a chain of four dependent loads
+// each) are made 64 at a time, one per thread.  The 2D log displacement is the
 // same for every target of a pair: sum_sid nmlz[sid] f[sid], accumulated in
 // LDS while the densities are staged and added when the pair ends (only
 // used where no entry is missing: the scalar kernel drops the displacement
 // of a missing entry, list1.py:1111-1116).
-constexpr int kNFPitch = 34;  // doubles per column of a staged chunk (32 + 2)
+// Bound: the FP64 matrix pipe.  3D q = 4, 4096 boxes, 16 densities (1.3e10
+// flop): 1752 us with 64 columns whatever the densities and each descriptor
+// made by all threads when its pair began; 404 us so (32 TFLOP/s: the pipe is
+// busy 45% of the time, the rest goes to the loads' issue and the sums' chain).
+constexpr int kNFPairs = 64;  // pair descriptors made at a time
 constexpr int kNFMaxK = 256;  // source particles per box in the MFMA form
 
 typedef __attribute__((ext_vector_type(4))) double nf_doublex4;
@@ -317,27 +323,36 @@ __device__ inline NFPair nf_pair(const NFParams& p, int li, const double (&ct)[3
   return d;
 }
 
-template <int W, int NRT>
-__global__ void __launch_bounds__(64 * W) near_field_mfma_kernel(const NFParams p, int KP) {
-  constexpr int T = 64 * W;
-  constexpr int VPT = 2048 / T;  // densities of a chunk per thread
-  __shared__ __align__(16) double sX[2][64 * kNFPitch];
-  __shared__ int sMode[2][kNFMaxK];
-  __shared__ double sDisp[2][64];
+template <int W, int NRT, int NC, int KC>
+__global__ void __launch_bounds__(64 * W, NC * NRT == 1 ? 4 : 1)
+near_field_mfma_kernel(const NFParams p, int KP, int n_tgt_boxes, int finite) {
+  constexpr int T = 64 * W, COLS = 16 * NC, KU = KC / 4;
+  constexpr int VPT = KC * COLS / T;  // densities of a chunk per thread
+  constexpr int PITCH = KC + 2;       // doubles per column of a staged chunk
+  __shared__ __align__(16) double sX[2][COLS * PITCH];
+  __shared__ NFPair sPair[2][kNFPairs];
+  constexpr int KMAX = (16 * W * NRT + 31) / 32 * 32;  // KP at most
+  __shared__ __align__(16) int sRow[3][KMAX];  // table row of a source particle, in bytes
+  __shared__ bool sOk[3][KMAX];                // whether it has one
+  __shared__ double sDisp[3][COLS];
 
   const int n = p.n;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;
   const int l16 = lane % 16, lg = lane / 16;
-  const int tbox = blockIdx.x;
-  const int r0 = blockIdx.y * 64;
-  const int rc = min(64, p.n_rhs - r0);
+  // neighbouring boxes on one XCD (workgroup i runs on XCD i % 8): their
+  // sources meet in its L2
+  const int per = (n_tgt_boxes + 7) / 8;
+  const int tbox = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+  if (tbox >= n_tgt_boxes) return;  // uniform over the workgroup
+  const int r0 = blockIdx.y * COLS;
+  const int rc = min(COLS, p.n_rhs - r0);
   const int tb = p.target_boxes[tbox];
   const int tbeg = p.tgt_starts[tb];
   const int ntb = min(p.tgt_counts[tb], n);
   const int l0 = p.nbr_starts[tbox];
   const int npairs = p.nbr_starts[tbox + 1] - l0;
-  const int nkc = KP / 32;
+  const int nkc = KP / KC;  // KP: a multiple of KC
   double ct[3] = {0.0, 0.0, 0.0};
   for (int k = 0; k < p.dim; ++k) ct[k] = p.centers[(int64_t)k * p.nboxes + tb];
 
@@ -352,128 +367,170 @@ __global__ void __launch_bounds__(64 * W) near_field_mfma_kernel(const NFParams 
     tmA[rt] = (unsigned)m < (unsigned)n ? m : -1;
   }
 
-  // pair k's source modes into sMode[k & 1] (-1 past the box or invalid);
-  // its displacement sums start at zero
-  auto prep_pair = [&](const NFPair& d, int slot) {
-    for (int i = tid; i < KP; i += T) {
-      const int m = i < d.ns ? p.src_ids[d.sbeg + i] : -1;
-      sMode[slot][i] = (unsigned)m < (unsigned)n ? m : -1;
+  // descriptors of pairs [64 blk, 64 blk + 64)
+  auto make_pairs = [&](int blk) {
+    const int k = blk * kNFPairs + tid;
+    if (tid < kNFPairs && k < npairs) {
+      const NFPair d = nf_pair(p, l0 + k, ct);
+      if (!d.ok && p.err) atomicOr(p.err, 1);
+      sPair[blk & 1][tid] = d;
     }
-    if (tid < 64) sDisp[slot][tid] = 0.0;
   };
-  // densities of chunk kc of a pair: thread value v is column (tid + T v) / 32,
-  // source particle 32 kc + (tid + T v) % 32 (consecutive threads read
-  // consecutive particles of one density)
+  auto pair = [&](int k) -> const NFPair& { return sPair[(k / kNFPairs) & 1][k % kNFPairs]; };
+  // pair k's source modes (-1 past the box or invalid: a zero density and any
+  // row); its displacement sums start at zero
+  auto mode_of = [&](int k) {
+    if (k >= npairs || tid >= KP) return -1;
+    const NFPair& d = pair(k);
+    const int m = tid < d.ns ? p.src_ids[d.sbeg + tid] : -1;
+    return (unsigned)m < (unsigned)n ? m : -1;
+  };
+  auto put_mode = [&](int k, int m) {
+    if (tid < KP) {
+      sRow[k % 3][tid] = 8 * n * max(m, 0);
+      sOk[k % 3][tid] = m >= 0;
+    }
+    if (tid < COLS) sDisp[k % 3][tid] = 0.0;
+  };
+  // densities of chunk kc of a pair: thread value v is column xcol + v T / KC,
+  // source particle KC kc + xk (consecutive threads read consecutive particles
+  // of one density); loads past the box or the densities read a valid one
+  static_assert(T % KC == 0, "a thread keeps one particle of the chunk");
+  const int xk = tid % KC, xcol = tid / KC;
+  int64_t xoff[VPT];
+#pragma unroll
+  for (int v = 0; v < VPT; ++v) xoff[v] = (int64_t)min(xcol + v * (T / KC), rc - 1) * p.ldf;
   auto load_x = [&](const NFPair& d, int kc, double (&x)[VPT]) {
+    const int ns = __builtin_amdgcn_readfirstlane(d.ns);
+    const double* f = p.f + (int64_t)r0 * p.ldf + __builtin_amdgcn_readfirstlane(d.sbeg);
+    if (ns > 0) {
+      const int sid = min(KC * kc + xk, ns - 1);
 #pragma unroll
-    for (int v = 0; v < VPT; ++v) {
-      const int u = tid + T * v;
-      const int col = u / 32, sid = 32 * kc + u % 32;
-      x[v] = (col < rc && sid < d.ns) ? p.f[(int64_t)(r0 + col) * p.ldf + d.sbeg + sid] : 0.0;
+      for (int v = 0; v < VPT; ++v) x[v] = f[xoff[v] + sid];
     }
   };
-  auto store_x = [&](const NFPair& d, int kc, int slot, int ring, const double (&x)[VPT]) {
+  auto store_x = [&](const NFPair& d, int kc, int k, int ring, const double (&x)[VPT]) {
+    const int slot = k % 3, sid = KC * kc + xk;
+    const bool live = sOk[slot][sid];
+    const double scal = d.scal;
 #pragma unroll
     for (int v = 0; v < VPT; ++v) {
-      const int u = tid + T * v;
-      const int col = u / 32, k = u % 32, sid = 32 * kc + k;
-      const bool live = sMode[slot][sid] >= 0;
-      sX[ring][col * kNFPitch + k] = live ? d.scal * x[v] : 0.0;
+      const int col = xcol + v * (T / KC);
+      sX[ring][col * PITCH + xk] = live ? scal * x[v] : 0.0;
       if (p.log_disp && live && x[v] != 0.0)
         atomicAdd(&sDisp[slot][col], p.nmlz[(int64_t)d.tlev * n + sid] * x[v]);
     }
   };
   // table fragments of chunk kc: lane (l16, lg) of k group u holds
-  // A[row 16 rt16 + l16][sid 32 kc + 4 u + lg]
-  auto load_a = [&](const NFPair& d, int kc, int slot, double (&a)[NRT][8]) {
+  // A[row 16 rt16 + l16][sid KC kc + KU lg + u] (a lane's particles adjacent, so
+  // that their rows and densities come in 16-byte LDS reads).  A row without a
+  // target reads another's entries: its sums go nowhere.
+  int rowA[NRT];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int m = sMode[slot][32 * kc + 4 * u + lg];
+  for (int rt = 0; rt < NRT; ++rt) rowA[rt] = 8 * max(tmA[rt], 0);
+  double ac[NRT][KU];
+  auto base_of = [&](const NFPair& d) {
+    const int lo = __builtin_amdgcn_readfirstlane((int)(unsigned)d.dbase);
+    const int hi = __builtin_amdgcn_readfirstlane((int)(d.dbase >> 32));
+    return reinterpret_cast<const char*>(p.dense + ((int64_t)hi << 32 | (unsigned)lo));
+  };
+  typedef __attribute__((ext_vector_type(4))) int int4_t;
+  typedef __attribute__((ext_vector_type(2))) double double2_t;
+  // the lane's particles 4 g .. 4 g + 3 of chunk kc
+  auto rows_of = [&](int kc, int k, int g) {
+    return *reinterpret_cast<const int4_t*>(&sRow[k % 3][KC * kc + KU * lg + 4 * g]);
+  };
+  auto load_a = [&](const char* D, int row, int u) {
 #pragma unroll
-      for (int rt = 0; rt < NRT; ++rt) {
-        double v = 0.0;
-        if (m >= 0 && tmA[rt] >= 0) v = p.dense[d.dbase + (int64_t)m * n + tmA[rt]];
-        a[rt][u] = v == v ? v : 0.0;  // NaN: no entry
-      }
-    }
+    for (int rt = 0; rt < NRT; ++rt)
+      ac[rt][u] = *reinterpret_cast<const double*>(D + (unsigned)(row + rowA[rt]));
   };
 
-  nf_doublex4 yacc[NRT][4];
+  nf_doublex4 yacc[NRT][NC];
 #pragma unroll
   for (int rt = 0; rt < NRT; ++rt)
 #pragma unroll
-    for (int c = 0; c < 4; ++c) yacc[rt][c] = nf_doublex4{0.0, 0.0, 0.0, 0.0};
+    for (int c = 0; c < NC; ++c) yacc[rt][c] = nf_doublex4{0.0, 0.0, 0.0, 0.0};
 
-  NFPair pdC{}, pdN{};
-  double ac[NRT][8], an[NRT][8];
+  double x[VPT] = {};
   const int total = npairs * nkc;
   if (total > 0) {
-    pdC = nf_pair(p, l0, ct);
-    if (tid == 0 && !pdC.ok && p.err) atomicOr(p.err, 1);
-    prep_pair(pdC, 0);
-    if (npairs > 1) {
-      pdN = nf_pair(p, l0 + 1, ct);
-      prep_pair(pdN, 1);
-    }
+    make_pairs(0);
+    make_pairs(1);
     __syncthreads();
-    double x[VPT];
-    load_x(pdC, 0, x);
-    store_x(pdC, 0, 0, 0, x);
-    load_a(pdC, 0, 0, ac);
+    put_mode(0, mode_of(0));
+    put_mode(1, mode_of(1));
+    __syncthreads();
+    load_x(pair(0), 0, x);
+    const char* D = base_of(pair(0));
+#pragma unroll
+    for (int u = 0; u < KU; ++u) load_a(D, rows_of(0, 0, u / 4)[u % 4], u);
+    store_x(pair(0), 0, 0, 0, x);
   }
   __syncthreads();
 
-  for (int it = 0; it < total; ++it) {
-    const int k = it / nkc, kc = it % nkc;
-    if (kc == 0 && k > 0) {  // pair k begins: the next pair's descriptor and modes
-      pdC = pdN;
-      if (tid == 0 && !pdC.ok && p.err) atomicOr(p.err, 1);
-      if (k + 1 < npairs) {
-        pdN = nf_pair(p, l0 + k + 1, ct);
-        prep_pair(pdN, (k + 1) & 1);
-      }
-      if (nkc == 1) __syncthreads();  // read within this same iteration
-    }
+  for (int it = 0, k = 0, kc = 0; it < total; ++it) {
     const bool has_next = it + 1 < total;
     const bool pair_end = kc + 1 == nkc;
-    const int nk = pair_end ? k + 1 : k, nkc_ = pair_end ? 0 : kc + 1;
-    const NFPair& pdX = pair_end ? pdN : pdC;
-    double x[VPT];
-    if (has_next) {
-      load_x(pdX, nkc_, x);
-      load_a(pdX, nkc_, nk & 1, an);
+    // the chunk to load: the next one, or this one again after the last
+    const int kn = pair_end && has_next ? k + 1 : k, kcn = !has_next ? kc : (pair_end ? 0 : kc + 1);
+    int m2 = -1;
+    if (kc == 0) {
+      // the block after the one entered, into the slot of the one left
+      if (k > 0 && k % kNFPairs == 0) make_pairs(k / kNFPairs + 1);
+      m2 = mode_of(k + 2);
     }
-    const double* rX = sX[it & 1];
+    load_x(pair(kn), kcn, x);
+    const char* Dn = base_of(pair(kn));
+    const double* rX = &sX[it & 1][l16 * PITCH + KU * lg];
+    auto mul = [&](auto finite) {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      double bx[4];
+      for (int g = 0; g < KU / 4; ++g) {
+        const int4_t rows = rows_of(kcn, kn, g);
 #pragma unroll
-      for (int c = 0; c < 4; ++c) bx[c] = rX[(16 * c + l16) * kNFPitch + 4 * u + lg];
+        for (int h = 0; h < 4; ++h) {
+          const int u = 4 * g + h;
+          double bx[NC];
 #pragma unroll
-      for (int rt = 0; rt < NRT; ++rt)
-        if (rt == 0 || rows_rt1)  // a second row tile past the box's targets is skipped
+          for (int c = 0; c < NC; ++c)
+            bx[c] = (*reinterpret_cast<const double2_t*>(rX + 16 * c * PITCH + (u & ~1)))[u & 1];
+          bool ok = true;
+          if constexpr (!decltype(finite)::value) ok = sOk[k % 3][KC * kc + KU * lg + u];
 #pragma unroll
-          for (int c = 0; c < 4; ++c)
-            yacc[rt][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(ac[rt][u], bx[c], yacc[rt][c], 0, 0, 0);
-    }
+          for (int rt = 0; rt < NRT; ++rt)
+            if (rt == 0 || rows_rt1) {  // a second row tile past the box's targets is skipped
+              double a = ac[rt][u];
+              if constexpr (!decltype(finite)::value) a = ok && a == a ? a : 0.0;  // NaN: no entry
+#pragma unroll
+              for (int c = 0; c < NC; ++c)
+                yacc[rt][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bx[c], yacc[rt][c], 0, 0, 0);
+            }
+          load_a(Dn, rows[h], u);  // in place: a chunk ahead
+        }
+        // (else all groups' LDS reads move up and their registers spill)
+        if constexpr (NRT * NC >= 4) __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    // a finite table needs no look at its entries: the densities are zero
+    // where no source is
+    if (finite) mul(std::true_type{});
+    else mul(std::false_type{});
     if (pair_end && p.log_disp) {
+      const double dscale = pair(k).dscale;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const double ds = pdC.dscale * sDisp[k & 1][16 * c + l16];
+      for (int c = 0; c < NC; ++c) {
+        const double ds = dscale * sDisp[k % 3][16 * c + l16];
 #pragma unroll
         for (int rt = 0; rt < NRT; ++rt)
 #pragma unroll
           for (int e = 0; e < 4; ++e) yacc[rt][c][e] += ds;
       }
     }
-    if (has_next) {
-#pragma unroll
-      for (int rt = 0; rt < NRT; ++rt)
-#pragma unroll
-        for (int u = 0; u < 8; ++u) ac[rt][u] = an[rt][u];
-      store_x(pdX, nkc_, nk & 1, (it + 1) & 1, x);
-    }
+    if (kc == 0) put_mode(k + 2, m2);
+    if (has_next) store_x(pair(kn), kcn, kn, (it + 1) & 1, x);
     __syncthreads();
+    k = kn;
+    kc = kcn;
   }
 
   // outputs: lane holds rows 16 rt16 + lg + 4 e, column 16 c + l16
@@ -486,7 +543,7 @@ __global__ void __launch_bounds__(64 * W) near_field_mfma_kernel(const NFParams 
       const int m = p.tgt_ids[tbeg + row];
       if ((unsigned)m >= (unsigned)n) continue;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
+      for (int c = 0; c < NC; ++c) {
         const int col = 16 * c + l16;
         if (col < rc) p.y[(int64_t)(r0 + col) * p.ldy + tbeg + row] = yacc[rt][c][e];
       }
@@ -500,7 +557,8 @@ template <typename IdxT>
 __global__ void __launch_bounds__(256)
 dense_table_kernel(int n, int n_cases, int n_tables, int vw, const IdxT* __restrict__ rowmap,
                    const uint16_t* __restrict__ ranks, const int32_t* __restrict__ offs,
-                   const double* __restrict__ table, int64_t n_entries, double* __restrict__ D) {
+                   const double* __restrict__ table, int64_t n_entries, double* __restrict__ D,
+                   int* __restrict__ not_finite) {
   const int64_t nn = (int64_t)n * n;
   const int64_t total = (int64_t)n_tables * n_cases * nn;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
@@ -514,6 +572,7 @@ dense_table_kernel(int n, int n_cases, int n_tables, int vw, const IdxT* __restr
     const double* T = table + ((int64_t)lev * n_entries + offs[ranks[c]] + rel) * vw;
     D[i * vw] = sg * T[0];
     if (vw == 2) D[i * vw + 1] = sg * T[1];
+    if (!isfinite(T[0])) atomicOr(not_finite, 1);
   }
 }
 
@@ -526,21 +585,67 @@ static hipError_t ensure_dense(const vl1_payload* pl, hipStream_t s) {
   const int64_t total = (int64_t)pl->n_tables * pl->n_cases * pl->n * pl->n;
   hipError_t e = pl->dense.alloc((size_t)total * vw * sizeof(double));
   if (e != hipSuccess) return e;
+  DevBuf flag;  // an entry is not finite
+  int not_finite = 0;
+  e = upload(flag, &not_finite, sizeof(int), s);
+  if (e != hipSuccess) {
+    pl->dense.release();
+    return e;
+  }
   const int grid = (int)std::min<int64_t>((total + 255) / 256, 65536);
   if (pl->rowmap_u16)
     hipLaunchKernelGGL(dense_table_kernel<uint16_t>, dim3(grid), dim3(256), 0, s, pl->n,
                        pl->n_cases, pl->n_tables, vw, pl->rowmap.as<uint16_t>(),
                        pl->ranks.as<uint16_t>(), pl->offs.as<int32_t>(), pl->table.as<double>(),
-                       pl->n_entries, pl->dense.as<double>());
+                       pl->n_entries, pl->dense.as<double>(), flag.as<int>());
   else
     hipLaunchKernelGGL(dense_table_kernel<int32_t>, dim3(grid), dim3(256), 0, s, pl->n,
                        pl->n_cases, pl->n_tables, vw, pl->rowmap.as<int32_t>(),
                        pl->ranks.as<uint16_t>(), pl->offs.as<int32_t>(), pl->table.as<double>(),
-                       pl->n_entries, pl->dense.as<double>());
+                       pl->n_entries, pl->dense.as<double>(), flag.as<int>());
   e = hipGetLastError();
+  if (e == hipSuccess) e = hipMemcpyAsync(&not_finite, flag.ptr, sizeof(int), hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) pl->dense.release();
+  else pl->dense_finite = !not_finite;
   return e;
+}
+
+// Column tiles per workgroup: the split of the densities with the least work,
+// columns past the last density included.  A wider tile reads each table
+// fragment less often; 16 densities cost, against wider tiles per 16 columns
+// (us, uniform trees): 3D q = 5, 512 boxes 207, 180 (2 tiles), 160 (4); 3D q =
+// 4, 4096 boxes 404, 397, 368; 2D q = 4, 4096 boxes 91, 90, 125 (registers of
+// its single wave: boxes of up to two waves take one tile).
+// Chunks of 64 source particles where they divide the box and the columns are
+// few (the registers of four column tiles leave room for 32).
+template <int W, int NRT>
+static void launch_nf_mfma(const NFParams& prm, int KP, int n_tgt_boxes, int finite,
+                           hipStream_t s) {
+  const int t16 = (prm.n_rhs + 15) / 16;
+  int nc = 1;
+  if (W >= 4) {
+    const double c2 = W >= 8 ? 1.75 : 1.97, c4 = W >= 8 ? 3.1 : 3.65;
+    const double cost1 = t16, cost2 = (t16 + 1) / 2 * c2, cost4 = (t16 + 3) / 4 * c4;
+    nc = cost4 <= cost1 && cost4 <= cost2 ? 4 : (cost2 <= cost1 ? 2 : 1);
+  }
+  const dim3 grid((n_tgt_boxes + 7) / 8 * 8, (t16 + nc - 1) / nc);
+  auto go = [&](auto ncc, auto kcc) {
+    hipLaunchKernelGGL((near_field_mfma_kernel<W, NRT, decltype(ncc)::value, decltype(kcc)::value>),
+                       grid, dim3(64 * W), 0, s, prm, KP, n_tgt_boxes, finite);
+  };
+  constexpr std::integral_constant<int, 1> n1{};
+  constexpr std::integral_constant<int, 32> k32{};
+  if constexpr (W < 4) {
+    go(n1, k32);
+  } else {
+    constexpr std::integral_constant<int, 2> n2{};
+    constexpr std::integral_constant<int, 64> k64{};
+    const bool wide = KP % 64 == 0;
+    if (nc == 1) wide ? go(n1, k64) : go(n1, k32);
+    else if (nc == 2) wide ? go(n2, k64) : go(n2, k32);
+    else go(std::integral_constant<int, 4>{}, k32);
+  }
 }
 
 template <typename IdxT, int RC, bool CPLX, bool DENSE>
@@ -710,28 +815,24 @@ extern "C" int vl1_near_field_f64(const vl1_payload* pl, const vl1_near_field_ar
     prm.dense = pl->dense.as<double>();
   }
   prm.n_cases = pl->n_cases;
-  // FP64-MFMA form: real tables, boxes of at most 256 nodes, 16 or more
-  // densities (a pass always computes 64 columns), and no missing entry
-  // under the log displacement (VL1_PLAIN_KERNEL=scalar selects the scalar
-  // kernel below)
+  // FP64-MFMA form: real tables, boxes of at most 256 nodes, 5 or more
+  // densities (16 columns are computed whatever the count: at 8 densities, 3D
+  // q = 4, 4096 boxes 1417 us on the scalar kernel, 404 here; 2D q = 6 337 and
+  // 230; at 4 the scalar kernel takes 162 there), and no missing entry under
+  // the log displacement (VL1_PLAIN_KERNEL=scalar selects the scalar kernel
+  // below)
   const char* kern_env = std::getenv("VL1_PLAIN_KERNEL");
   const bool force_scalar = kern_env && std::string(kern_env) == "scalar";
-  if (dense && !force_scalar && !pl->is_complex && pl->n <= kNFMaxK && a->n_rhs >= 16 &&
+  if (dense && !force_scalar && !pl->is_complex && pl->n <= kNFMaxK && a->n_rhs >= 5 &&
       !(pl->has_missing && prm.log_disp)) {
     const int m16 = (pl->n + 15) / 16;
     const int KP = (pl->n + 31) / 32 * 32;
-    const dim3 grid(a->n_tgt_boxes, (a->n_rhs + 63) / 64);
     hipStream_t st = (hipStream_t)stream;
-    if (m16 <= 1)
-      hipLaunchKernelGGL((near_field_mfma_kernel<1, 1>), grid, dim3(64), 0, st, prm, KP);
-    else if (m16 <= 2)
-      hipLaunchKernelGGL((near_field_mfma_kernel<2, 1>), grid, dim3(128), 0, st, prm, KP);
-    else if (m16 <= 4)
-      hipLaunchKernelGGL((near_field_mfma_kernel<4, 1>), grid, dim3(256), 0, st, prm, KP);
-    else if (m16 <= 8)
-      hipLaunchKernelGGL((near_field_mfma_kernel<8, 1>), grid, dim3(512), 0, st, prm, KP);
-    else
-      hipLaunchKernelGGL((near_field_mfma_kernel<8, 2>), grid, dim3(512), 0, st, prm, KP);
+    if (m16 <= 1) launch_nf_mfma<1, 1>(prm, KP, a->n_tgt_boxes, pl->dense_finite, st);
+    else if (m16 <= 2) launch_nf_mfma<2, 1>(prm, KP, a->n_tgt_boxes, pl->dense_finite, st);
+    else if (m16 <= 4) launch_nf_mfma<4, 1>(prm, KP, a->n_tgt_boxes, pl->dense_finite, st);
+    else if (m16 <= 8) launch_nf_mfma<8, 1>(prm, KP, a->n_tgt_boxes, pl->dense_finite, st);
+    else launch_nf_mfma<8, 2>(prm, KP, a->n_tgt_boxes, pl->dense_finite, st);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess)
       return fail(VL1_E_HIP, std::string("near_field_mfma launch: ") + hipGetErrorString(e));

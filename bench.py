@@ -169,17 +169,16 @@ class F64Runner:
         self.capi.check(self.L.vl1_near_field_f64(self.payload.handle, self.args, stream_handle))
 
 
-# declared FP64 work of the segmented table build, 3D Laplace q=6: per
-# (chunk, node) the node, 1/r, the weight and 3 x 6 Lagrange values by
-# prefix/suffix products (105 flop); per (entry, node) the basis product and
-# the accumulation (4 flop)
-FLOP_PER_CHUNK_NODE_3D = 105.0
-FLOP_PER_ENTRY_NODE_3D = 4.0
+# declared FP64 work of the table build, 3D Laplace q=6, per target point and
+# node of its nonempty sign blocks: the node and 1/r (13 flop), the weight (2),
+# six basis values by prefix/suffix products into six sums (28), and the outer
+# axes' sums per node (5)
+FLOP_PER_TARGET_NODE_3D = 48.0
 
 
 def table_build_record(rules):
     """Near-field table build, 3D Laplace q=6: every canonical entry of all
-    139 cases (140,496 entries) in one launch of vl1_duffy_build per rule
+    139 cases (140,496 entries) in one vl1_duffy_build_tensor per rule
     (GL tail order, tanh-sinh-fast order); kernel time from HIP events."""
     from volumential_amd.kernels import LaplaceKernel
     from volumential_amd.table import DuffyBuildConfig, NearFieldInteractionTable
@@ -191,18 +190,20 @@ def table_build_record(rules):
         ms = t.last_build_kernel_ms
         ne = t.last_build_node_evals
         rate = ne / (ms * 1e-3)
-        flops = (t.last_build_chunks * t.last_build_n_nodes * FLOP_PER_CHUNK_NODE_3D
-                 + ne * FLOP_PER_ENTRY_NODE_3D)
+        ids = t.reduced_entry_ids
+        key = np.unique(ids // t.n_pairs * t.n_q_points + ids % t.n_q_points)
+        x = t.case_target_points()[:, key // t.n_q_points, key % t.n_q_points]
+        blocks = np.prod((x > 0.0).astype(int) + (x < 2.0), axis=0).sum()  # nonempty
+        flops = blocks * t.last_build_n_nodes / 8 * FLOP_PER_TARGET_NODE_3D
         tf = flops / (ms * 1e-3) / 1e12
         out.append({"rule": [reg, rad], "entries": int(t.reduced_entry_ids.size),
                     "target_point_chunks": int(t.last_build_chunks),
                     "kernel_ms": ms, "build_s": t.last_build_seconds,
                     "node_evals": ne, "node_evals_per_s": rate,
                     "fp64_tflops_declared": tf, "fp64_frac": tf / PEAK_FP64_TFLOPS})
-        log(f"table build rule {reg}/{rad}: kernel {ms:.1f} ms, {rate:.3e} node-evals/s, "
+        log(f"table build rule {reg}/{rad}: kernel {ms:.2f} ms, {rate:.3e} node-evals/s, "
             f"{tf:.1f} TFLOP/s = {out[-1]['fp64_frac'] * 100:.1f} % of FP64 peak (declared "
-            f"{FLOP_PER_CHUNK_NODE_3D:.0f} flop per chunk-node + "
-            f"{FLOP_PER_ENTRY_NODE_3D:.0f} per entry-node)")
+            f"{FLOP_PER_TARGET_NODE_3D:.0f} flop per target point and node)")
     return out
 
 
@@ -1107,7 +1108,7 @@ def run_c5(args):
          "node_evals": r20["node_evals"], "parallelism": "single GPU"},
         {"bound": "fp64 valu", "achieved": r20["fp64_tflops_declared"], "peak": PEAK_FP64_TFLOPS,
          "unit": "TFLOP/s", "frac": r20["fp64_frac"], "traffic": None,
-         "kernel": "duffy_seg_kernel<3, 1, 6>", "kernel_ms": ms,
+         "kernel": "duffy_tensor_kernel<1, 6>", "kernel_ms": ms,
          "flops_per_launch": r20["fp64_tflops_declared"] * 1e12 * ms * 1e-3},
         {}, extra, metric="near-field table build Gnode-evals/s (3D Laplace q=6, all cases)",
         unit="Gnode-evals/s")

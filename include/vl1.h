@@ -421,6 +421,37 @@ typedef struct vl1_duffy_args {
 
 int vl1_duffy_build(const vl1_duffy_args* a, void* stream);
 
+/* The same entries in 3D from the rule's one-dimensional parts (all sign
+ * vectors and axis orders; radial nodes x tail nodes x tail nodes), summed
+ * axis by axis: entries grouped by target point. */
+typedef struct vl1_duffy_tensor_args {
+  int dim;                  /* 3 */
+  int quad_order;
+  int kernel_kind;
+  int deriv_axis;
+  int power;
+  int n_radial;
+  int n_tail;               /* at most 256 */
+  double helmholtz_k;
+  double source_box_extent;
+  int64_t n_targets;
+  int64_t n_entries;
+  int64_t max_entries;      /* entries of a target point at most */
+  /* device pointers */
+  const double* target_points;   /* [3][n_targets] */
+  const int64_t* entry_start;    /* [n_targets + 1] */
+  const int32_t* modes;          /* [n_entries] source mode, axis 0 slowest */
+  const double* radial_x;        /* [n_radial] in (0, 1) */
+  const double* radial_w;
+  const double* tail_x;          /* [n_tail] in (0, 1) */
+  const double* tail_w;
+  const double* interp_nodes;    /* [quad_order] */
+  double* work;                  /* [8][n_entries] (x2 if Helmholtz) */
+  double* result;                /* [n_entries] (x2 interleaved if Helmholtz) */
+} vl1_duffy_tensor_args;
+
+int vl1_duffy_build_tensor(const vl1_duffy_tensor_args* a, void* stream);
+
 /* ------------------------------------------------------------------ */
 /* Helmholtz split correction of list 1.                               */
 /* Replaces eval_direct_helmholtz_split_correction,                    */

@@ -75,6 +75,7 @@ EXPORTED_SYMBOLS = (
     "vl1_csr_builder_fill",
     "vl1_csr_builder_destroy",
     "vl1_duffy_build",
+    "vl1_duffy_build_tensor",
     "vl1_split_correction",
     "vl1_orbit_rows_host",
     "vl1_orbit_signs_host",
@@ -243,6 +244,33 @@ class DuffyArgs(C.Structure):
     ]
 
 
+class DuffyTensorArgs(C.Structure):
+    _fields_ = [
+        ("dim", C.c_int),
+        ("quad_order", C.c_int),
+        ("kernel_kind", C.c_int),
+        ("deriv_axis", C.c_int),
+        ("power", C.c_int),
+        ("n_radial", C.c_int),
+        ("n_tail", C.c_int),
+        ("helmholtz_k", f64),
+        ("source_box_extent", f64),
+        ("n_targets", i64),
+        ("n_entries", i64),
+        ("max_entries", i64),
+        ("target_points", vp),
+        ("entry_start", vp),
+        ("modes", vp),
+        ("radial_x", vp),
+        ("radial_w", vp),
+        ("tail_x", vp),
+        ("tail_w", vp),
+        ("interp_nodes", vp),
+        ("work", vp),
+        ("result", vp),
+    ]
+
+
 class SplitArgs(C.Structure):
     _fields_ = [
         ("dim", C.c_int),
@@ -312,6 +340,7 @@ def lib():
                                 C.c_int, C.POINTER(i32), C.POINTER(f64), vp]
     L.vl1_plan_set_variant.argtypes = [vp, C.c_int, C.c_int, C.c_int, C.c_int]
     L.vl1_duffy_build.argtypes = [C.POINTER(DuffyArgs), vp]
+    L.vl1_duffy_build_tensor.argtypes = [C.POINTER(DuffyTensorArgs), vp]
     L.vl1_split_correction.argtypes = [C.POINTER(SplitArgs), vp]
     L.vl1_csr_builder_create.argtypes = [C.POINTER(vp), C.c_int, C.c_int, vp, vp, C.POINTER(i64), vp]
     L.vl1_csr_builder_fill.argtypes = [vp, vp, vp, vp]

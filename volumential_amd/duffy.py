@@ -39,14 +39,73 @@ def target_point_chunks(table, entry_ids, max_chunk=64):
     return order, np.asarray(starts, dtype=np.int64)
 
 
+def _tensor_values(L, table, entry_ids, regular_order, radial_order, stream):
+    """3D values by sum factorization over the rule's axes
+    (``vl1_duffy_build_tensor``): entries grouped by target point, the rule as
+    its one-dimensional parts."""
+    entry_ids = np.asarray(entry_ids, dtype=np.int64)
+    n = table.n_q_points
+    case, pair = np.divmod(entry_ids, table.n_pairs)
+    mode, node = np.divmod(pair, n)
+    key = case * n + node
+    order = np.argsort(key, kind="stable")
+    ks = key[order]
+    first = np.flatnonzero(np.r_[True, ks[1:] != ks[:-1]])
+    start = np.append(first, ks.size)
+    points = table.case_target_points()[:, ks[first] // n, ks[first] % n]
+    rho, w_rho = quadrature.tanh_sinh_fast(radial_order)
+    eta, w_eta = quadrature.gauss_legendre_01(regular_order)
+    cplx = bool(table.integral_knl.is_complex_valued)
+    vw = 2 if cplx else 1
+    # one upload: points, rule and nodes, then starts and modes
+    d_f = _dev(np.concatenate([points.ravel(), rho, w_rho, eta, w_eta, table.interp_nodes]))
+    d_start, d_mode = _dev(start.astype(np.int64)), _dev(mode[order].astype(np.int32))
+    at = [8 * int(k) for k in np.cumsum([0, points.size, rho.size, rho.size, eta.size, eta.size])]
+    base = d_f.data_ptr()
+    work = torch.empty(9 * vw * ks.size, dtype=torch.float64, device="cuda")
+    out = work[8 * vw * ks.size:]
+    args = _capi.DuffyTensorArgs(
+        dim=3, quad_order=table.quad_order, kernel_kind=int(table.integral_knl.kind),
+        deriv_axis=int(getattr(table.integral_knl, "axis", -1)),
+        power=int(getattr(table.integral_knl.get_base_kernel(), "power", 0)),
+        n_radial=rho.size, n_tail=eta.size,
+        helmholtz_k=float(getattr(table.integral_knl.get_base_kernel(), "k", 0.0)),
+        source_box_extent=table.source_box_extent, n_targets=first.size, n_entries=ks.size,
+        max_entries=int(np.diff(start).max()), target_points=base + at[0],
+        entry_start=d_start.data_ptr(), modes=d_mode.data_ptr(), radial_x=base + at[1],
+        radial_w=base + at[2], tail_x=base + at[3], tail_w=base + at[4],
+        interp_nodes=base + at[5], work=work.data_ptr(), result=out.data_ptr())
+    st = stream if stream is not None else torch.cuda.current_stream()
+    ev0 = torch.cuda.Event(enable_timing=True)
+    ev1 = torch.cuda.Event(enable_timing=True)
+    ev0.record(st)
+    _capi.check(L.vl1_duffy_build_tensor(args, _capi.stream_handle(st)), "vl1_duffy_build_tensor")
+    ev1.record(st)
+    torch.cuda.synchronize()
+    n_nodes = 48 * rho.size * eta.size**2
+    table.last_build_kernel_ms = ev0.elapsed_time(ev1)
+    table.last_build_node_evals = int(ks.size) * n_nodes
+    table.last_build_chunks = int(first.size)
+    table.last_build_n_nodes = n_nodes
+    got = out.cpu().numpy()
+    if cplx:
+        got = got[0::2] + 1j * got[1::2]
+    res = np.empty_like(got)
+    res[order] = got
+    return res
+
+
 def duffy_values(table, entry_ids, regular_order, radial_order, stream=None,
                  segmented=True) -> np.ndarray:
     """Duffy values of ``entry_ids`` (one launch).  ``segmented``: share each
     node's geometry and kernel value among the entries of one target point
-    (the fast form); ``False`` runs one lane per entry."""
+    (the fast form; 3D: axis by axis, ``_tensor_values``); ``False`` runs one
+    lane per entry."""
     if not torch.cuda.is_available():
         raise RuntimeError("the Duffy table build runs on the GPU; no GPU is visible")
     L = _capi.lib()
+    if segmented and table.dim == 3 and np.size(entry_ids) and int(regular_order) <= 256:
+        return _tensor_values(L, table, entry_ids, int(regular_order), int(radial_order), stream)
     nodes = quadrature.duffy_node_set(table.dim, int(regular_order), int(radial_order))
     entry_ids = np.asarray(entry_ids, dtype=np.int64)
     order = None

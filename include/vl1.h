@@ -554,6 +554,19 @@ int vl1_orbit_rows_host(int dim, int q, const uint8_t* perm, const int8_t* sign,
 int vl1_orbit_signs_host(int dim, int q, const uint8_t* perm, const int8_t* sign,
                          const uint8_t* axis_sign_power, const int32_t* s, const int32_t* t,
                          int64_t count, int8_t* out);
+/* Full entry ids (case n^2 + s n + t) of the orbit representatives in
+ * compact-row order (orbit_arithmetic.py:748-790): case_ids / sign / group of
+ * the n_orbits canonical cases ([n_orbits], [n_orbits][dim]), out [count]. */
+int vl1_orbit_representatives_host(int dim, int q, int n_orbits, const int32_t* case_ids,
+                                   const int8_t* sign, const uint8_t* group, int64_t count,
+                                   int64_t* out);
+/* Entry ids grouped by target point key = case n + t (ascending, ids of a
+ * point in the given order): order [count] positions in ids, mode [count]
+ * their source modes, start [n_points + 1], key [n_points]; start and key
+ * hold up to min(count, n_cases n) + 1 values. */
+int vl1_table_groups_host(int64_t n_cases, int64_t n, int64_t count, const int64_t* ids,
+                          int64_t* order, int32_t* mode, int64_t* start, int64_t* key,
+                          int64_t* n_points);
 
 #ifdef __cplusplus
 }

@@ -79,6 +79,8 @@ EXPORTED_SYMBOLS = (
     "vl1_split_correction",
     "vl1_orbit_rows_host",
     "vl1_orbit_signs_host",
+    "vl1_orbit_representatives_host",
+    "vl1_table_groups_host",
 )
 
 vp = C.c_void_p
@@ -347,6 +349,8 @@ def lib():
     L.vl1_csr_builder_destroy.argtypes = [vp]
     L.vl1_orbit_rows_host.argtypes = [C.c_int, C.c_int, vp, vp, vp, vp, vp, i64, vp]
     L.vl1_orbit_signs_host.argtypes = [C.c_int, C.c_int, vp, vp, vp, vp, vp, i64, vp]
+    L.vl1_orbit_representatives_host.argtypes = [C.c_int, C.c_int, C.c_int, vp, vp, vp, i64, vp]
+    L.vl1_table_groups_host.argtypes = [i64, i64, i64, vp, vp, vp, vp, vp, C.POINTER(i64)]
     if L.vl1_abi_version() != 11:
         raise RuntimeError("libvl1.so ABI version mismatch; rebuild the library")
     _lib = L

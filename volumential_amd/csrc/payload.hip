@@ -7,6 +7,8 @@
 //     rowmap[case][s][t] = compact row of (case, s, t) - first row of its orbit
 // so evaluation kernels gather table values without redoing the orbit
 // arithmetic for every (box pair, s, t).
+#include <vector>
+#include <exception>
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -346,6 +348,103 @@ int vl1_orbit_signs_host(int dim, int q, const uint8_t* perm, const int8_t* sign
   int mask = 0;
   for (int a = 0; a < dim; ++a) mask |= (axis_sign_power[a] & 1) << a;
   for (int64_t i = 0; i < count; ++i) out[i] = (int8_t)entry_sign(dim, q, perm, sign, mask, s[i], t[i]);
+  return VL1_OK;
+}
+
+// The axes of a case in group order; codes run over the multisets of each
+// group (nondecreasing), the first group slowest.
+int vl1_orbit_representatives_host(int dim, int q, int n_orbits, const int32_t* case_ids,
+                                   const int8_t* sign, const uint8_t* group, int64_t count,
+                                   int64_t* out) {
+  clear_error();
+  if ((dim != 2 && dim != 3) || q < 1 || n_orbits < 0 || !case_ids || !sign || !group || !out)
+    return fail(VL1_E_ARG, "vl1_orbit_representatives_host: bad argument");
+  int64_t n = 1, pw[3] = {0, 0, 0};  // node stride of an axis
+  for (int a = dim - 1; a >= 0; --a) {
+    pw[a] = n;
+    n *= q;
+  }
+  int64_t pos = 0;
+  for (int o = 0; o < n_orbits; ++o) {
+    const int8_t* sg = sign + (int64_t)o * dim;
+    const uint8_t* gr = group + (int64_t)o * dim;
+    int ax[3], alpha[3], k = 0;
+    bool same[3];  // whether the axis continues the group of the one before
+    for (int g = 0; g < dim; ++g) {
+      bool folded = false;
+      for (int a = 0; a < dim; ++a) folded = folded || (gr[a] == g && sg[a] == 0);
+      bool first = true;
+      for (int a = 0; a < dim; ++a)
+        if (gr[a] == g) {
+          ax[k] = a;
+          alpha[k] = folded ? (q * q + 1) / 2 : q * q;
+          same[k++] = !first;
+          first = false;
+        }
+    }
+    if (k != dim) return fail(VL1_E_ARG, "vl1_orbit_representatives_host: bad axis group");
+    int c[3] = {0, 0, 0};
+    int64_t id[4] = {case_ids[o] * n * n, 0, 0, 0};  // id of the codes so far
+    auto add = [&](int j) { id[j + 1] = id[j] + pw[ax[j]] * ((c[j] / q) * n + c[j] % q); };
+    for (int j = 0; j < dim; ++j) add(j);
+    while (true) {
+      if (pos >= count)
+        return fail(VL1_E_ARG, "vl1_orbit_representatives_host: more entries than the count");
+      out[pos++] = id[dim];
+      int j = dim - 1;
+      while (j >= 0 && c[j] + 1 >= alpha[j]) --j;
+      if (j < 0) break;
+      ++c[j];
+      add(j);
+      for (++j; j < dim; ++j) {
+        c[j] = same[j] ? c[j - 1] : 0;
+        add(j);
+      }
+    }
+  }
+  if (pos != count)
+    return fail(VL1_E_ARG, "vl1_orbit_representatives_host: fewer entries than the count");
+  return VL1_OK;
+}
+
+int vl1_table_groups_host(int64_t n_cases, int64_t n, int64_t count, const int64_t* ids,
+                          int64_t* order, int32_t* mode, int64_t* start, int64_t* key,
+                          int64_t* n_points) {
+  clear_error();
+  if (n_cases < 1 || n < 1 || n > INT32_MAX || count < 0 || (count && !ids) || !order || !mode ||
+      !start || !key || !n_points)
+    return fail(VL1_E_ARG, "vl1_table_groups_host: bad argument");
+  const int64_t n_keys = n_cases * n;
+  try {
+    std::vector<int64_t> at(n_keys + 1, 0);
+    std::vector<int64_t> k_of(count);
+    std::vector<int32_t> m_of(count);
+    for (int64_t i = 0; i < count; ++i) {
+      if (ids[i] < 0 || ids[i] >= n_keys * n)
+        return fail(VL1_E_ARG, "vl1_table_groups_host: entry id out of range");
+      const int64_t a = ids[i] / n, c = a / n;
+      k_of[i] = c * n + (ids[i] - a * n);
+      m_of[i] = (int32_t)(a - c * n);
+      ++at[k_of[i] + 1];
+    }
+    int64_t p = 0;
+    for (int64_t k = 0; k < n_keys; ++k) {
+      if (at[k + 1]) {
+        start[p] = at[k];
+        key[p++] = k;
+      }
+      at[k + 1] += at[k];
+    }
+    start[p] = count;
+    *n_points = p;
+    for (int64_t i = 0; i < count; ++i) {
+      const int64_t to = at[k_of[i]]++;
+      order[to] = i;
+      mode[to] = m_of[i];
+    }
+  } catch (const std::exception& e) {
+    return fail(VL1_E_ARG, std::string("vl1_table_groups_host: ") + e.what());
+  }
   return VL1_OK;
 }
 

@@ -7,6 +7,8 @@ geometry, uploads the node set once, launches one kernel over all entries.
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import torch
 
@@ -43,34 +45,35 @@ def _tensor_values(L, table, entry_ids, regular_order, radial_order, stream):
     """3D values by sum factorization over the rule's axes
     (``vl1_duffy_build_tensor``): entries grouped by target point, the rule as
     its one-dimensional parts."""
-    entry_ids = np.asarray(entry_ids, dtype=np.int64)
-    n = table.n_q_points
-    case, pair = np.divmod(entry_ids, table.n_pairs)
-    mode, node = np.divmod(pair, n)
-    key = case * n + node
-    order = np.argsort(key, kind="stable")
-    ks = key[order]
-    first = np.flatnonzero(np.r_[True, ks[1:] != ks[:-1]])
-    start = np.append(first, ks.size)
-    points = table.case_target_points()[:, ks[first] // n, ks[first] % n]
+    entry_ids = np.ascontiguousarray(entry_ids, dtype=np.int64)
+    n, count = table.n_q_points, entry_ids.size
+    order, mode = np.empty(count, dtype=np.int64), np.empty(count, dtype=np.int32)
+    start, key = np.empty((2, min(count, table.n_cases * n) + 1), dtype=np.int64)
+    n_points = ctypes.c_int64()
+    _capi.check(L.vl1_table_groups_host(
+        table.n_cases, n, count, entry_ids.ctypes.data, order.ctypes.data, mode.ctypes.data,
+        start.ctypes.data, key.ctypes.data, ctypes.byref(n_points)), "vl1_table_groups_host")
+    start, key = start[:n_points.value + 1], key[:n_points.value]
+    cases, case = np.unique(key // n, return_inverse=True)
+    points = table.case_target_points(cases)[:, case, key % n]
     rho, w_rho = quadrature.tanh_sinh_fast(radial_order)
     eta, w_eta = quadrature.gauss_legendre_01(regular_order)
     cplx = bool(table.integral_knl.is_complex_valued)
     vw = 2 if cplx else 1
     # one upload: points, rule and nodes, then starts and modes
     d_f = _dev(np.concatenate([points.ravel(), rho, w_rho, eta, w_eta, table.interp_nodes]))
-    d_start, d_mode = _dev(start.astype(np.int64)), _dev(mode[order].astype(np.int32))
+    d_start, d_mode = _dev(start), _dev(mode)
     at = [8 * int(k) for k in np.cumsum([0, points.size, rho.size, rho.size, eta.size, eta.size])]
     base = d_f.data_ptr()
-    work = torch.empty(9 * vw * ks.size, dtype=torch.float64, device="cuda")
-    out = work[8 * vw * ks.size:]
+    work = torch.empty(9 * vw * count, dtype=torch.float64, device="cuda")
+    out = work[8 * vw * count:]
     args = _capi.DuffyTensorArgs(
         dim=3, quad_order=table.quad_order, kernel_kind=int(table.integral_knl.kind),
         deriv_axis=int(getattr(table.integral_knl, "axis", -1)),
         power=int(getattr(table.integral_knl.get_base_kernel(), "power", 0)),
         n_radial=rho.size, n_tail=eta.size,
         helmholtz_k=float(getattr(table.integral_knl.get_base_kernel(), "k", 0.0)),
-        source_box_extent=table.source_box_extent, n_targets=first.size, n_entries=ks.size,
+        source_box_extent=table.source_box_extent, n_targets=key.size, n_entries=count,
         max_entries=int(np.diff(start).max()), target_points=base + at[0],
         entry_start=d_start.data_ptr(), modes=d_mode.data_ptr(), radial_x=base + at[1],
         radial_w=base + at[2], tail_x=base + at[3], tail_w=base + at[4],
@@ -84,8 +87,8 @@ def _tensor_values(L, table, entry_ids, regular_order, radial_order, stream):
     torch.cuda.synchronize()
     n_nodes = 48 * rho.size * eta.size**2
     table.last_build_kernel_ms = ev0.elapsed_time(ev1)
-    table.last_build_node_evals = int(ks.size) * n_nodes
-    table.last_build_chunks = int(first.size)
+    table.last_build_node_evals = count * n_nodes
+    table.last_build_chunks = int(key.size)
     table.last_build_n_nodes = n_nodes
     got = out.cpu().numpy()
     if cplx:

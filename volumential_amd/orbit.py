@@ -34,7 +34,6 @@ entry ids + values) map onto the same rows.
 
 from __future__ import annotations
 
-import itertools
 import math
 from dataclasses import dataclass
 from functools import lru_cache
@@ -211,51 +210,20 @@ def kernel_case_metadata(kernel, quad_order: int) -> ArithmeticCaseMetadata:
     return build_case_metadata(kernel.dim, quad_order, fixed, power)
 
 
-def _combos_with_replacement(alpha: int, k: int) -> np.ndarray:
-    return np.asarray(
-        list(itertools.combinations_with_replacement(range(alpha), k)), dtype=np.int64
-    ).reshape(-1, k)
-
-
 def enumerate_representatives(meta: ArithmeticCaseMetadata) -> np.ndarray:
     """Full entry ids of the canonical representatives in compact-row order.
 
     ``orbit_arithmetic.py:748-790``.  Full id = ``case*n^2 + s*n + t``.
     """
-    dim, q = meta.dim, meta.quad_order
-    n = q**dim
+    from . import _capi
+
+    cases = np.ascontiguousarray(meta.canonical_case_ids, dtype=np.int32)
+    sign = np.ascontiguousarray(meta.case_axis_sign[cases], dtype=np.int8)
+    group = np.ascontiguousarray(meta.case_axis_group[cases], dtype=np.uint8)
     out = np.empty(meta.n_compact_entries, dtype=np.int64)
-    pos = 0
-    for rank, cid in enumerate(meta.canonical_case_ids.tolist()):
-        groups = meta.case_axis_group[cid]
-        signs = meta.case_axis_sign[cid]
-        group_axes = []
-        group_opts = []
-        for gid in range(int(groups.max()) + 1):
-            axes = np.flatnonzero(groups == gid)
-            alpha = group_alphabet(q, bool(np.any(signs[axes] == 0)))
-            group_axes.append(axes)
-            group_opts.append(_combos_with_replacement(alpha, axes.size))
-        # itertools.product order over groups: first group slowest
-        sizes = [o.shape[0] for o in group_opts]
-        total = int(np.prod(sizes))
-        idx = np.indices(sizes).reshape(len(sizes), -1)
-        s_axes = np.zeros((total, dim), dtype=np.int64)
-        t_axes = np.zeros((total, dim), dtype=np.int64)
-        for g, axes in enumerate(group_axes):
-            codes = group_opts[g][idx[g]]  # (total, k)
-            for j, ax in enumerate(axes):
-                s_axes[:, ax] = codes[:, j] // q
-                t_axes[:, ax] = codes[:, j] % q
-        s_id = np.zeros(total, dtype=np.int64)
-        t_id = np.zeros(total, dtype=np.int64)
-        for ax in range(dim):
-            s_id = s_id * q + s_axes[:, ax]
-            t_id = t_id * q + t_axes[:, ax]
-        out[pos : pos + total] = cid * n * n + s_id * n + t_id
-        assert pos == int(meta.case_value_offsets[rank])
-        pos += total
-    assert pos == out.size
+    _capi.check(_capi.lib().vl1_orbit_representatives_host(
+        meta.dim, meta.quad_order, cases.size, cases.ctypes.data, sign.ctypes.data,
+        group.ctypes.data, out.size, out.ctypes.data), "vl1_orbit_representatives_host")
     return out
 
 

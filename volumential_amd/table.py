@@ -83,11 +83,14 @@ class NearFieldInteractionTable:
         """1D interpolation nodes of the source box (last-axis nodes)."""
         return np.ascontiguousarray(self.q_points[: self.quad_order, self.dim - 1])
 
-    def case_target_points(self) -> np.ndarray:
-        """``[dim, n_cases, n_q_points]`` target node coordinates per case."""
+    def case_target_points(self, cases=None) -> np.ndarray:
+        """``[dim, n_cases, n_q_points]`` target node coordinates per case
+        (of the list ``cases``, all by default)."""
         vecs = np.asarray(self.interaction_case_vecs, dtype=np.float64)
+        if cases is not None:
+            vecs = vecs[cases]
         offsets = (self.q_points - self.center).T  # [dim, n]
-        out = np.empty((self.dim, self.n_cases, self.n_q_points))
+        out = np.empty((self.dim, len(vecs), self.n_q_points))
         for c, vec in enumerate(vecs):
             cntr = 0.5 * self.source_box_extent + vec / 4.0 * self.source_box_extent
             size = gallery.target_box_size(vec)

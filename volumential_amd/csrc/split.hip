@@ -13,12 +13,21 @@
 // pair value is +(-)(x_a - y_a) R'(r) / r, and self pairs give 0 (the
 // reference's limit for a wrapped chain, 5293-5300).
 //
-// GPU mapping: one workgroup per target box.  Each listed source box's
-// point coordinates and complex strengths (a chunk of RC densities) are
-// staged in LDS; a lane owns one target point and a share of the source
-// points; R is evaluated once per (target, source) pair and applied to all
-// RC densities; partial sums are reduced through LDS.  The series
-// coefficients sit in LDS for the whole launch.
+// GPU mapping: one workgroup per target box.  The sources of its boxes, up to
+// 64 boxes' at a time, are staged in LDS in chunks regardless of box limits
+// (coordinates and the complex strengths of RC densities); a lane owns one
+// target point and a share of the sources; R is evaluated once per (target,
+// source) pair and applied to all RC densities; partial sums are reduced
+// through LDS.
+// Bound: FP64 VALU, about 2 N + 60 instructions per pair for a real wave
+// number.  The series coefficients are kernel arguments, so that a term is one
+// instruction with a scalar operand; from LDS each wave took 32 bytes per lane
+// and term, and the LDS return path (128 bytes per clock and CU) was the bound:
+// 2D, 4096 boxes of 36 points, k = 40, one density 509 us, 147 us so
+// (251 us with the library's log).
+// A lane takes four sources at a time for the same coefficient.  Where the
+// imaginary parts are a quarter of the real log series (real k, order 1), that
+// chain serves both.
 #include <algorithm>
 #include <cmath>
 #include <complex>
@@ -38,11 +47,10 @@ constexpr int kSplitBlock = 256;
 constexpr int kPairSeries = 0, kPairDeriv = 1, kPairLegacy = 2, kPairLegacyDeriv = 3;
 
 struct SplitParams {
-  int dim, n_rhs, nt, n_terms, chunk, ncoef;
+  int dim, n_rhs, nt, n_terms, chunk;
   double k_re, k_im;   // wave number (legacy subtraction)
   int deriv_axis;      // derivative wrapper (DERIV kernels): axis and sign
   double deriv_sign;   // +1 target derivative, -1 source derivative
-  const double* coef;  // split_coefficients / split_derivative_coefficients
   const int32_t* target_boxes;
   const int32_t* nbr_starts;
   const int32_t* nbr_lists;
@@ -60,22 +68,119 @@ struct SplitParams {
   int64_t ldr;
 };
 
-template <int DIM, int RC, int MODE>
-__global__ void __launch_bounds__(kSplitBlock) split_correction_kernel(const SplitParams p) {
+// split_coefficients / split_derivative_coefficients: 2 + 4 values a term at most
+struct SplitCoef {
+  double v[2 + 4 * kSplitMaxTerms];
+};
+
+constexpr int kSplitBoxes = 64;  // source boxes staged together
+constexpr int kSplitPairs = 4;   // sources per lane and pass over the series
+
+// log x for x > 0 by a table of 64 reciprocals (Tang's method): x = 2^e m, m in
+// [1/2, 1), c the midpoint of m's 1/128 interval, log x = e log 2 - log(1/c) +
+// log1p(m / c - 1), the last a polynomial of degree 7 (|m / c - 1| <= 1/128:
+// truncated at 2e-18).  Within 1.2 units of the last place of max(1, |log x|), in 15
+// instructions; the library's log took more than half of the kernel's time.
+struct SplitLog {
+  double inv, log_c;  // 1 / c rounded, -log of that
+};
+constexpr int kSplitLogs = 64;
+__device__ inline void split_log_table(SplitLog* t, int i) {
+  const double inv = 1.0 / (0.5 + (i + 0.5) / (2.0 * kSplitLogs));
+  t[i] = SplitLog{inv, -log(inv)};
+}
+__device__ __forceinline__ double split_log(double x, const SplitLog* t) {
+  const double m = __builtin_amdgcn_frexp_mant(x);
+  const int e = __builtin_amdgcn_frexp_exp(x);
+  const SplitLog q = t[(__double2hiint(m) >> 14) & (kSplitLogs - 1)];
+  const double r = fma(m, q.inv, -1.0), r2 = r * r;
+  double p = fma(r, 1.0 / 7.0, -1.0 / 6.0);
+  p = fma(p, r, 1.0 / 5.0);
+  p = fma(p, r, -1.0 / 4.0);
+  p = fma(p, r, 1.0 / 3.0);
+  p = fma(p, r, -1.0 / 2.0);
+  return fma((double)e, M_LN2, q.log_c) + fma(p, r2, r);
+}
+
+// The series of remainder_value / remainder_radial_derivative at U points, with
+// each coefficient read once.  QUARTER (2D): s_n real and Im b_n = s_n / 4.
+template <int DIM, bool DERIV, bool QUARTER, int U>
+__device__ __forceinline__ void split_series(const double (&r2)[U], const SplitCoef& cf,
+                                             const SplitLog* logs, int N, double (&vr)[U],
+                                             double (&vi)[U]) {
+  if constexpr (DIM == 2) {
+    constexpr int base = DERIV ? 0 : 2;
+    double ar[U], ai[U], br[U], bi[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) ar[u] = ai[u] = br[u] = bi[u] = 0.0;
+    for (int n = N; n >= 1; --n) {
+      const double* c = cf.v + base + 4 * (n - 1);
+      const double c0 = c[0], c1 = c[1], c2 = c[2], c3 = c[3];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        ar[u] = fma(ar[u], r2[u], c0);
+        br[u] = fma(br[u], r2[u], c2);
+        if constexpr (!QUARTER) {
+          ai[u] = fma(ai[u], r2[u], c1);
+          bi[u] = fma(bi[u], r2[u], c3);
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const double lg = r2[u] > 0.0 ? -0.25 / M_PI * split_log(r2[u], logs) : 0.0;  // -log(r) / (2 pi)
+      if constexpr (QUARTER) bi[u] = 0.25 * ar[u];
+      const double w = DERIV ? 1.0 : r2[u];
+      vr[u] = w * br[u] + lg * (w * ar[u]);
+      vi[u] = QUARTER ? w * bi[u] : w * bi[u] + lg * (w * ai[u]);
+      if constexpr (!DERIV) {
+        vr[u] += cf.v[0];
+        vi[u] += cf.v[1];
+      }
+    }
+  } else {
+    double r[U], pr[U], pi[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      r[u] = sqrt(r2[u]);
+      pr[u] = pi[u] = 0.0;
+    }
+    for (int n = DERIV ? N - 1 : N; n >= 1; --n) {
+      const double c0 = cf.v[2 * (n - 1)], c1 = cf.v[2 * (n - 1) + 1];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        pr[u] = fma(pr[u], r[u], c0);
+        pi[u] = fma(pi[u], r[u], c1);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const double w = DERIV ? 1.0 / r[u] : 1.0;
+      vr[u] = w * pr[u];
+      vi[u] = w * pi[u];
+    }
+  }
+}
+
+template <int DIM, int RC, int MODE, bool QUARTER>
+__global__ void __launch_bounds__(kSplitBlock)
+    split_correction_kernel(const SplitParams p, const SplitCoef cf) {
   constexpr bool DERIV = MODE == kPairDeriv || MODE == kPairLegacyDeriv;
-  extern __shared__ double smem[];
+  constexpr bool LEGACY = MODE == kPairLegacy || MODE == kPairLegacyDeriv;
+  constexpr int U = LEGACY ? 1 : kSplitPairs;
+  extern __shared__ __align__(16) double smem[];
+  __shared__ int sOff[kSplitBoxes + 1], sBeg[kSplitBoxes];
+  __shared__ __align__(16) SplitLog sLog[kSplitLogs];
   const int N = p.n_terms;
-  const int ncoef = p.ncoef;
   const int P = kSplitBlock / p.nt;
-  double* sC = smem;                 // series coefficients
-  double* sX = sC + ncoef;           // source coordinates [DIM][chunk]
   const int chunk = p.chunk;         // source points staged per pass
-  double* sF = sX + DIM * chunk;     // strengths [chunk][RC][2]
-  double* red = sX;                  // part sums [256][RC][2], after the staging is done
+  double* sF = smem;                 // strengths [chunk][RC][2]
+  double* sX = sF + (size_t)chunk * RC * 2;  // source coordinates [DIM][chunk]
+  double* red = smem;                // part sums [256][RC][2], after the staging is done
   const int tid = threadIdx.x;
   const int lane_t = tid % p.nt;
   const int part = tid / p.nt;
-  for (int i = tid; i < ncoef; i += kSplitBlock) sC[i] = p.coef[i];
+  if (DIM == 2 && tid < kSplitLogs) split_log_table(sLog, tid);  // (a barrier follows)
 
   const int tbox = blockIdx.x;
   const int tb = p.target_boxes[tbox];
@@ -94,62 +199,92 @@ __global__ void __launch_bounds__(kSplitBlock) split_correction_kernel(const Spl
       double acc[RC], aci[RC];
 #pragma unroll
       for (int r = 0; r < RC; ++r) acc[r] = aci[r] = 0.0;
-      for (int li = l0; li < l1; ++li) {
-        const int sb = p.nbr_lists[li];
-        const int sbeg = p.src_starts[sb];
-        const int ns = p.src_counts[sb];
-        for (int c0 = 0; c0 < ns; c0 += chunk) {
-          const int nc = min(chunk, ns - c0);
-          __syncthreads();  // previous chunk done with LDS (and coefficients staged)
-          for (int i = tid; i < DIM * nc; i += kSplitBlock) {
-            const int a = i / nc, j = i % nc;
-            sX[a * chunk + j] = p.src_points[(int64_t)a * p.n_src + sbeg + c0 + j];
+      for (int lb = l0; lb < l1; lb += kSplitBoxes) {
+        const int nb = min(kSplitBoxes, l1 - lb);
+        __syncthreads();  // the previous boxes are done with
+        if (tid < kSplitBoxes) {  // one wave: the boxes' places in the run of sources
+          const int sb = tid < nb ? p.nbr_lists[lb + tid] : -1;
+          const int ns = sb < 0 ? 0 : p.src_counts[sb];
+          int sum = ns;
+          for (int o = 1; o < kSplitBoxes; o <<= 1) {
+            const int v = __shfl_up(sum, o);
+            if (tid >= o) sum += v;
           }
-          for (int i = tid; i < nc * RC * 2; i += kSplitBlock) {
-            const int c = i & 1, rj = i >> 1;
-            const int j = rj / RC, r = rj % RC;
-            sF[i] = r < rc ? p.strengths[(int64_t)(r0 + r) * p.lds + 2 * (int64_t)(sbeg + c0 + j) + c]
-                           : 0.0;
+          sOff[tid + 1] = sum;
+          if (tid == 0) sOff[0] = 0;
+          sBeg[tid] = (sb < 0 ? 0 : p.src_starts[sb]) - (sum - ns);
+        }
+        __syncthreads();
+        const int total = sOff[nb];
+        for (int c0 = 0; c0 < total; c0 += chunk) {
+          const int nc = min(chunk, total - c0);
+          if (c0 > 0) __syncthreads();  // previous chunk done with LDS
+          for (int j = tid; j < nc; j += kSplitBlock) {
+            int b = 0;  // the last box that begins at or before source c0 + j
+#pragma unroll
+            for (int o = kSplitBoxes / 2; o > 0; o >>= 1)
+              if (b + o < nb && sOff[b + o] <= c0 + j) b += o;
+            const int64_t src = (int64_t)sBeg[b] + c0 + j;
+#pragma unroll
+            for (int a = 0; a < DIM; ++a) sX[a * chunk + j] = p.src_points[(int64_t)a * p.n_src + src];
+#pragma unroll
+            for (int r = 0; r < RC; ++r) {
+              double fr = 0.0, fi = 0.0;
+              if (r < rc) {
+                const double* f = p.strengths + (int64_t)(r0 + r) * p.lds + 2 * src;
+                fr = f[0];
+                fi = f[1];
+              }
+              sF[((size_t)j * RC + r) * 2] = fr;
+              sF[((size_t)j * RC + r) * 2 + 1] = fi;
+            }
           }
           __syncthreads();
           if (tact && part < P) {  // threads past P * nt (nt not dividing 256) idle
-            for (int j = part; j < nc; j += P) {
-              double r2 = 0.0, da = 0.0;
+            for (int j0 = part; j0 < nc; j0 += U * P) {
+              double r2[U], da[U], vr[U], vi[U];
 #pragma unroll
-              for (int a = 0; a < DIM; ++a) {
-                const double d = xt[a] - sX[a * chunk + j];
-                r2 = fma(d, d, r2);
-                if (DERIV && a == p.deriv_axis) da = d;
-              }
-              double vr, vi;
-              if constexpr (DERIV) {
-                // +-(x_a - y_a) R'(r) / r; the self pair (r = 0) gives 0
-                vr = vi = 0.0;
-                if (r2 > 0.0) {
-                  if constexpr (MODE == kPairLegacyDeriv)
-                    legacy_radial_derivative<DIM>(r2, p.k_re, p.k_im, vr, vi);
-                  else
-                    remainder_radial_derivative<DIM>(r2, sC, N, vr, vi);
-                  const double f = p.deriv_sign * da;
-                  vr *= f;
-                  vi *= f;
+              for (int u = 0; u < U; ++u) {
+                const int j = min(j0 + u * P, nc - 1);  // past the chunk: not added below
+                r2[u] = da[u] = 0.0;
+#pragma unroll
+                for (int a = 0; a < DIM; ++a) {
+                  const double d = xt[a] - sX[a * chunk + j];
+                  r2[u] = fma(d, d, r2[u]);
+                  if (DERIV && a == p.deriv_axis) da[u] = d;
                 }
-              } else if constexpr (MODE == kPairLegacy) {
-                // closed forms off the diagonal; a self pair takes the
-                // series at r = 0, the limit the reference adds back
-                if (r2 > 0.0)
-                  legacy_difference<DIM>(r2, p.k_re, p.k_im, vr, vi);
-                else
-                  remainder_value<DIM>(r2, sC, N, vr, vi);
-              } else {
-                remainder_value<DIM>(r2, sC, N, vr, vi);
               }
-              const double* f = sF + (size_t)j * RC * 2;
+              if constexpr (LEGACY) {
+                // closed forms off the diagonal; a self pair takes the series at
+                // r = 0, the limit the reference adds back (0 under a derivative)
+                vr[0] = vi[0] = 0.0;
+                if constexpr (MODE == kPairLegacyDeriv) {
+                  if (r2[0] > 0.0) legacy_radial_derivative<DIM>(r2[0], p.k_re, p.k_im, vr[0], vi[0]);
+                } else if (r2[0] > 0.0) {
+                  legacy_difference<DIM>(r2[0], p.k_re, p.k_im, vr[0], vi[0]);
+                } else {
+                  split_series<DIM, false, false>(r2, cf, sLog, N, vr, vi);
+                }
+              } else {
+                split_series<DIM, DERIV, QUARTER>(r2, cf, sLog, N, vr, vi);
+              }
 #pragma unroll
-              for (int r = 0; r < RC; ++r) {
-                const double fr = f[2 * r], fi = f[2 * r + 1];
-                acc[r] = fma(vr, fr, fma(-vi, fi, acc[r]));
-                aci[r] = fma(vr, fi, fma(vi, fr, aci[r]));
+              for (int u = 0; u < U; ++u) {
+                const int j = j0 + u * P;
+                if (DERIV) {
+                  // +-(x_a - y_a) R'(r) / r; the self pair (r = 0) gives 0
+                  const double f = p.deriv_sign * da[u];
+                  vr[u] = r2[u] > 0.0 ? vr[u] * f : 0.0;
+                  vi[u] = r2[u] > 0.0 ? vi[u] * f : 0.0;
+                }
+                if (u > 0 && j >= nc) continue;
+                const double* f = sF + (size_t)j * RC * 2;
+#pragma unroll
+                for (int r = 0; r < RC; ++r) {
+                  const double fr = f[2 * r], fi = f[2 * r + 1];
+                  acc[r] = fma(vr[u], fr, fma(-vi[u], fi, acc[r]));
+                  aci[r] = fma(vr[u], fi, fma(vi[u], fr, aci[r]));
+                }
               }
             }
           }
@@ -181,13 +316,14 @@ __global__ void __launch_bounds__(kSplitBlock) split_correction_kernel(const Spl
   }
 }
 
-template <int DIM, int RC, int MODE>
-static hipError_t launch_split(const SplitParams& prm, int grid, size_t smem, hipStream_t s) {
-  auto fn = split_correction_kernel<DIM, RC, MODE>;
+template <int DIM, int RC, int MODE, bool QUARTER>
+static hipError_t launch_split(const SplitParams& prm, const SplitCoef& cf, int grid, size_t smem,
+                               hipStream_t s) {
+  auto fn = split_correction_kernel<DIM, RC, MODE, QUARTER>;
   hipError_t e = hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      (int)smem);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(fn, dim3(grid), dim3(kSplitBlock), smem, s, prm);
+  hipLaunchKernelGGL(fn, dim3(grid), dim3(kSplitBlock), smem, s, prm, cf);
   return hipGetLastError();
 }
 
@@ -245,21 +381,20 @@ extern "C" int vl1_split_correction(const vl1_split_args* a, void* stream) {
     coef = deriv ? split_derivative_coefficients(a->dim, k, a->series_nmax, a->split_order)
                  : split_coefficients(a->dim, k, a->series_nmax, a->split_order);
   }
-  if (coef.empty()) coef.assign(2, 0.0);  // 3D derivative with one term: R' = 0
-  DevBuf dcoef;
-  hipError_t e = upload(dcoef, coef.data(), coef.size() * sizeof(double), s);
-  if (e != hipSuccess) return fail(VL1_E_HIP, std::string("vl1_split_correction: ") + hipGetErrorString(e));
+  SplitCoef cf{};  // zeros past the coefficients (3D derivative with one term: R' = 0)
+  std::copy(coef.begin(), coef.end(), cf.v);
+  bool quarter = a->dim == 2;
+  for (size_t i = deriv ? 0 : 2; i + 3 < coef.size() && quarter; i += 4)
+    quarter = coef[i + 1] == 0.0 && coef[i + 3] == 0.25 * coef[i];
 
   SplitParams prm{};
   prm.dim = a->dim;
   prm.n_rhs = a->n_rhs;
   prm.n_terms = a->series_nmax;
-  prm.ncoef = (int)coef.size();
   prm.k_re = a->k_re;
   prm.k_im = a->k_im;
   prm.deriv_axis = deriv ? a->deriv_axis : -1;
   prm.deriv_sign = a->deriv_kind == VL1_SPLIT_DERIV_SOURCE ? -1.0 : 1.0;
-  prm.coef = dcoef.as<double>();
   prm.target_boxes = a->target_boxes;
   prm.nbr_starts = a->nbr_starts;
   prm.nbr_lists = a->nbr_lists;
@@ -283,22 +418,26 @@ extern "C" int vl1_split_correction(const vl1_split_args* a, void* stream) {
   // the remainder is evaluated once per (target, source) pair and RC-chunk;
   // RC <= 8 keeps the LDS small enough for several workgroups per CU
   const int RC = a->n_rhs == 1 ? 1 : (a->n_rhs <= 4 ? 4 : 8);
-  // source points staged per pass: the source box size, rounded up to the parts
-  const int msrc = sep ? a->max_src_box_points : a->max_box_points;
-  const int chunk = std::min(nt * P, (msrc + P - 1) / P * P);
+  // source points staged per pass
+  const int chunk = RC == 1 ? 512 : 256;
   prm.chunk = chunk;
   const size_t stage = (size_t)a->dim * chunk + (size_t)chunk * RC * 2;
   const size_t reduce = P > 1 ? (size_t)kSplitBlock * RC * 2 : 0;  // aliases the staging
-  const size_t smem = sizeof(double) * ((size_t)coef.size() + std::max(stage, reduce));
-  if (smem > 160 * 1024) return fail(VL1_E_UNSUPPORTED, "vl1_split_correction: LDS budget exceeded");
+  const size_t smem = sizeof(double) * std::max(stage, reduce);
   const int grid = a->n_tgt_boxes;
   const int mode = deriv ? (legacy ? kPairLegacyDeriv : kPairDeriv)
                          : (legacy ? kPairLegacy : kPairSeries);
   auto pick = [&](auto dimc, auto modec) {
     constexpr int D = decltype(dimc)::value, M = decltype(modec)::value;
-    return RC == 1   ? launch_split<D, 1, M>(prm, grid, smem, s)
-           : RC == 4 ? launch_split<D, 4, M>(prm, grid, smem, s)
-                     : launch_split<D, 8, M>(prm, grid, smem, s);
+    if constexpr (D == 2 && (M == kPairSeries || M == kPairDeriv)) {
+      if (quarter)
+        return RC == 1   ? launch_split<D, 1, M, true>(prm, cf, grid, smem, s)
+               : RC == 4 ? launch_split<D, 4, M, true>(prm, cf, grid, smem, s)
+                         : launch_split<D, 8, M, true>(prm, cf, grid, smem, s);
+    }
+    return RC == 1   ? launch_split<D, 1, M, false>(prm, cf, grid, smem, s)
+           : RC == 4 ? launch_split<D, 4, M, false>(prm, cf, grid, smem, s)
+                     : launch_split<D, 8, M, false>(prm, cf, grid, smem, s);
   };
   using D2 = std::integral_constant<int, 2>;
   using D3 = std::integral_constant<int, 3>;
@@ -314,8 +453,8 @@ extern "C" int vl1_split_correction(const vl1_split_args* a, void* stream) {
       default: return pick(dimc, MS{});
     }
   };
-  e = a->dim == 2 ? by_mode(D2{}) : by_mode(D3{});
-  // the coefficient buffer is freed when dcoef leaves scope: wait for the launch
+  hipError_t e = a->dim == 2 ? by_mode(D2{}) : by_mode(D3{});
+  // as documented: the result is there on return
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) return fail(VL1_E_HIP, std::string("vl1_split_correction: ") + hipGetErrorString(e));
   return VL1_OK;

@@ -58,14 +58,19 @@ struct FoldDims {
   uint64_t kgs[2] = {0, 0};        // byte r: first K group of round r
 };
 
+// A tile's place in the lists, and its first chunk words (one scalar load).
+struct FoldTileInfo {
+  int32_t step, n_steps, chunk, n_chunks;
+  uint32_t words[4];
+};
+
 struct FoldParams {
   FoldDims d;
   int B, Rc, R;            // boxes per tile, densities per tile, densities in all
   int nb;                  // boxes; index nb of X holds zeros
   int n_box_tiles;
   int nm, cplx, rows;      // modes per box; rows per box (2 nm if complex)
-  const int32_t* tile_step_start;   // [n_box_tiles + 1]
-  const int32_t* tile_chunk_start;  // [n_box_tiles + 1]
+  const FoldTileInfo* tiles;        // [n_box_tiles]
   const int32_t* tile_boxes;        // [n_box_tiles][B] target box or -1
   const uint32_t* chunks;           // chunk words, kFoldPad more at the end
   const int32_t* step_src;          // [n_steps + kFoldPad][B][np] source boxes (nb: none)

@@ -21,6 +21,17 @@ __device__ __forceinline__ void fold_for(F&& f) {
   }
 }
 
+// 4-row groups of all parities, by the counts of a parity with 0..3 odd axes.
+constexpr int fold_rows4(int np, int g0, int g1, int g2, int g3) {
+  return 4 * (np == 8 ? g0 + 3 * g1 + 3 * g2 + g3 : (np == 4 ? g0 + 2 * g1 + g2 : (np == 2 ? g0 + g1 : g0)));
+}
+// Whether all columns' outputs go through LDS at once: in a slot of at most the
+// 8 units' and 4.5 KB more (two workgroups of 3D q = 6 still share a CU).
+constexpr bool fold_whole(int np, int nct, int g0, int g1, int g2, int g3) {
+  return nct == 1 ||
+         fold_rows4(np, g0, g1, g2, g3) * (16 * nct + 1) <= kFoldUnits * np * nct * 64 + 576;
+}
+
 // A workgroup of NP waves computes 16 NCT columns (B target boxes x Rc
 // densities) of all rows; wave w owns the rows of one output parity, G groups
 // of 4, in the accumulators of v_mfma_f64_16x16x4f64 (G / 4 full 16-row
@@ -56,7 +67,7 @@ __device__ __forceinline__ void fold_for(F&& f) {
 // CU with two slots, 1060 us for two of 32 columns (general form: 7816 us).
 // The FP64 pipe is then busy about 55% of the time; the load path (fragments
 // and values) about 60%.
-template <int NP, int NCT, int G>
+template <int NP, int NCT, int G, bool WHOLE>
 __device__ __forceinline__ void fold_run(const FoldParams& p, double* smem, int bt, int rcx,
                                          int pout, int grow) {
   constexpr int T = 64 * NP, COLS = 16 * NCT, UW = kFoldUnits;
@@ -87,8 +98,11 @@ __device__ __forceinline__ void fold_run(const FoldParams& p, double* smem, int 
   // one per thread and step
   uint32_t* ring = reinterpret_cast<uint32_t*>(smem + p.slot_doubles);
   double* sPart = smem + p.slot_doubles + 32 * NP * 2;  // [T / COLS][COLS] log-term sums
+  double* sD = sPart + T;
+  int64_t* sBox = reinterpret_cast<int64_t*>(sD + COLS);  // column -> its box's modes, y row offset
   const int n_src = p.B * NP;  // <= T
-  const int32_t* srow = p.step_src + (int64_t)p.tile_step_start[bt] * n_src + (tid < n_src ? tid : 0);
+  const FoldTileInfo ti = p.tiles[bt];
+  const int32_t* srow = p.step_src + (int64_t)ti.step * n_src + (tid < n_src ? tid : 0);
   int step = 0, carry = 0;      // the step last entered; the list on its way to the ring
   bool pending = false;
   // the list fetched when this step was entered (step + 3) into the slot of the
@@ -205,9 +219,9 @@ __device__ __forceinline__ void fold_run(const FoldParams& p, double* smem, int 
 
   // ---- pipeline.  Words past the tile's last chunk belong to the next tile
   // (or the lists' padding): what they prefetch is valid and not used.
-  const int c0 = p.tile_chunk_start[bt], nch = p.tile_chunk_start[bt + 1] - c0;
-  const uint32_t* words = p.chunks + c0;
-  uint32_t w0 = words[0], w1 = words[1], w2 = words[2];
+  const int nch = ti.n_chunks;
+  const uint32_t* words = p.chunks + ti.chunk;
+  uint32_t w0 = ti.words[0], w1 = ti.words[1], w2 = ti.words[2];
   Units uC = units_of(w0), uN = units_of(w1);
   {
     int s4[4];
@@ -218,15 +232,21 @@ __device__ __forceinline__ void fold_run(const FoldParams& p, double* smem, int 
       load_a(w0, uC.a.y, std::integral_constant<int, 1>{});
       load_a(w0, uC.a.z, std::integral_constant<int, 2>{});
     }
+    if (tid < COLS) {  // for the outputs
+      const int b = tid / p.Rc, r = tid % p.Rc;
+      const int tb = b < p.B && r0 + r < p.R ? p.tile_boxes[bt * p.B + b] : -1;
+      sBox[2 * tid] = tb < 0 ? -1 : (int64_t)tb * p.nm;
+      sBox[2 * tid + 1] = (int64_t)(r0 + r) * p.ldy;
+    }
     if (tid < n_src)
 #pragma unroll
       for (int k = 0; k < 4; ++k) ring[k * 32 * NP + tid] = (uint32_t)s4[k] * box_bytes;
     srow += (int64_t)4 * n_src;
     if (p.dl) {  // 2D log term: this thread's part of its column's sources
-      const int n = (p.tile_step_start[bt + 1] - p.tile_step_start[bt]) * NP;
+      const int n = ti.n_steps * NP;
       const int b = (tid % COLS) / p.Rc, r = (tid % COLS) % p.Rc;
       const bool in = b < p.B && r0 + r < p.R;
-      const int32_t* q = p.step_src + (int64_t)p.tile_step_start[bt] * n_src + (in ? b : 0) * NP;
+      const int32_t* q = p.step_src + (int64_t)ti.step * n_src + (in ? b : 0) * NP;
       const double* dlc = p.dl + (int64_t)rcx * (p.nb + 1) * p.Rc + (in ? r : 0);
       double a = 0.0;
       for (int e = tid / COLS; e < n; e += T / COLS)
@@ -291,63 +311,66 @@ __device__ __forceinline__ void fold_run(const FoldParams& p, double* smem, int 
     w2 = w3;
   }
 
-  // ---- output: back to box nodes, 16 columns at a time through LDS; a thread
-  // keeps one row (rows <= T) and takes every cpt-th column
-  constexpr int PITCH = 17;
-  double* sD = sPart + T;
-  int64_t* sBox = reinterpret_cast<int64_t*>(sD + COLS);  // column -> y row offset, its box's modes
-  if (tid < COLS) {
-    if (p.dl) {
-      double a = 0.0;
-      for (int k = 0; k < T / COLS; ++k) a += sPart[k * COLS + tid];
-      sD[tid] = a;
-    }
-    const int b = tid / p.Rc, r = tid % p.Rc;
-    const int tb = b < p.B && r0 + r < p.R ? p.tile_boxes[bt * p.B + b] : -1;
-    sBox[2 * tid] = tb < 0 ? -1 : (int64_t)tb * p.nm;
-    sBox[2 * tid + 1] = (int64_t)(r0 + r) * p.ldy;
-  }
+  // ---- output: back to box nodes through LDS, all columns at once (WHOLE; 16
+  // where the rows are too many); a thread keeps one row (rows <= T) and takes
+  // every cpt-th column, KB at a time, with their points loaded a batch ahead
+  constexpr int OC = WHOLE ? COLS : 16, PITCH = OC + 1, KB = 4;
   const int cpt = T / p.rows, t = tid % p.rows, cc = tid / p.rows;
   const FoldOut o = p.out[t];
   const int tm = t % p.nm, part = t / p.nm;
+  int mp[KB];
+  auto points = [&](int c0) {  // of columns c0 + k cpt
+#pragma unroll
+    for (int k = 0; k < KB; ++k) {
+      const int c = c0 + k * cpt;
+      const int64_t bm = cc < cpt && c < COLS ? sBox[2 * c] : -1;
+      mp[k] = p.mode_point[bm < 0 ? 0 : bm + tm];
+      if (bm < 0) mp[k] = -1;
+    }
+  };
+  points(cc);
+  if (p.dl && tid < COLS) {
+    double a = 0.0;
+    for (int k = 0; k < T / COLS; ++k) a += sPart[k * COLS + tid];
+    sD[tid] = a;
+  }
   const double scale = 1.0 / (double)(1 << o.shift);
-  fold_for<0, NCT>([&](auto ctc) {
-    constexpr int ct = decltype(ctc)::value;
+  fold_for<0, COLS / OC>([&](auto occ) {
+    constexpr int oc = decltype(occ)::value;
     __syncthreads();
     double* yh = smem + (4 * grow + lane / 16) * PITCH + lane % 16;
 #pragma unroll
-    for (int k = 0; k < NT; ++k)
+    for (int ct = oc * (OC / 16); ct < (oc + 1) * (OC / 16); ++ct) {
+      double* yc = yh + 16 * ct - OC * oc;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) yh[(16 * k + 4 * e) * PITCH] = accF[k][ct][e];
+      for (int k = 0; k < NT; ++k)
 #pragma unroll
-    for (int g = 0; g < GC; ++g) yh[(16 * NT + 4 * g) * PITCH] = accC[g][ct];
+        for (int e = 0; e < 4; ++e) yc[(16 * k + 4 * e) * PITCH] = accF[k][ct][e];
+#pragma unroll
+      for (int g = 0; g < GC; ++g) yc[(16 * NT + 4 * g) * PITCH] = accC[g][ct];
+    }
     __syncthreads();
     if (cc < cpt) {
-      constexpr int KB = 4;  // columns in flight
-      for (int c0 = cc; c0 < 16; c0 += KB * cpt) {
-        int mp[KB];
-        int64_t row[KB];
+      for (int c0 = OC * oc + cc; c0 < OC * (oc + 1); c0 += KB * cpt) {
+        int mc[KB];
+#pragma unroll
+        for (int k = 0; k < KB; ++k) mc[k] = mp[k];
+        const int cn = c0 + KB * cpt;
+        points(cn < OC * (oc + 1) ? cn : OC * (oc + 1) + cc);
 #pragma unroll
         for (int k = 0; k < KB; ++k) {
           const int c = c0 + k * cpt;
-          const int64_t bm = c < 16 ? sBox[2 * (16 * ct + c)] : -1;
-          row[k] = bm < 0 ? -1 : sBox[2 * (16 * ct + c) + 1];
-          mp[k] = p.mode_point[bm < 0 ? 0 : bm + tm];
-        }
-#pragma unroll
-        for (int k = 0; k < KB; ++k) {
-          if (row[k] < 0) continue;
-          const int c = c0 + k * cpt;
+          if (mc[k] < 0 || c >= OC * (oc + 1)) continue;
           double v = 0.0;
 #pragma unroll
           for (int q = 0; q < NP; ++q)
             if (o.row[q] >= 0) {
-              const double h = smem[o.row[q] * PITCH + c];
+              const double h = smem[o.row[q] * PITCH + c - OC * oc];
               v += (__popc(q & o.flips) & 1) ? -h : h;
             }
           v *= scale;
-          if (p.dl) v += sD[16 * ct + c];
-          p.y[row[k] + (p.cplx ? 2 * (int64_t)mp[k] + part : (int64_t)mp[k])] = v;
+          if (p.dl) v += sD[c];
+          p.y[sBox[2 * c + 1] + (p.cplx ? 2 * (int64_t)mc[k] + part : (int64_t)mc[k])] = v;
         }
       }
     }
@@ -368,15 +391,16 @@ __global__ void __launch_bounds__(64 * NP, G0 <= 8 ? 4 : 2) fold_f64_kernel(cons
   int grow = 0;  // groups before this parity
   for (int k = 0; k < NP; ++k)
     if (k < pout) grow += (int)((p.d.groups_lo >> (8 * k)) & 255);
+  constexpr bool WHOLE = fold_whole(NP, NCT, G0, G1, G2, G3);
   if constexpr (G0 == G1 && G1 == G2 && G2 == G3) {
-    fold_run<NP, NCT, G0>(p, fold_smem, bt, rcx, pout, grow);
+    fold_run<NP, NCT, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
   } else {
     // the loops hold the same barriers, so waves may run different ones
     const int odd = __popc(pout);
-    if (odd == 0) fold_run<NP, NCT, G0>(p, fold_smem, bt, rcx, pout, grow);
-    else if (odd == 1) fold_run<NP, NCT, G1>(p, fold_smem, bt, rcx, pout, grow);
-    else if (odd == 2) fold_run<NP, NCT, G2>(p, fold_smem, bt, rcx, pout, grow);
-    else if constexpr (NP == 8) fold_run<NP, NCT, G3>(p, fold_smem, bt, rcx, pout, grow);
+    if (odd == 0) fold_run<NP, NCT, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
+    else if (odd == 1) fold_run<NP, NCT, G1, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
+    else if (odd == 2) fold_run<NP, NCT, G2, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
+    else if constexpr (NP == 8) fold_run<NP, NCT, G3, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
   }
 }
 
@@ -394,7 +418,8 @@ hipError_t launch_fold(const FoldParams& p, hipStream_t s) {
     done.fetch_or(bit, std::memory_order_acq_rel);
   }
   FoldParams q = p;
-  q.slot_doubles = std::max(kFoldUnits * NP * NCT * 64, p.d.rows4 * 17);
+  const int out_cols = fold_whole(NP, NCT, G0, G1, G2, G3) ? 16 * NCT : 16;
+  q.slot_doubles = std::max(kFoldUnits * NP * NCT * 64, p.d.rows4 * (out_cols + 1));
   const size_t doubles = (size_t)q.slot_doubles + 32 * NP * 2 + 64 * NP + 3 * 16 * NCT;
   const int grid = (p.n_box_tiles + 7) / 8 * 8 * ((p.R + p.Rc - 1) / p.Rc);
   hipLaunchKernelGGL(fn, dim3(grid), dim3(64 * NP), doubles * sizeof(double), s, q);

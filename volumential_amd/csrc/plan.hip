@@ -1163,7 +1163,7 @@ struct TileSchedule {
 struct FoldSchedule {
   int B = 0, n_tiles = 0;
   int64_t n_steps = 0;
-  DevBuf tile_step_start, tile_chunk_start, tile_boxes, chunks, step_src;
+  DevBuf tiles, tile_boxes, chunks, step_src;
 };
 
 // The dynamic-LDS limit of a tile kernel is raised to the full 160 KiB (less
@@ -1531,7 +1531,7 @@ static int build_fold_schedule(vl1_plan* pl, int B, bool morton_only, FoldSchedu
       for (int at = i + (x - i % 8 + 8) % 8; at < j; at += 8) place[at] = by_len[k++];
     i = j;
   }
-  std::vector<int32_t> tss(sch->n_tiles + 1, 0), tcs(sch->n_tiles + 1, 0);
+  std::vector<FoldTileInfo> tiles(sch->n_tiles);
   std::vector<int32_t> tboxes((size_t)sch->n_tiles * B, -1), src;
   std::vector<uint32_t> words;
   src.reserve(classes.size() * B * np + (size_t)kFoldPad * B * np);
@@ -1540,6 +1540,7 @@ static int build_fold_schedule(vl1_plan* pl, int B, bool morton_only, FoldSchedu
     const int32_t* cl = classes.data() + cls_at[place[t]];
     const size_t n_cl = cls_at[place[t] + 1] - cls_at[place[t]];
     const size_t base = src.size();
+    tiles[t].chunk = (int32_t)words.size();
     src.resize(base + n_cl * B * np, pl->nboxes);  // nboxes: the zero box
     for (int b = 0; b < n; ++b) {
       const int tg = order[first + b];
@@ -1557,16 +1558,18 @@ static int build_fold_schedule(vl1_plan* pl, int B, bool morton_only, FoldSchedu
       for (int k = 0; k < fold_chunks(fp.d, m); ++k)
         words.push_back(fold_chunk_word(cl[i], z, m, k, k == 0));
     }
-    tss[t + 1] = tss[t] + (int32_t)n_cl;
-    tcs[t + 1] = (int32_t)words.size();
+    tiles[t].step = (int32_t)sch->n_steps;
+    tiles[t].n_steps = (int32_t)n_cl;
+    tiles[t].n_chunks = (int32_t)words.size() - tiles[t].chunk;
+    sch->n_steps += (int64_t)n_cl;
   }
-  sch->n_steps = tss.back();
   // the kernel prefetches past a tile's end
   words.resize(words.size() + kFoldPad, fold_chunk_word(0, 0, 0, 0, true));
   src.resize(src.size() + (size_t)kFoldPad * B * np, pl->nboxes);
-  hipError_t e = upload(sch->tile_step_start, tss.data(), tss.size() * 4, s);
+  for (FoldTileInfo& t : tiles)
+    for (int k = 0; k < 4; ++k) t.words[k] = words[t.chunk + k];
+  hipError_t e = upload(sch->tiles, tiles.data(), tiles.size() * sizeof(FoldTileInfo), s);
   if (e == hipSuccess) e = upload(sch->tile_boxes, tboxes.data(), tboxes.size() * 4, s);
-  if (e == hipSuccess) e = upload(sch->tile_chunk_start, tcs.data(), tcs.size() * 4, s);
   if (e == hipSuccess) e = upload(sch->chunks, words.data(), words.size() * 4, s);
   if (e == hipSuccess) e = upload(sch->step_src, src.data(), src.size() * 4, s);
   if (e != hipSuccess) {
@@ -2451,9 +2454,8 @@ static int fold_contract(vl1_plan* pl, const Prepared& pr, int R, double* y, int
   p.nm = f.nm;
   p.cplx = f.cplx;
   p.rows = f.rows;
-  p.tile_step_start = pr.fold->tile_step_start.as<int32_t>();
+  p.tiles = pr.fold->tiles.as<FoldTileInfo>();
   p.tile_boxes = pr.fold->tile_boxes.as<int32_t>();
-  p.tile_chunk_start = pr.fold->tile_chunk_start.as<int32_t>();
   p.chunks = pr.fold->chunks.as<uint32_t>();
   p.lut_u = f.u_lut;
   p.lut_l = f.l_lut;

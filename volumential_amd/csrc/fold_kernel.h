@@ -76,6 +76,8 @@ __device__ __forceinline__ void fold_run(const FoldParams& p, double* smem, int 
   constexpr int SLOT = UW * NP * NCT * 64;  // doubles of the LDS slot
   constexpr int NT = G / 4, GC = G % 4, NF = NT > 0 ? NT : 1, NG = GC > 0 ? GC : 1;
   constexpr int CV = NCT - 1;  // load table of this width
+  constexpr bool AHEAD = NP < 8 || G <= 4;  // columns read a unit ahead
+  constexpr int NB = AHEAD ? 2 : 1;
   const int tid = threadIdx.x, lane = tid % 64;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int r0 = rcx * p.Rc;
@@ -275,6 +277,9 @@ __device__ __forceinline__ void fold_run(const FoldParams& p, double* smem, int 
     load_x(w1, kg1);
     kg1 = kgs_of(w2);
     __syncthreads();
+    // matrix work first: the other workgroup's sums and loads fill its gaps
+    __builtin_amdgcn_s_setprio(1);
+    double bx[NB][NCT];
     fold_for<0, UW>([&](auto uc) {
       constexpr int u = decltype(uc)::value;
       auto word = [](const Units& x, int k) {
@@ -285,25 +290,30 @@ __device__ __forceinline__ void fold_run(const FoldParams& p, double* smem, int 
       constexpr int un = u + NS - 1;
       load_a(un < UW ? w0 : w1, un < UW ? word(uC, un % UW) : word(uN, un % UW),
              std::integral_constant<int, un % NS>{});
-      const double* b = smem + (unit & 255) * (NCT * 64) + lane;
-      double bx[NCT];
+      // the unit's columns; a unit ahead where the registers allow
+      auto columns = [&](uint32_t w, int k) {
+        const double* b = smem + (w & 255) * (NCT * 64) + lane;
 #pragma unroll
-      for (int ct = 0; ct < NCT; ++ct) bx[ct] = b[64 * ct];
+        for (int ct = 0; ct < NCT; ++ct) bx[k][ct] = b[64 * ct];
+      };
+      if (u == 0 || !AHEAD) columns(unit, u % NB);
+      if (AHEAD && u + 1 < UW) columns(word(uC, (u + 1) % UW), (u + 1) % NB);
       if (unit >> 16) {  // uniform; no load inside
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
           for (int ct = 0; ct < NCT; ++ct)
             accF[t][ct] =
-                __builtin_amdgcn_mfma_f64_16x16x4f64(aF[u % NS][t], bx[ct], accF[t][ct], 0, 0, 0);
+                __builtin_amdgcn_mfma_f64_16x16x4f64(aF[u % NS][t], bx[u % NB][ct], accF[t][ct], 0, 0, 0);
 #pragma unroll
         for (int g = 0; g < GC; ++g)
 #pragma unroll
           for (int ct = 0; ct < NCT; ++ct)
             accC[g][ct] =
-                __builtin_amdgcn_mfma_f64_4x4x4f64(aC[u % NS][g], bx[ct], accC[g][ct], 0, 0, 0);
+                __builtin_amdgcn_mfma_f64_4x4x4f64(aC[u % NS][g], bx[u % NB][ct], accC[g][ct], 0, 0, 0);
       }
     });
+    __builtin_amdgcn_s_setprio(0);
     uC = uN;
     uN = uF;
     w0 = w1;

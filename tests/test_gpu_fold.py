@@ -93,7 +93,7 @@ def test_fold_graded(cuda, dim, q, n_rhs):
 @pytest.mark.parametrize("cplx", [False, True])
 @pytest.mark.parametrize("dim,q", [(2, 2), (2, 5), (2, 8), (3, 2), (3, 3), (3, 5), (3, 6)])
 def test_fold_many_densities(cuda, dim, q, cplx):
-    """Enough tiles for the wide ones; 192 densities are three passes of 64."""
+    """Enough tiles for the wide ones (24 groups of 8 densities)."""
     print(f"case: fold {dim}D q={q} R=192 {'complex' if cplx else 'real'}", flush=True)
     tr, table, f = _case(dim, q, cplx, 4 if dim == 2 else 2, 192, q)
     _check(tr, table, f, cplx, [0, 63, 64, 191])

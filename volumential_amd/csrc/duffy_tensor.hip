@@ -73,7 +73,7 @@ __global__ void __launch_bounds__(kDtThreads) duffy_tensor_kernel(const DuffyTen
   const int b = blockIdx.y;
   const int64_t e0 = p.start[tgt] + (int64_t)blockIdx.z * kDtThreads * kDtAcc;
   const int ne = (int)min<int64_t>(p.start[tgt + 1] - e0, kDtThreads * kDtAcc);
-  if (ne <= 0) return;  // uniform
+  if (ne <= 0 || e0 < 0 || e0 + ne > p.n_entries) return;  // uniform
   double* out = p.part + ((int64_t)b * p.n_entries + e0) * VW;
 
   double x[3], v[3], sl[3], lenprod = 1.0;
@@ -126,7 +126,8 @@ __global__ void __launch_bounds__(kDtThreads) duffy_tensor_kernel(const DuffyTen
 #pragma unroll
   for (int c = 0; c < kDtAcc; ++c) {
     const int i = tid + c * kDtThreads;
-    const int m = i < ne ? p.mode[e0 + i] : 0;
+    int m = i < ne ? p.mode[e0 + i] : 0;
+    if ((unsigned)m >= (unsigned)(q * q * q)) m = 0;  // outside the contract: some entry's value
     m2[c] = m % q;
     m1[c] = m / q % q;
     m0[c] = m / (q * q);

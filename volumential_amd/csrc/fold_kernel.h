@@ -1,5 +1,5 @@
-// Tile kernel of the folded FP64 form (see fold.h); instantiated in
-// fold_2d.hip and fold_3d.hip.
+// Tile kernel of the folded FP64 form (see fold.h); instantiated in fold_2d.hip,
+// fold_2dc.hip, fold_3d.hip and fold_3dodd.hip.
 #pragma once
 
 #include <algorithm>
@@ -64,7 +64,8 @@ constexpr bool fold_whole(int np, int nct, int g0, int g1, int g2, int g3) {
 // registers (at most 128 for G <= 8) and the one LDS slot are sized for two
 // workgroups per CU, each running its MFMAs while the other loads and sums: 3D
 // q = 6, 24 densities, 4096 boxes: 1146 us for one workgroup of 64 columns per
-// CU with two slots, 1060 us for two of 32 columns (general form: 7816 us).
+// CU with two slots, 1060 us for two of 32 columns (general form: 7816 us; 1015
+// us with the products at raised priority and the tile's entry and exit as below).
 // The FP64 pipe is then busy about 55% of the time; the load path (fragments
 // and values) about 60%.
 template <int NP, int NCT, int G, bool WHOLE>

@@ -258,8 +258,7 @@ __global__ void __launch_bounds__(kNFBlock) near_field_f64_kernel(const NFParams
 // semantics of the scalar kernel above: an invalid id (or a missing entry,
 // NaN in the expanded blocks) gives A = 0.  v_mfma_f64_16x16x4f64 tiles:
 // wave w owns row tiles w, w + 8 (16 rows each) and all NC 16-column tiles
-// (the fewest of 1, 2, 4 for the densities: fewer columns are computed than
-// asked for only past the last density).  K advances in chunks of KC source
+// (1, 2 or 4, by the densities: see launch_nf_mfma).  K advances in chunks of KC source
 // particles; a chunk's densities go through a two-slot LDS ring and its table
 // fragments through registers, both loaded one chunk ahead, and a pair's source
 // modes two pairs ahead.  Pair descriptors (a chain of four dependent loads

@@ -2315,9 +2315,9 @@ struct Prepared {
 // counts that aim at the 1e-10 bar: a folded block costs 1/8 (3D) or 1/4 (2D)
 // of the products, a split one S (S + 1) / 2 times them on faster units.
 // Measured at S = 5, split against folded, us per call: int8 3D q = 6, 32768
-// boxes, 64 densities 29651 / 22939; int8 2D q = 6 complex per-level, 12919
-// boxes, 16 densities 1323 / 468; int8 fused Helmholtz split, 16384 boxes, 16
-// densities 647 / 513; BF16 3D q = 4, 4096 boxes, 20 densities 1023 / 244.
+// boxes, 64 densities 31225 / 22010; int8 2D q = 6 complex per-level, 12919
+// boxes, 16 densities 1313 / 441; int8 fused Helmholtz split, 16384 boxes, 16
+// densities 604 / 491; BF16 3D q = 4, 4096 boxes, 20 densities 1157 / 217.
 // Below 5 slices a caller asks for the split itself, its error included.
 // Calls whose int8 sums might leave int32 stay with the int8 form, which
 // refuses them by its own schedule (i8_check_range).

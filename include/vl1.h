@@ -363,6 +363,11 @@ int vl1_plan_tune(vl1_plan* plan, int form, const double* f, int64_t ldf, int n_
  * VL1_E_UNSUPPORTED for one row tile per wave on blocks of more than 128
  * rows.  n_slices is ignored for VL1_FORM_F64. */
 int vl1_plan_set_variant(vl1_plan* plan, int form, int n_slices, int n_rhs, int variant);
+/* The tile a folded plan of these sizes takes (host only): {1 if the folded
+ * kernel takes such boxes, columns, densities per tile, boxes per tile, bytes
+ * of a box's staged densities in a tile}, zeros if it does not. */
+int vl1_plan_fold_tile_host(int dim, int q, int is_complex, int64_t n_boxes, int64_t n_tgt_boxes,
+                            int n_rhs, int64_t* out5);
 /* Plan statistics: [0] list-1 pairs, [1] tiles, [2] (tile, case) steps,
  * [3] distinct (case, level) blocks, [4] device bytes. */
 int vl1_plan_stats(const vl1_plan* plan, int64_t* out5);

@@ -67,6 +67,7 @@ EXPORTED_SYMBOLS = (
     "vl1_plan_eval",
     "vl1_plan_stage",
     "vl1_plan_contract",
+    "vl1_plan_fold_tile_host",
     "vl1_plan_stats",
     "vl1_plan_eval_noalloc",
     "vl1_plan_tune",
@@ -341,6 +342,7 @@ def lib():
     L.vl1_plan_tune.argtypes = [vp, C.c_int, vp, i64, C.c_int, vp, i64, C.POINTER(SplitOpts),
                                 C.c_int, C.POINTER(i32), C.POINTER(f64), vp]
     L.vl1_plan_set_variant.argtypes = [vp, C.c_int, C.c_int, C.c_int, C.c_int]
+    L.vl1_plan_fold_tile_host.argtypes = [C.c_int, C.c_int, C.c_int, i64, i64, C.c_int, vp]
     L.vl1_duffy_build.argtypes = [C.POINTER(DuffyArgs), vp]
     L.vl1_duffy_build_tensor.argtypes = [C.POINTER(DuffyTensorArgs), vp]
     L.vl1_split_correction.argtypes = [C.POINTER(SplitArgs), vp]

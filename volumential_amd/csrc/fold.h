@@ -136,8 +136,15 @@ struct FoldPlan {
 // Folded basis of q^dim nodes (2 values per node if complex); false: sizes
 // the kernel does not take.
 bool fold_layout(FoldPlan& f, int dim, int q, int cplx, uint32_t sign_mask);
-// Tile shape for R densities over n_tgt boxes (16 nct columns; 0: choose).
-FoldTile fold_tile(int n_tgt, int R, int nct = 0);
+// Whether the tile kernel's 32-bit byte offsets reach all nb boxes and the zero
+// box at Rc densities per tile (a box holds kg K groups of 32 Rc bytes; a lane
+// reads up to one box past its own offset).
+inline bool fold_fits(const FoldDims& d, int nb, int Rc) {
+  return ((uint64_t)nb + 2) * (uint64_t)d.kg * (uint64_t)Rc * 32 <= (uint64_t)1 << 32;
+}
+// Tile shape for R densities over n_tgt of nb boxes (16 nct columns; 0:
+// choose); nb boxes must fit at one density per tile.
+FoldTile fold_tile(const FoldDims& d, int nb, int n_tgt, int R, int nct = 0);
 // X and dl sizes in doubles for one evaluation.
 size_t fold_x_size(const FoldDims& d, const FoldTile& t, int nb, int R);
 size_t fold_dl_size(const FoldTile& t, int nb, int R);

@@ -174,15 +174,19 @@ bool fold_layout(FoldPlan& f, int dim, int q, int cplx, uint32_t sign_mask) {
 // Densities per tile: the split of R over tiles of `cols` columns that fills
 // them best (R = 24 over 64 columns: 3 x 8 densities of 8 boxes, all columns
 // in use; 59: 15 x 4), the largest up to 8 among equals -- neighbouring boxes
-// in a tile share their sources' cache lines.
-FoldTile fold_tile(int n_tgt, int R, int nct) {
+// in a tile share their sources' cache lines.  Large trees take as many as the
+// kernel's 32-bit offsets reach (3D q = 6: 8 densities up to 299,591 boxes, 4 up
+// to 599,184).
+FoldTile fold_tile(const FoldDims& d, int nb, int n_tgt, int R, int nct) {
   const int Rq = std::min(R, 64);  // larger counts are whole multiples of 64
+  int rc_max = Rq;
+  while (rc_max > 1 && !fold_fits(d, nb, rc_max)) --rc_max;
   auto pick = [&](int nct) {
     const int cols = 16 * nct;
     FoldTile t;
     t.nct = nct;
     double best = -1.0;
-    for (int rc = std::min(Rq, cols); rc >= 1; --rc) {
+    for (int rc = std::min(rc_max, cols); rc >= 1; --rc) {
       const int nrc = (Rq + rc - 1) / rc, B = cols / rc;
       double u = (double)Rq / (nrc * rc) * (B * rc) / cols;
       if (rc > 8) u -= 1e-3;
@@ -522,6 +526,7 @@ bool fold_has_kernel(const FoldDims& d) {
 }
 
 hipError_t fold_contract_launch(const FoldParams& p, const FoldTile& t, hipStream_t s) {
+  if (!fold_fits(p.d, p.nb, p.Rc)) return hipErrorInvalidValue;
   int g[4];
   odd_groups(p.d, g);
   return p.d.np == 8 ? fold_launch_3d(p, t.nct, g, s) : fold_launch_2d(p, t.nct, g, s);

@@ -1766,13 +1766,13 @@ static hipError_t expand_plan_blocks(const vl1_payload* pay, const vl1_plan* pl,
 // the classes of the plan's keys under reflections of the folded axes.  A class
 // representative (all folded components positive) that is no key itself is
 // appended to `keys`.  Null for boxes the tile kernel does not take and trees
-// beyond its 32-bit byte offsets: the dense form runs.
+// beyond its 32-bit byte offsets at one density per tile: the dense form runs.
 static std::unique_ptr<FoldPlan> fold_classes(const vl1_plan* pl, const vl1_payload* pay, bool split,
                                               const std::vector<int64_t>& key_vid, BlockList& keys) {
   const int dim = pl->dim;
   auto f = std::unique_ptr<FoldPlan>(new FoldPlan());
   if (!fold_layout(*f, dim, pay->q, pl->cplx, (uint32_t)pay->sign_mask)) return nullptr;
-  if ((double)(pl->nboxes + 1) * f->d.kg * 32.0 >= 4294967296.0) return nullptr;
+  if (!fold_fits(f->d, pl->nboxes, 1)) return nullptr;
   // blocks of a level: the table level, or the split's source level
   auto level_key = [&](int k) {
     int64_t l = keys.lev[k];
@@ -2331,6 +2331,10 @@ static bool uses_fold(const vl1_plan* pl, int form, int S, int n_rhs) {
   return form != VL1_FORM_SPLIT_I8 || i8_sums_fit(steps, pl->KP, S);
 }
 
+static FoldTile plan_tile(const vl1_plan* pl, int n_rhs, int nct = 0) {
+  return fold_tile(pl->fold->d, pl->nboxes, pl->n_tgt, n_rhs, nct);
+}
+
 // Checks, then builds (allocating) the slice set and tile schedule this
 // evaluation needs if the plan does not hold them yet.
 static int plan_prepare(vl1_plan* pl, int form, int n_rhs, const vl1_split_opts* opts,
@@ -2351,7 +2355,7 @@ static int plan_prepare(vl1_plan* pl, int form, int n_rhs, const vl1_split_opts*
   }
   if (fold) {
     pl->fold_ready |= fold_bit(form, S);
-    out->tile = fold_tile(pl->n_tgt, n_rhs);
+    out->tile = plan_tile(pl, n_rhs);
     if (pl->fold_schedules.empty()) pl->fold_rc = Rc;
     rc = build_fold_schedule(pl, out->tile.B, morton, &out->fold, s);
   } else {
@@ -2366,7 +2370,7 @@ static int plan_prepare(vl1_plan* pl, int form, int n_rhs, const vl1_split_opts*
   for (int R : pl->prepared_rhs) {
     FoldSchedule* fs = nullptr;
     TileSchedule* ts = nullptr;
-    rc = build_fold_schedule(pl, fold_tile(pl->n_tgt, R).B, false, &fs, s);
+    rc = build_fold_schedule(pl, plan_tile(pl, R).B, false, &fs, s);
     if (rc == VL1_OK) rc = build_schedule(pl, R, false, &ts, s);
     if (rc != VL1_OK) return rc;
   }
@@ -2781,9 +2785,9 @@ int vl1_plan_eval_noalloc(vl1_plan* pl, int form, const double* f, int64_t ldf, 
   if (fold) {
     // either tile width serves: a count prepared at another multiple of 64
     // may have taken the other one
-    pr.tile = fold_tile(pl->n_tgt, n_rhs);
+    pr.tile = plan_tile(pl, n_rhs);
     for (int k = 0; k < 2 && !pr.fold; ++k) {
-      if (k) pr.tile = fold_tile(pl->n_tgt, n_rhs, 3 - pr.tile.nct);
+      if (k) pr.tile = plan_tile(pl, n_rhs, 3 - pr.tile.nct);
       auto it = pl->fold_schedules.find(pr.tile.B * 2 + (morton ? 1 : 0));
       if (it != pl->fold_schedules.end()) pr.fold = it->second;
     }
@@ -2921,6 +2925,24 @@ int vl1_plan_set_variant(vl1_plan* pl, int form, int n_slices, int n_rhs, int va
   if ((variant & kVarOneRow) && pl->MP > 128)
     return fail(VL1_E_UNSUPPORTED, "vl1_plan_set_variant: one row tile per wave needs blocks of at most 128 rows");
   pl->tuned[key] = variant;
+  return VL1_OK;
+}
+
+int vl1_plan_fold_tile_host(int dim, int q, int is_complex, int64_t n_boxes, int64_t n_tgt_boxes,
+                            int n_rhs, int64_t* out5) {
+  clear_error();
+  if ((dim != 2 && dim != 3) || q < 1 || q > 16 || n_boxes < 1 || n_boxes > INT32_MAX ||
+      n_tgt_boxes < 0 || n_tgt_boxes > INT32_MAX || n_rhs < 1 || !out5)
+    return fail(VL1_E_ARG, "vl1_plan_fold_tile_host: bad argument");
+  for (int k = 0; k < 5; ++k) out5[k] = 0;
+  FoldPlan f;
+  if (!fold_layout(f, dim, q, is_complex != 0, 0) || !fold_fits(f.d, (int)n_boxes, 1)) return VL1_OK;
+  const FoldTile t = fold_tile(f.d, (int)n_boxes, (int)n_tgt_boxes, n_rhs);
+  out5[0] = 1;
+  out5[1] = 16 * t.nct;
+  out5[2] = t.Rc;
+  out5[3] = t.B;
+  out5[4] = (int64_t)f.d.kg * t.Rc * 32;
   return VL1_OK;
 }
 

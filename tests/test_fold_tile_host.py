@@ -48,3 +48,13 @@ def test_offsets_reach_every_box(dim, q, cplx, nb, n_rhs, factor):
 def test_small_trees_keep_eight_densities():
     assert _tile(3, 6, False, 32768, 64)["rhs"] == 8
     assert _tile(2, 8, True, 4096, 24)["rhs"] == 8
+
+
+@pytest.mark.parametrize("n_rhs", [7, 11, 13, 17, 19, 23, 29, 31, 37, 41, 43, 47, 53, 59, 61])
+def test_prime_counts_share_tiles(n_rhs):
+    """Prime density counts take tiles of several densities with a few columns
+    idle, not one density per tile."""
+    t = _tile(3, 4, False, 4096, n_rhs)
+    groups = -(-n_rhs // t["rhs"])
+    assert t["rhs"] >= 2
+    assert n_rhs * t["boxes"] >= 0.85 * groups * t["columns"]

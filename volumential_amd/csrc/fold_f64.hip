@@ -171,12 +171,21 @@ bool fold_layout(FoldPlan& f, int dim, int q, int cplx, uint32_t sign_mask) {
   return true;
 }
 
-// Densities per tile: the split of R over tiles of `cols` columns that fills
-// them best (R = 24 over 64 columns: 3 x 8 densities of 8 boxes, all columns
-// in use; 59: 15 x 4), the largest up to 8 among equals -- neighbouring boxes
-// in a tile share their sources' cache lines.  Large trees take as many as the
-// kernel's 32-bit offsets reach (3D q = 6: 8 densities up to 299,591 boxes, 4 up
-// to 599,184).
+// Densities per tile: the split of R over tiles of `cols` columns that leaves
+// the fewest columns idle (R = 24 over 64 columns: 3 x 8 densities of 8 boxes,
+// all columns in use; 59: 15 x 4), at a cost by the densities themselves:
+// neighbouring boxes in a tile share their sources' cache lines, so a run of
+// 128 bytes or more per box and K group (4, 8) is best, one density per tile
+// reads a quarter line per box (13 % slower at 64 densities), and counts that
+// are no power of two straddle lines.  Measured, us at 1 / 2 / 4 / 8 densities
+// per tile: 3D q = 6, 4096 boxes, 64 densities 3020 / 2750 / 2651 / 2663; 2D q =
+// 6, 4096 boxes 277 / 245 / 249 / 252.  Prime counts then take 2 or 4 with a few
+// columns idle and not 1: 13 densities, 3D q = 4, 4096 boxes 183 / 164; 29, 2D q
+// = 3, 16384 boxes 346 / 279; 11, 3D q = 6, 4096 boxes 558 / 531.  Narrow tiles
+// run at one workgroup per CU or less, where fewer tiles count for more (7
+// densities, 3D q = 3, 512 boxes: 26 at 1 per tile, 29 at 4).  Large trees
+// take as many as the kernel's 32-bit offsets reach (3D q = 6: 8 densities up
+// to 299,591 boxes, 4 up to 599,184).
 FoldTile fold_tile(const FoldDims& d, int nb, int n_tgt, int R, int nct) {
   const int Rq = std::min(R, 64);  // larger counts are whole multiples of 64
   int rc_max = Rq;
@@ -188,9 +197,18 @@ FoldTile fold_tile(const FoldDims& d, int nb, int n_tgt, int R, int nct) {
     double best = -1.0;
     for (int rc = std::min(rc_max, cols); rc >= 1; --rc) {
       const int nrc = (Rq + rc - 1) / rc, B = cols / rc;
-      double u = (double)Rq / (nrc * rc) * (B * rc) / cols;
-      if (rc > 8) u -= 1e-3;
-      if (rc < 8) u -= 0.02 * std::log2(8.0 / rc);  // short runs per box, more boxes to match
+      double u = (double)Rq * B / (nrc * cols);
+      if (nct == 1) {
+        u -= rc < 8 ? 0.02 * std::log2(8.0 / rc) : (rc > 8 ? 1e-3 : 0.0);
+      } else {
+        switch (rc) {
+          case 8: break;
+          case 4: u *= 0.995; break;
+          case 2: u *= 0.965; break;
+          case 1: u *= 0.87; break;
+          default: u *= (rc & (rc - 1)) == 0 ? 0.97 : 0.92;
+        }
+      }
       if (u > best) {
         best = u;
         t.Rc = rc;

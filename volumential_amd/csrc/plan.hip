@@ -2736,7 +2736,7 @@ int vl1_plan_contract(vl1_plan* pl, int form, int n_rhs, double* y, int64_t ldy,
 // with that device current.
 // Staging is accepted up to kScratchBytes by the plain layouts; the folded
 // layout of the same call pads its parities to 4 and its densities to whole
-// tiles, and holds 8 bytes where 5 int8 slices take 5 (at most 1.64 x 1.08 of
+// tiles, and holds 8 bytes where 5 int8 slices take 5 (at most 1.64 x 1.15 of
 // the plain layout beyond a few boxes, 3D q = 3), which the array holds too.
 constexpr size_t kScratchBytes = (size_t)64 << 20;
 constexpr size_t kScratchArray = (size_t)128 << 20;

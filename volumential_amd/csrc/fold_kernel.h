@@ -51,7 +51,10 @@ constexpr bool fold_whole(int np, int nct, int g0, int g1, int g2, int g3) {
 // for a class with m nonzero axes; which units a wave takes comes from a table
 // (scalar loads).  Per chunk every thread loads the same number of values (16
 // bytes each), forms the 2^m signed sums of its sources in registers and
-// writes them, in MFMA operand order (conflict free), to the LDS slot.  The
+// writes them, in MFMA operand order (conflict free), to the LDS slot.  Orders
+// of few rounds skip the loads that no unit of theirs reads (known when
+// compiled: 3D q = 4, 32768 boxes, 64 densities 5309 -> 5038 us, the digit kernel
+// at 5 slices 5066; 3D q = 2 1431 -> 1038; 2D q = 4, 65536 boxes 2318 -> 2006).  The
 // loads of the next chunk are issued before this chunk's MFMAs; table
 // fragments run one or three units ahead and the lists of source boxes four steps
 // ahead (an LDS ring).  All of them are issued unconditionally -- a skipped
@@ -68,11 +71,14 @@ constexpr bool fold_whole(int np, int nct, int g0, int g1, int g2, int g3) {
 // us with the products at raised priority and the tile's entry and exit as below).
 // The FP64 pipe is then busy about 55% of the time; the load path (fragments
 // and values) about 60%.
-template <int NP, int NCT, int G, bool WHOLE>
+template <int NP, int NCT, int G, int RMAX, bool WHOLE>
 __device__ __forceinline__ void fold_run(const FoldParams& p, double* smem, int bt, int rcx,
                                          int pout, int grow) {
   constexpr int T = 64 * NP, COLS = 16 * NCT, UW = kFoldUnits;
   constexpr int LPT = COLS / 4;             // 16-byte loads per thread and chunk
+  // ... of which those past the orders' RMAX rounds (the rows of the largest
+  // parity, groups of 4) hold nothing: a round is one load of 32 columns, half of 16
+  constexpr int NU = COLS == 32 ? RMAX : (RMAX + 1) / 2;
   constexpr int NXB = LPT > NP ? LPT : NP;  // registers for them (2^m <= NP)
   constexpr int SLOT = UW * NP * NCT * 64;  // doubles of the LDS slot
   constexpr int NT = G / 4, GC = G % 4, NF = NT > 0 ? NT : 1, NG = GC > 0 ? GC : 1;
@@ -121,7 +127,7 @@ __device__ __forceinline__ void fold_run(const FoldParams& p, double* smem, int 
   const uint2* lutl = p.lut_l + (int64_t)CV * 4 * p.maxc * NP + wave;
   auto load_m = [&](uint2 kgs, auto mc) {
     constexpr int M = decltype(mc)::value;
-    constexpr int NI = (LPT >> M) > 0 ? (LPT >> M) : 1;
+    constexpr int NI = std::min((LPT >> M) > 0 ? (LPT >> M) : 1, NU);
     const uint32_t* q = ring + (step & 3) * 32 * NP + (live ? cb : 0) * NP;
     uint32_t vo[1 << M];
 #pragma unroll
@@ -138,7 +144,7 @@ __device__ __forceinline__ void fold_run(const FoldParams& p, double* smem, int 
   const int lds0 = (kgo * NCT + col / 16) * 64 + 48 * kp + col % 16;
   auto store_m = [&](auto mc) {
     constexpr int M = decltype(mc)::value;
-    constexpr int NI = (LPT >> M) > 0 ? (LPT >> M) : 1, NK = (UW * NP) >> M;
+    constexpr int NI = std::min((LPT >> M) > 0 ? (LPT >> M) : 1, NU), NK = (UW * NP) >> M;
     // (opaque, so that the addresses of every m are not all kept in registers)
     int lds = lds0;
     asm volatile("" : "+v"(lds));
@@ -404,14 +410,14 @@ __global__ void __launch_bounds__(64 * NP, G0 <= 8 ? 4 : 2) fold_f64_kernel(cons
     if (k < pout) grow += (int)((p.d.groups_lo >> (8 * k)) & 255);
   constexpr bool WHOLE = fold_whole(NP, NCT, G0, G1, G2, G3);
   if constexpr (G0 == G1 && G1 == G2 && G2 == G3) {
-    fold_run<NP, NCT, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
+    fold_run<NP, NCT, G0, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
   } else {
     // the loops hold the same barriers, so waves may run different ones
     const int odd = __popc(pout);
-    if (odd == 0) fold_run<NP, NCT, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
-    else if (odd == 1) fold_run<NP, NCT, G1, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
-    else if (odd == 2) fold_run<NP, NCT, G2, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
-    else if constexpr (NP == 8) fold_run<NP, NCT, G3, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
+    if (odd == 0) fold_run<NP, NCT, G0, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
+    else if (odd == 1) fold_run<NP, NCT, G1, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
+    else if (odd == 2) fold_run<NP, NCT, G2, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
+    else if constexpr (NP == 8) fold_run<NP, NCT, G3, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
   }
 }
 

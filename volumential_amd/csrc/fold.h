@@ -133,9 +133,9 @@ struct FoldPlan {
   std::vector<int32_t> start, cls, src;  // src [entry][np], -1: none
 };
 
-// Folded basis of q^dim nodes (2 values per node if complex); false: sizes
-// the kernel does not take.
-bool fold_layout(FoldPlan& f, int dim, int q, int cplx, uint32_t sign_mask);
+// Folded basis of q^dim nodes (2 values per node if complex) for plans of n_tgt
+// target boxes; false: sizes the kernel does not take.
+bool fold_layout(FoldPlan& f, int dim, int q, int cplx, uint32_t sign_mask, int n_tgt);
 // Whether the tile kernel's 32-bit byte offsets reach all nb boxes and the zero
 // box at Rc densities per tile (a box holds kg K groups of 32 Rc bytes; a lane
 // reads up to one box past its own offset).

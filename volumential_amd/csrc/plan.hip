@@ -1771,7 +1771,7 @@ static std::unique_ptr<FoldPlan> fold_classes(const vl1_plan* pl, const vl1_payl
                                               const std::vector<int64_t>& key_vid, BlockList& keys) {
   const int dim = pl->dim;
   auto f = std::unique_ptr<FoldPlan>(new FoldPlan());
-  if (!fold_layout(*f, dim, pay->q, pl->cplx, (uint32_t)pay->sign_mask)) return nullptr;
+  if (!fold_layout(*f, dim, pay->q, pl->cplx, (uint32_t)pay->sign_mask, pl->n_tgt)) return nullptr;
   if (!fold_fits(f->d, pl->nboxes, 1)) return nullptr;
   // blocks of a level: the table level, or the split's source level
   auto level_key = [&](int k) {
@@ -2936,7 +2936,7 @@ int vl1_plan_fold_tile_host(int dim, int q, int is_complex, int64_t n_boxes, int
     return fail(VL1_E_ARG, "vl1_plan_fold_tile_host: bad argument");
   for (int k = 0; k < 5; ++k) out5[k] = 0;
   FoldPlan f;
-  if (!fold_layout(f, dim, q, is_complex != 0, 0) || !fold_fits(f.d, (int)n_boxes, 1)) return VL1_OK;
+  if (!fold_layout(f, dim, q, is_complex != 0, 0, (int)n_tgt_boxes) || !fold_fits(f.d, (int)n_boxes, 1)) return VL1_OK;
   const FoldTile t = fold_tile(f.d, (int)n_boxes, (int)n_tgt_boxes, n_rhs);
   out5[0] = 1;
   out5[1] = 16 * t.nct;

@@ -363,6 +363,9 @@ int vl1_plan_tune(vl1_plan* plan, int form, const double* f, int64_t ldf, int n_
  * VL1_E_UNSUPPORTED for one row tile per wave on blocks of more than 128
  * rows.  n_slices is ignored for VL1_FORM_F64. */
 int vl1_plan_set_variant(vl1_plan* plan, int form, int n_slices, int n_rhs, int variant);
+/* *folded = 1 if the plan holds the reflection-folded FP64 form (then the FP64
+ * form and the split forms at 5 and 6 slices run on it), else 0. */
+int vl1_plan_folded(const vl1_plan* plan, int* folded);
 /* The tile a folded plan of these sizes takes (host only): {1 if the folded
  * kernel takes such boxes, columns, densities per tile, boxes per tile, bytes
  * of a box's staged densities in a tile}, zeros if it does not. */

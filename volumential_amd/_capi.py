@@ -67,6 +67,7 @@ EXPORTED_SYMBOLS = (
     "vl1_plan_eval",
     "vl1_plan_stage",
     "vl1_plan_contract",
+    "vl1_plan_folded",
     "vl1_plan_fold_tile_host",
     "vl1_plan_stats",
     "vl1_plan_eval_noalloc",
@@ -342,6 +343,7 @@ def lib():
     L.vl1_plan_tune.argtypes = [vp, C.c_int, vp, i64, C.c_int, vp, i64, C.POINTER(SplitOpts),
                                 C.c_int, C.POINTER(i32), C.POINTER(f64), vp]
     L.vl1_plan_set_variant.argtypes = [vp, C.c_int, C.c_int, C.c_int, C.c_int]
+    L.vl1_plan_folded.argtypes = [vp, C.POINTER(C.c_int)]
     L.vl1_plan_fold_tile_host.argtypes = [C.c_int, C.c_int, C.c_int, i64, i64, C.c_int, vp]
     L.vl1_duffy_build.argtypes = [C.POINTER(DuffyArgs), vp]
     L.vl1_duffy_build_tensor.argtypes = [C.POINTER(DuffyTensorArgs), vp]

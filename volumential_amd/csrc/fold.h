@@ -150,8 +150,10 @@ size_t fold_x_size(const FoldDims& d, const FoldTile& t, int nb, int R);
 size_t fold_dl_size(const FoldTile& t, int nb, int R);
 // A[class] from the representatives' blocks in M [blocks x n_rg][MP][KP], and
 // *flag = 1 unless every key's block is the reflection of its class's
-// representative by the folded axes key_flips[key], to 1e-14 of that block's
-// largest entry.  Returns after the device has finished.
+// representative by the folded axes key_flips[key], and every representative
+// its own reflection along each folded axis on which its case vector is zero
+// (the product has no terms between the parities of such an axis), to 1e-14 of
+// the representative's largest entry.  Returns after the device has finished.
 hipError_t fold_build_launch(FoldPlan& f, int dim, int q, const double* M, int MP, int KP, int n_rg,
                              int rg_size, int32_t* flag, hipStream_t s);
 hipError_t fold_stage_launch(const FoldPlan& f, const FoldTile& t, int nb, int R, const double* fin,

@@ -340,12 +340,14 @@ __global__ void __launch_bounds__(256)
   if (threadIdx.x == 0) mx[blockIdx.x] = red[0];
 }
 
+// Check b: block blk[b] against class cls[b]'s representative reflected along
+// flips[b].
 __global__ void __launch_bounds__(256)
     fold_check_kernel(int dim, int q, int n, int rows, uint32_t sp, const double* __restrict__ M,
                       int MP, int KP, int n_rg, int rg_size, const int32_t* __restrict__ rep_blk,
-                      const int32_t* __restrict__ key_cls, const int32_t* __restrict__ key_flips,
-                      int n_keys, const double* __restrict__ blk_max, int32_t* __restrict__ flag) {
-  const int64_t total = (int64_t)n_keys * rows * rows;
+                      const int32_t* __restrict__ blk_of, const int32_t* __restrict__ cls,
+                      const int32_t* __restrict__ flips, int n_checks, const double* __restrict__ blk_max, int32_t* __restrict__ flag) {
+  const int64_t total = (int64_t)n_checks * rows * rows;
   auto at = [&](int blk, int t, int s) {
     return M[((int64_t)(blk * n_rg + t / rg_size) * MP + t % rg_size) * KP + s];
   };
@@ -353,9 +355,9 @@ __global__ void __launch_bounds__(256)
        i += (int64_t)gridDim.x * blockDim.x) {
     const int s = (int)(i % rows), t = (int)((i / rows) % rows);
     const int b = (int)(i / ((int64_t)rows * rows));
-    const int c = key_cls[b], J = key_flips[b];
+    const int c = cls[b], J = flips[b];
     const double want = at(rep_blk[c], t, s);
-    const double got = at(b, t / n * n + reflect_node(dim, q, t % n, J),
+    const double got = at(blk_of[b], t / n * n + reflect_node(dim, q, t % n, J),
                           s / n * n + reflect_node(dim, q, s % n, J));
     const double e = (__popc((unsigned)J & sp) & 1) ? got + want : got - want;
     if (!(fabs(e) <= 1e-14 * blk_max[c]) || !(blk_max[c] <= 1.7e308)) atomicOr(flag, 1);
@@ -472,14 +474,26 @@ hipError_t fold_build_launch(FoldPlan& f, int dim, int q, const double* M, int M
     if (src) std::memcpy(h.data() + at, src, bytes);
     return at;
   };
+  // every key against its representative, then every representative against
+  // itself along its zero axes
   const int n_keys = (int)f.key_cls.size();
+  std::vector<int32_t> blk(n_keys), cls(f.key_cls), flips(f.key_flips);
+  for (int k = 0; k < n_keys; ++k) blk[k] = k;
+  for (int c = 0; c < f.n_cls; ++c)
+    for (int a = 0; a < f.d.nf; ++a)
+      if (!((f.zmask[c] >> a) & 1)) {
+        blk.push_back(f.rep_blk[c]);
+        cls.push_back(c);
+        flips.push_back(1 << a);
+      }
   const size_t o_u = put(f.lut_u.data(), f.lut_u.size() * sizeof(uint4));
   const size_t o_l = put(f.lut_l.data(), f.lut_l.size() * sizeof(uint2));
   const size_t o_s = put(f.slots.data(), f.slots.size() * sizeof(FoldSlot));
   const size_t o_o = put(f.outs.data(), f.outs.size() * sizeof(FoldOut));
   const size_t o_r = put(f.rep_blk.data(), f.rep_blk.size() * 4);
-  const size_t o_c = put(f.key_cls.data(), f.key_cls.size() * 4);
-  const size_t o_f = put(f.key_flips.data(), f.key_flips.size() * 4);
+  const size_t o_b = put(blk.data(), blk.size() * 4);
+  const size_t o_c = put(cls.data(), cls.size() * 4);
+  const size_t o_f = put(flips.data(), flips.size() * 4);
   const size_t o_m = put(nullptr, (size_t)f.n_cls * 8);
   const size_t o_g = put(nullptr, 4);
   f.cls_stride = (int64_t)f.d.kg * f.d.rows4 * 4;
@@ -498,10 +512,11 @@ hipError_t fold_build_launch(FoldPlan& f, int dim, int q, const double* M, int M
   auto blocks = [](int64_t n) { return dim3((unsigned)std::min<int64_t>((n + 255) / 256, 65536)); };
   hipLaunchKernelGGL(fold_max_kernel, dim3(f.n_cls), dim3(256), 0, s, (int64_t)n_rg * MP * KP, rep, M,
                      mx);
-  hipLaunchKernelGGL(fold_check_kernel, blocks((int64_t)n_keys * f.rows * f.rows), dim3(256), 0, s, dim,
+  hipLaunchKernelGGL(fold_check_kernel, blocks((int64_t)blk.size() * f.rows * f.rows), dim3(256), 0, s, dim,
                      q, f.nm, f.rows, f.d.sp, M, MP, KP, n_rg, rg_size, rep,
+                     reinterpret_cast<const int32_t*>(d + o_b),
                      reinterpret_cast<const int32_t*>(d + o_c),
-                     reinterpret_cast<const int32_t*>(d + o_f), n_keys, mx, dflag);
+                     reinterpret_cast<const int32_t*>(d + o_f), (int)blk.size(), mx, dflag);
   hipLaunchKernelGGL(fold_table_kernel, blocks(total), dim3(256), 0, s, f.d, f.n_cls, f.slot_lut, rep,
                      MP, KP, n_rg, rg_size, M, f.A.as<double>());
   e = hipGetLastError();

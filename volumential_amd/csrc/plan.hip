@@ -1824,8 +1824,9 @@ static std::unique_ptr<FoldPlan> fold_classes(const vl1_plan* pl, const vl1_payl
 
 // Second half, after the blocks are expanded: the representatives' blocks in
 // the folded basis, kept unless a block is not the reflection of its class's
-// representative (descriptors without the reflection symmetry of a list-1
-// table).
+// representative or a representative not its own along an axis where its case
+// vector is zero (descriptors without the reflection symmetry of a list-1
+// table, middle-node values of a derivative table).
 static hipError_t fold_tables(vl1_plan* pl, std::unique_ptr<FoldPlan> f, int q, hipStream_t s) {
   int32_t flag = 0;
   const hipError_t e = fold_build_launch(*f, pl->dim, q, pl->M.as<double>(), pl->MP, pl->KP, pl->n_rg,
@@ -2925,6 +2926,13 @@ int vl1_plan_set_variant(vl1_plan* pl, int form, int n_slices, int n_rhs, int va
   if ((variant & kVarOneRow) && pl->MP > 128)
     return fail(VL1_E_UNSUPPORTED, "vl1_plan_set_variant: one row tile per wave needs blocks of at most 128 rows");
   pl->tuned[key] = variant;
+  return VL1_OK;
+}
+
+int vl1_plan_folded(const vl1_plan* pl, int* folded) {
+  clear_error();
+  if (!pl || !folded) return fail(VL1_E_ARG, "vl1_plan_folded: null argument");
+  *folded = pl->fold ? 1 : 0;
   return VL1_OK;
 }
 

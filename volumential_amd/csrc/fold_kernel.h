@@ -76,9 +76,12 @@ __device__ __forceinline__ void fold_run(const FoldParams& p, double* smem, int 
                                          int pout, int grow) {
   constexpr int T = 64 * NP, COLS = 16 * NCT, UW = kFoldUnits;
   constexpr int LPT = COLS / 4;             // 16-byte loads per thread and chunk
-  // ... of which those past the orders' RMAX rounds (the rows of the largest
-  // parity, groups of 4) hold nothing: a round is one load of 32 columns, half of 16
-  constexpr int NU = COLS == 32 ? RMAX : (RMAX + 1) / 2;
+  // ... of which those past the order's RMAX rounds (the rows of the largest
+  // parity, groups of 4) hold nothing: a round is one load of 32 columns, half of
+  // 16.  From 4 rounds on all are issued: of the chunks only a step with no
+  // nonzero axis has such loads, and the kernel built without them was slower (3D
+  // q = 4 complex, 4096 boxes, 5 densities 118 -> 130 us; 2D q = 6 equal).
+  constexpr int NU = RMAX >= 4 ? LPT : (COLS == 32 ? RMAX : (RMAX + 1) / 2);
   constexpr int NXB = LPT > NP ? LPT : NP;  // registers for them (2^m <= NP)
   constexpr int SLOT = UW * NP * NCT * 64;  // doubles of the LDS slot
   constexpr int NT = G / 4, GC = G % 4, NF = NT > 0 ? NT : 1, NG = GC > 0 ? GC : 1;

@@ -52,17 +52,17 @@ def as_dict(m, dim, q):
 
 
 def plan_of(tr, dim, q, m, v, **kw):
-    nm = np.random.default_rng(5).standard_normal((1, q**dim))
+    nm = np.random.default_rng(5).standard_normal((1, q**dim)).astype(v.dtype)
     pay = DevicePayload(dim, q, v[None], nm, orbit_ref.case_metadata(dim, q)["case_indices"], m)
     return List1Plan(tr, pay, scaling_mode=_capi.SCALING_CANONICAL, scaling_power=2,
                      table_root_extent=2.0, **kw), nm
 
 
-def check(plan, nm, tr, dim, q, m, v, f):
+def check(plan, nm, tr, dim, q, m, v, f, scale=1.0):
     got = plan.eval(torch.as_tensor(f, device="cuda"), form="f64").cpu().numpy()
     ref = list1_ref.near_field_from_tree(tr, v[None], nm, as_dict(m, dim, q), f, mode="canonical",
                                          scaling_power=2, table_root_extent=2.0)
-    l2, linf = rel_errors(got, ref)
+    l2, linf = rel_errors(got * scale, ref * scale)
     assert l2 <= TOL and linf <= TOL, (l2, linf)
 
 
@@ -90,6 +90,21 @@ def test_middle_node_derivative_values(cuda, dim, q):
     plan, nm = plan_of(tr, dim, q, m, v)
     assert not folded(plan)
     check(plan, nm, tr, dim, q, m, v, rng.standard_normal((3, tr.n_points)))
+
+
+@pytest.mark.parametrize("dim,q", [(2, 4), (3, 4)])
+def test_entries_near_overflow(cuda, dim, q):
+    """The folded blocks add up to 64 entries: tables whose sums leave the
+    range keep the general form."""
+    print(f"case: entries near overflow {dim}D q={q}", flush=True)
+    tr = adaptive(dim, q, max_level=3)
+    m = orbit.build_case_metadata(dim, q)
+    rng = np.random.default_rng(q)
+    v = 1e308 * rng.uniform(0.5, 1.0, m.n_compact_entries)
+    plan, nm = plan_of(tr, dim, q, m, v)
+    assert not folded(plan)
+    # (the norms' squares stay in range at 2^-600)
+    check(plan, nm, tr, dim, q, m, v, 1e-10 * rng.standard_normal((3, tr.n_points)), 2.0**-600)
 
 
 @pytest.mark.parametrize("kernel", ["laplace", "gradient", "helmholtz", "helmholtz gradient"])

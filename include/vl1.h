@@ -266,7 +266,8 @@ typedef struct vl1_split_opts {
    * diagonal kept, the size of the first diagonal dropped, per output; 2^-52
    * where nothing is dropped (5 and 6 slices of a plan with
    * reflection-symmetric blocks run on the FP64 form's folded kernel, which is
-   * faster there).  FP64 rounding itself is not part of it. */
+   * faster there).  FP64 rounding itself is not part of it.  NaN where an
+   * output is infinite or NaN. */
   double* error_est;
 } vl1_split_opts;
 

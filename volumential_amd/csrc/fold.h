@@ -64,6 +64,15 @@ struct FoldTileInfo {
   uint32_t words[4];
 };
 
+// The blocks themselves, for outputs that are not finite (fold_nonfinite): read
+// through one pointer, so that the tile kernel keeps none of it in registers.
+struct FoldBlocks {
+  const FoldSlot* slots;   // [kg][4]
+  const double* M;         // [blocks x n_rg][MP][KP]
+  const int32_t* rep_blk;  // block of a class's representative
+  int dim, q, MP, KP, n_rg, rg_size;
+};
+
 struct FoldParams {
   FoldDims d;
   int B, Rc, R;            // boxes per tile, densities per tile, densities in all
@@ -86,7 +95,26 @@ struct FoldParams {
   const int32_t* mode_point;
   double* y;
   int64_t ldy;
+  const struct FoldBlocks* blocks;  // device: for outputs that are not finite
+  double* est;                     // their densities' error estimates [R][2], or null
 };
+
+// A value of a density that is not finite makes all sums of its mirror nodes
+// so.  Their places in X then hold the nodes' own values instead: infinities
+// and NaN as they are, finite ones as this NaN.
+constexpr double kFoldMax = 1.7976931348623157e308;
+constexpr uint64_t kFoldFinite = 0x7ff8000000f01d00ull;
+
+__device__ inline int reflect_node(int dim, int q, int node, int flips) {
+  int out = 0, stride = 1;
+  for (int a = dim - 1; a >= 0; --a) {
+    const int i = node % q;
+    node /= q;
+    out += (((flips >> a) & 1) ? q - 1 - i : i) * stride;
+    stride *= q;
+  }
+  return out;
+}
 
 // A chunk of a step: class, its nonzero folded axes z and their number m, the
 // chunk within the step, and whether it is the step's first.
@@ -118,9 +146,10 @@ struct FoldPlan {
   std::vector<uint4> lut_u;
   std::vector<uint2> lut_l;
   int maxc = 0;
-  DevBuf lut, A;  // lut: the four tables, and the class lists of the build
+  DevBuf lut, A;  // lut: the tables, and the class lists of the build
   const FoldSlot* slot_lut = nullptr;  // device, in lut
   const FoldOut* out_lut = nullptr;
+  const FoldBlocks* blocks = nullptr;
   const uint4* u_lut = nullptr;
   const uint2* l_lut = nullptr;
   int64_t cls_stride = 0;
@@ -153,7 +182,8 @@ size_t fold_dl_size(const FoldTile& t, int nb, int R);
 // representative by the folded axes key_flips[key], and every representative
 // its own reflection along each folded axis on which its case vector is zero
 // (the product has no terms between the parities of such an axis), to 1e-14 of
-// the representative's largest entry.  Returns after the device has finished.
+// the representative's largest entry.  Keeps M for outputs that are not finite.
+// Returns after the device has finished.
 hipError_t fold_build_launch(FoldPlan& f, int dim, int q, const double* M, int MP, int KP, int n_rg,
                              int rg_size, int32_t* flag, hipStream_t s);
 hipError_t fold_stage_launch(const FoldPlan& f, const FoldTile& t, int nb, int R, const double* fin,

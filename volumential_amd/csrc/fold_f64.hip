@@ -306,17 +306,6 @@ __global__ void __launch_bounds__(256)
   }
 }
 
-__device__ inline int reflect_node(int dim, int q, int node, int flips) {
-  int out = 0, stride = 1;
-  for (int a = dim - 1; a >= 0; --a) {
-    const int i = node % q;
-    node /= q;
-    out += (((flips >> a) & 1) ? q - 1 - i : i) * stride;
-    stride *= q;
-  }
-  return out;
-}
-
 // mx[c] = largest |entry| of class c's representative (infinite if one is not
 // finite); rows past a group are zero in M.
 __global__ void __launch_bounds__(256)
@@ -372,7 +361,8 @@ __global__ void __launch_bounds__(256)
 // values of one (box, density), with the box's node ids read once for all
 // densities and kStageK values in flight per lane, into LDS in mode order; then
 // a thread keeps one entry of the basis, reads its up to 8 terms at once and
-// writes in output order (consecutive threads, consecutive doubles; 4 x 2^re
+// writes in output order (values that are not finite: see kFoldFinite;
+// consecutive threads, consecutive doubles; 4 x 2^re
 // threads for the densities of a K group, 2^gl K groups, the rest of the block
 // for other boxes: 8.5 -> 5.9 us at q = 4, 4096 boxes, one density).
 // Bound: memory, once the loads overlap: 4096 boxes, q = 6, 24 densities (350
@@ -400,6 +390,7 @@ __global__ void __launch_bounds__(256)
   const int ebx = tid >> (2 + re + gl), bxstep = 64 >> (re + gl);
   for (int q0 = 0; q0 < Rc; q0 += rs) {
     const int nr = min(rs, Rc - q0);
+    double finite = 0.0;
     for (int b = bln; b < nbx; b += bstep) {
       const int box = b0 + b;
       const double al = box < nb ? box_alpha[box] : 0.0;
@@ -458,6 +449,22 @@ __global__ void __launch_bounds__(256)
           }
           X[(((int64_t)rcx * (nb + 1) + box) * d.kg + kg) * Rc * 4 + (q0 + er) * 4 + ek] =
               s.valid ? v : 0.0;
+          finite = fma(v, 0.0, finite);
+        }
+      }
+    if (finite != 0.0 && er < nr)  // NaN: some sum of this thread's is not finite
+      for (int kg = ekg; kg < d.kg; kg += kgstep) {
+        const FoldSlot s = slots[kg * 4 + (ek ^ (ek >> 1))];
+        for (int b = ebx; b < nbx; b += bxstep) {
+          double* at = X + (((int64_t)rcx * (nb + 1) + b0 + b) * d.kg + kg) * Rc * 4 + (q0 + er) * 4 + ek;
+          if (fabs(*at) <= kFoldMax) continue;
+          // the node of sign pattern par itself
+          int node = s.base;
+          for (int a = 0; a < d.nf; ++a)
+            if ((s.par >> a) & 1) node += s.d[a];
+          const double own = sv[(b * rs + er) * LS + node];
+          *at = fabs(own) <= kFoldMax ? __longlong_as_double(kFoldFinite)
+                                      : (own != own ? __builtin_nan("") : own);
         }
       }
     __syncthreads();
@@ -497,6 +504,7 @@ hipError_t fold_build_launch(FoldPlan& f, int dim, int q, const double* M, int M
   const size_t o_f = put(flips.data(), flips.size() * 4);
   const size_t o_m = put(nullptr, (size_t)f.n_cls * 8);
   const size_t o_g = put(nullptr, 4);
+  const size_t o_k = put(nullptr, sizeof(FoldBlocks));
   f.cls_stride = (int64_t)f.d.kg * f.d.rows4 * 4;
   const int64_t total = f.cls_stride * f.n_cls;
   hipError_t e = f.A.alloc((size_t)total * sizeof(double));
@@ -521,6 +529,10 @@ hipError_t fold_build_launch(FoldPlan& f, int dim, int q, const double* M, int M
   hipLaunchKernelGGL(fold_table_kernel, blocks(total), dim3(256), 0, s, f.d, f.n_cls, f.slot_lut, rep,
                      MP, KP, n_rg, rg_size, M, f.A.as<double>());
   e = hipGetLastError();
+  const FoldBlocks blocks_of{f.slot_lut, M, rep, dim, q, MP, KP, n_rg, rg_size};
+  f.blocks = reinterpret_cast<const FoldBlocks*>(d + o_k);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(d + o_k, &blocks_of, sizeof(blocks_of), hipMemcpyHostToDevice, s);
   if (e == hipSuccess) e = hipMemcpyAsync(flag, dflag, 4, hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   return e;

@@ -32,6 +32,60 @@ constexpr bool fold_whole(int np, int nct, int g0, int g1, int g2, int g3) {
          fold_rows4(np, g0, g1, g2, g3) * (16 * nct + 1) <= kFoldUnits * np * nct * 64 + 576;
 }
 
+// For a thread with outputs that came out infinite or NaN: each of its outputs
+// again, as the products of the densities' infinities and NaN with their entries
+// of the blocks, the signed infinity or NaN that the sum over sources has
+// (finite products do not matter).  Outputs without any keep what was written.
+template <int NP>
+__device__ inline void fold_nonfinite(const FoldParams& p, const double* smem) {
+  const int n_rc = (p.R + p.Rc - 1) / p.Rc;
+  const int i8 = (int)(blockIdx.x / 8), bt = i8 / n_rc * 8 + (int)(blockIdx.x % 8), rcx = i8 % n_rc;
+  const FoldTileInfo& ti = p.tiles[bt];
+  const double* log_sums = smem + p.slot_doubles + 32 * NP * 2 + 64 * NP;
+  const FoldBlocks& f = *p.blocks;
+  const int row = threadIdx.x % p.rows;
+  const double* Xc = p.X + (int64_t)rcx * (p.nb + 1) * p.d.kg * p.Rc * 4;
+  // (as in fold_run: one row, every cpt-th column)
+  const int cpt = 64 * NP / p.rows;
+  for (int c = threadIdx.x / p.rows; c < p.B * p.Rc; c += cpt) {
+    const int b = c / p.Rc, r = c % p.Rc, R = rcx * p.Rc + r, box = p.tile_boxes[bt * p.B + b];
+    if ((int)threadIdx.x >= cpt * p.rows || R >= p.R || box < 0) continue;
+    double sum = 0.0;
+    bool any = false;
+    int64_t step = ti.step - 1;
+    for (int i = 0; i < ti.n_chunks; ++i) {
+      const uint32_t w = p.chunks[ti.chunk + i];
+      if (!fold_chunk_first(w)) continue;
+      ++step;
+      const int z = fold_chunk_z(w), blk = f.rep_blk[fold_chunk_cls(w)] * f.n_rg;
+      for (int j = 0; j < 1 << fold_chunk_m(w); ++j) {
+        const int src = p.step_src[(step * p.B + b) * NP + j];
+        if (src == p.nb) continue;
+        int J = 0;  // the slot's negative axes
+        for (int a = 0, k = 0; a < 3; ++a)
+          if ((z >> a) & 1) J |= ((j >> k++) & 1) << a;
+        const int t = row / p.nm * p.nm + reflect_node(f.dim, f.q, row % p.nm, J);
+        const double* m = f.M + ((int64_t)(blk + t / f.rg_size) * f.MP + t % f.rg_size) * f.KP;
+        const double eps = (__popc((unsigned)J & p.d.sp) & 1) ? -1.0 : 1.0;
+        for (int e = 0; e < 4 * p.d.kg; ++e) {
+          const double x = Xc[(((int64_t)src * p.d.kg + e / 4) * p.Rc + r) * 4 + e % 4];
+          if (fabs(x) <= kFoldMax || (uint64_t)__double_as_longlong(x) == kFoldFinite) continue;
+          const FoldSlot s = f.slots[e / 4 * 4 + ((e % 4) ^ ((e % 4) >> 1))];
+          int node = s.base;
+          for (int a = 0; a < 3; ++a)
+            if ((s.par >> a) & 1) node += s.d[a];
+          sum += eps * m[node / p.nm * p.nm + reflect_node(f.dim, f.q, node % p.nm, J)] * x;
+          any = true;
+        }
+      }
+    }
+    if (!any) continue;
+    if (p.est) p.est[2 * R] = p.est[2 * R + 1] = __builtin_nan("");
+    const int64_t mp = p.mode_point[(int64_t)box * p.nm + row % p.nm];
+    p.y[R * p.ldy + (p.cplx ? 2 * mp + row / p.nm : mp)] = p.dl ? sum + log_sums[c] : sum;
+  }
+}
+
 // A workgroup of NP waves computes 16 NCT columns (B target boxes x Rc
 // densities) of all rows; wave w owns the rows of one output parity, G groups
 // of 4, in the accumulators of v_mfma_f64_16x16x4f64 (G / 4 full 16-row
@@ -71,9 +125,10 @@ constexpr bool fold_whole(int np, int nct, int g0, int g1, int g2, int g3) {
 // us with the products at raised priority and the tile's entry and exit as below).
 // The FP64 pipe is then busy about 55% of the time; the load path (fragments
 // and values) about 60%.
+// Returns 0, NaN if an output of this thread is not finite.
 template <int NP, int NCT, int G, int RMAX, bool WHOLE>
-__device__ __forceinline__ void fold_run(const FoldParams& p, double* smem, int bt, int rcx,
-                                         int pout, int grow) {
+__device__ __forceinline__ double fold_run(const FoldParams& p, double* smem, int bt, int rcx,
+                                           int pout, int grow) {
   constexpr int T = 64 * NP, COLS = 16 * NCT, UW = kFoldUnits;
   constexpr int LPT = COLS / 4;             // 16-byte loads per thread and chunk
   // ... of which those past the order's RMAX rounds (the rows of the largest
@@ -355,6 +410,7 @@ __device__ __forceinline__ void fold_run(const FoldParams& p, double* smem, int 
     sD[tid] = a;
   }
   const double scale = 1.0 / (double)(1 << o.shift);
+  double finite = 0.0;  // NaN if an output is not finite
   fold_for<0, COLS / OC>([&](auto occ) {
     constexpr int oc = decltype(occ)::value;
     __syncthreads();
@@ -389,12 +445,14 @@ __device__ __forceinline__ void fold_run(const FoldParams& p, double* smem, int 
               v += (__popc(q & o.flips) & 1) ? -h : h;
             }
           v *= scale;
+          finite = fma(v, 0.0, finite);
           if (p.dl) v += sD[c];
           p.y[sBox[2 * c + 1] + (p.cplx ? 2 * (int64_t)mc[k] + part : (int64_t)mc[k])] = v;
         }
       }
     }
   });
+  return finite;
 }
 
 template <int NP, int NCT, int G0, int G1, int G2, int G3>
@@ -412,15 +470,29 @@ __global__ void __launch_bounds__(64 * NP, G0 <= 8 ? 4 : 2) fold_f64_kernel(cons
   for (int k = 0; k < NP; ++k)
     if (k < pout) grow += (int)((p.d.groups_lo >> (8 * k)) & 255);
   constexpr bool WHOLE = fold_whole(NP, NCT, G0, G1, G2, G3);
+  double finite;
   if constexpr (G0 == G1 && G1 == G2 && G2 == G3) {
-    fold_run<NP, NCT, G0, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
+    finite = fold_run<NP, NCT, G0, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
   } else {
     // the loops hold the same barriers, so waves may run different ones
     const int odd = __popc(pout);
-    if (odd == 0) fold_run<NP, NCT, G0, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
-    else if (odd == 1) fold_run<NP, NCT, G1, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
-    else if (odd == 2) fold_run<NP, NCT, G2, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
-    else if constexpr (NP == 8) fold_run<NP, NCT, G3, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
+    if (odd == 0) finite = fold_run<NP, NCT, G0, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
+    else if (odd == 1) finite = fold_run<NP, NCT, G1, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
+    else if (odd == 2) finite = fold_run<NP, NCT, G2, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
+    else if constexpr (NP == 8) finite = fold_run<NP, NCT, G3, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
+  }
+  if (finite != 0.0) {
+    // the arguments read again: kept in registers for this they spill others of
+    // the loop (4 to 10 % slower)
+    auto args = (uintptr_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    typedef const __attribute__((address_space(4))) uint32_t* scalar_ptr;
+    struct Words {
+      uint32_t w[sizeof(FoldParams) / 4];
+    } words;
+#pragma unroll
+    for (size_t k = 0; k < sizeof(FoldParams) / 4; ++k) words.w[k] = ((scalar_ptr)args)[k];
+    fold_nonfinite<NP>(__builtin_bit_cast(FoldParams, words), fold_smem);
   }
 }
 

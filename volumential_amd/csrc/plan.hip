@@ -2474,12 +2474,16 @@ static int fold_contract(vl1_plan* pl, const Prepared& pr, int R, double* y, int
   p.mode_point = pl->mode_point.as<int32_t>();
   p.y = y;
   p.ldy = ldy;
-  hipError_t e = fold_contract_launch(p, pr.tile, s);
-  if (e == hipSuccess && est) {
-    // no product is cut: what is left is FP64 rounding, which the estimate does not cover
+  p.blocks = f.blocks;
+  p.est = est;
+  hipError_t e = hipSuccess;
+  if (est) {
+    // no product is cut: what is left is FP64 rounding, which the estimate does
+    // not cover; the tiles write NaN for densities with outputs that are not finite
     hipLaunchKernelGGL(fold_est_kernel, dim3((2 * R + 255) / 256), dim3(256), 0, s, 2 * R, est);
     e = hipGetLastError();
   }
+  if (e == hipSuccess) e = fold_contract_launch(p, pr.tile, s);
   if (e != hipSuccess) return fail(VL1_E_HIP, std::string("folded tile launch: ") + hipGetErrorString(e));
   return VL1_OK;
 }

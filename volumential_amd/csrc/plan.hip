@@ -2446,6 +2446,8 @@ static __global__ void fold_est_kernel(int n, double* __restrict__ est) {
   if (i < n) est[i] = 0x1p-52;
 }
 
+constexpr int64_t kMaxThreads = 0xffffffff;  // of one launch
+
 static int fold_contract(vl1_plan* pl, const Prepared& pr, int R, double* y, int64_t ldy,
                          const Staging& st, hipStream_t s, double* est) {
   const FoldPlan& f = *pl->fold;
@@ -2453,7 +2455,6 @@ static int fold_contract(vl1_plan* pl, const Prepared& pr, int R, double* y, int
   p.d = f.d;
   p.B = pr.tile.B;
   p.Rc = pr.tile.Rc;
-  p.R = R;
   p.nb = pl->nboxes;
   p.n_box_tiles = pr.fold->n_tiles;
   p.nm = f.nm;
@@ -2468,14 +2469,10 @@ static int fold_contract(vl1_plan* pl, const Prepared& pr, int R, double* y, int
   p.step_src = pr.fold->step_src.as<int32_t>();
   p.A = f.A.as<double>();
   p.cls_stride = f.cls_stride;
-  p.X = st.XF;
-  p.dl = pl->log_disp ? st.nmdot : nullptr;
   p.out = f.out_lut;
   p.mode_point = pl->mode_point.as<int32_t>();
-  p.y = y;
   p.ldy = ldy;
   p.blocks = f.blocks;
-  p.est = est;
   hipError_t e = hipSuccess;
   if (est) {
     // no product is cut: what is left is FP64 rounding, which the estimate does
@@ -2483,7 +2480,19 @@ static int fold_contract(vl1_plan* pl, const Prepared& pr, int R, double* y, int
     hipLaunchKernelGGL(fold_est_kernel, dim3((2 * R + 255) / 256), dim3(256), 0, s, 2 * R, est);
     e = hipGetLastError();
   }
-  if (e == hipSuccess) e = fold_contract_launch(p, pr.tile, s);
+  // one launch, or several where it would have 2^32 threads or more
+  const int Rc = p.Rc, n_rc = (R + Rc - 1) / Rc;
+  const int64_t threads = (int64_t)((p.n_box_tiles + 7) / 8 * 8) * 64 * f.d.np;
+  const int per = (int)std::max<int64_t>(1, std::min<int64_t>(n_rc, kMaxThreads / threads));
+  for (int g = 0; g < n_rc && e == hipSuccess; g += per) {
+    const int64_t r = (int64_t)g * Rc, cols = r * (p.nb + 1);
+    p.R = std::min(R - (int)r, per * Rc);
+    p.X = st.XF + cols * f.d.kg * 4;
+    p.dl = pl->log_disp ? st.nmdot + cols : nullptr;
+    p.y = y + r * ldy;
+    p.est = est ? est + 2 * r : nullptr;
+    e = fold_contract_launch(p, pr.tile, s);
+  }
   if (e != hipSuccess) return fail(VL1_E_HIP, std::string("folded tile launch: ") + hipGetErrorString(e));
   return VL1_OK;
 }

@@ -36,6 +36,7 @@
 #include <vector>
 
 #include "internal.h"
+#include "split_log.h"
 #include "split_series.h"
 
 namespace vl1 {
@@ -75,32 +76,6 @@ struct SplitCoef {
 
 constexpr int kSplitBoxes = 64;  // source boxes staged together
 constexpr int kSplitPairs = 4;   // sources per lane and pass over the series
-
-// log x for x > 0 by a table of 64 reciprocals (Tang's method): x = 2^e m, m in
-// [1/2, 1), c the midpoint of m's 1/128 interval, log x = e log 2 - log(1/c) +
-// log1p(m / c - 1), the last a polynomial of degree 7 (|m / c - 1| <= 1/128:
-// truncated at 2e-18).  Within 1.2 units of the last place of max(1, |log x|), in 15
-// instructions; the library's log took more than half of the kernel's time.
-struct SplitLog {
-  double inv, log_c;  // 1 / c rounded, -log of that
-};
-constexpr int kSplitLogs = 64;
-__device__ inline void split_log_table(SplitLog* t, int i) {
-  const double inv = 1.0 / (0.5 + (i + 0.5) / (2.0 * kSplitLogs));
-  t[i] = SplitLog{inv, -log(inv)};
-}
-__device__ __forceinline__ double split_log(double x, const SplitLog* t) {
-  const double m = __builtin_amdgcn_frexp_mant(x);
-  const int e = __builtin_amdgcn_frexp_exp(x);
-  const SplitLog q = t[(__double2hiint(m) >> 14) & (kSplitLogs - 1)];
-  const double r = fma(m, q.inv, -1.0), r2 = r * r;
-  double p = fma(r, 1.0 / 7.0, -1.0 / 6.0);
-  p = fma(p, r, 1.0 / 5.0);
-  p = fma(p, r, -1.0 / 4.0);
-  p = fma(p, r, 1.0 / 3.0);
-  p = fma(p, r, -1.0 / 2.0);
-  return fma((double)e, M_LN2, q.log_c) + fma(p, r2, r);
-}
 
 // The series of remainder_value / remainder_radial_derivative at U points, with
 // each coefficient read once.  QUARTER (2D): s_n real and Im b_n = s_n / 4.

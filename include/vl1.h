@@ -432,7 +432,9 @@ int vl1_duffy_build(const vl1_duffy_args* a, void* stream);
 
 /* The same entries in 3D from the rule's one-dimensional parts (all sign
  * vectors and axis orders; radial nodes x tail nodes x tail nodes), summed
- * axis by axis: entries grouped by target point. */
+ * axis by axis: entries grouped by target point.  Entries of no target point, of
+ * a range outside the arrays or past max_entries, and with a mode outside the box
+ * come out as NaN. */
 typedef struct vl1_duffy_tensor_args {
   int dim;                  /* 3 */
   int quad_order;

@@ -71,9 +71,12 @@ __global__ void __launch_bounds__(kDtThreads) duffy_tensor_kernel(const DuffyTen
   const int tid = threadIdx.x;
   const int64_t tgt = blockIdx.x;
   const int b = blockIdx.y;
-  const int64_t e0 = p.start[tgt] + (int64_t)blockIdx.z * kDtThreads * kDtAcc;
-  const int ne = (int)min<int64_t>(p.start[tgt + 1] - e0, kDtThreads * kDtAcc);
-  if (ne <= 0 || e0 < 0 || e0 + ne > p.n_entries) return;  // uniform
+  const int64_t first = p.start[tgt], last = p.start[tgt + 1];
+  const int64_t e0 = first + (int64_t)blockIdx.z * kDtThreads * kDtAcc;
+  // (uniform; entries of ranges outside the arrays, and those past max_entries
+  // or of no target point, keep duffy_tensor_fill_kernel's NaN)
+  if (last <= e0 || first < 0 || last > p.n_entries) return;
+  const int ne = (int)min<int64_t>(last - e0, kDtThreads * kDtAcc);
   double* out = p.part + ((int64_t)b * p.n_entries + e0) * VW;
 
   double x[3], v[3], sl[3], lenprod = 1.0;
@@ -122,12 +125,16 @@ __global__ void __launch_bounds__(kDtThreads) duffy_tensor_kernel(const DuffyTen
   };
 
   int m0[kDtAcc], m1[kDtAcc], m2[kDtAcc];
+  unsigned refused = 0;  // entries with a mode outside the box
   double acc[kDtAcc][VW];
 #pragma unroll
   for (int c = 0; c < kDtAcc; ++c) {
     const int i = tid + c * kDtThreads;
     int m = i < ne ? p.mode[e0 + i] : 0;
-    if ((unsigned)m >= (unsigned)(q * q * q)) m = 0;  // outside the contract: some entry's value
+    if ((unsigned)m >= (unsigned)(q * q * q)) {
+      m = 0;
+      refused |= 1u << c;
+    }
     m2[c] = m % q;
     m1[c] = m / q % q;
     m0[c] = m / (q * q);
@@ -221,16 +228,21 @@ __global__ void __launch_bounds__(kDtThreads) duffy_tensor_kernel(const DuffyTen
           acc[c][w] = fma(l0, sH[((size_t)(w * p.rows + row) * q + sel(a1)) * q + sel(a2)], acc[c][w]);
       }
     }
-    // (the next chunk's first barrier separates these reads from its sums)
-    __syncthreads();
+    __syncthreads();  // the next chunk overwrites sL0, sL1 and sG
   }
 #pragma unroll
   for (int c = 0; c < kDtAcc; ++c) {
     const int i = tid + c * kDtThreads;
     if (i < ne)
 #pragma unroll
-      for (int w = 0; w < VW; ++w) out[i * VW + w] = acc[c][w];
+      for (int w = 0; w < VW; ++w)
+        out[i * VW + w] = (refused >> c) & 1 ? __builtin_nan("") : acc[c][w];
   }
+}
+
+__global__ void __launch_bounds__(256) duffy_tensor_fill_kernel(int64_t n, double* __restrict__ part) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) part[i] = __builtin_nan("");
 }
 
 __global__ void __launch_bounds__(256)
@@ -261,12 +273,12 @@ static hipError_t launch_tensor_q(DuffyTensorParams p, int64_t max_entries, doub
   hipError_t e = hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      160 * 1024);
   if (e != hipSuccess) return e;
-  const int64_t per = kDtThreads * kDtAcc;
+  const int64_t per = kDtThreads * kDtAcc, n = p.n_entries * vw;
+  const dim3 flat((unsigned)((n + 255) / 256));
+  hipLaunchKernelGGL(duffy_tensor_fill_kernel, flat, dim3(256), 0, s, n, p.part);  // first sign block
   hipLaunchKernelGGL(fn, dim3((unsigned)p.n_targets, 8, (unsigned)((max_entries + per - 1) / per)),
                      dim3(kDtThreads), lds, s, p);
-  const int64_t n = p.n_entries * vw;
-  hipLaunchKernelGGL(duffy_tensor_sum_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n,
-                     p.part, out);
+  hipLaunchKernelGGL(duffy_tensor_sum_kernel, flat, dim3(256), 0, s, n, p.part, out);
   return hipGetLastError();
 }
 

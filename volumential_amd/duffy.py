@@ -41,6 +41,10 @@ def target_point_chunks(table, entry_ids, max_chunk=64):
     return order, np.asarray(starts, dtype=np.int64)
 
 
+# tail nodes of a rule that the build by sum factorization takes (a thread each)
+TENSOR_TAIL_NODES = 256
+
+
 def _tensor_values(L, table, entry_ids, regular_order, radial_order, stream):
     """3D values by sum factorization over the rule's axes
     (``vl1_duffy_build_tensor``): entries grouped by target point, the rule as
@@ -107,7 +111,8 @@ def duffy_values(table, entry_ids, regular_order, radial_order, stream=None,
     if not torch.cuda.is_available():
         raise RuntimeError("the Duffy table build runs on the GPU; no GPU is visible")
     L = _capi.lib()
-    if segmented and table.dim == 3 and np.size(entry_ids) and int(regular_order) <= 256:
+    if (segmented and table.dim == 3 and np.size(entry_ids)
+            and int(regular_order) <= TENSOR_TAIL_NODES):
         return _tensor_values(L, table, entry_ids, int(regular_order), int(radial_order), stream)
     nodes = quadrature.duffy_node_set(table.dim, int(regular_order), int(radial_order))
     entry_ids = np.asarray(entry_ids, dtype=np.int64)

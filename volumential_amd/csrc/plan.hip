@@ -2882,6 +2882,10 @@ int vl1_plan_tune(vl1_plan* pl, int form, const double* f, int64_t ldf, int n_rh
     return VL1_OK;
   }
   const bool multi_box = kCols / Rc > 1;
+  // the folded kernel knows the tile order only: the variants that differ in
+  // other bits are the same launch and take its time
+  const bool fold = uses_fold(pl, form, S, n_rhs);
+  float order_ms[2] = {-1.f, -1.f};
   hipEvent_t e0 = nullptr, e1 = nullptr;
   hipError_t e = hipEventCreate(&e0);
   if (e == hipSuccess) e = hipEventCreate(&e1);
@@ -2893,6 +2897,11 @@ int vl1_plan_tune(vl1_plan* pl, int form, const double* f, int64_t ldf, int n_rh
     // only the tile order is a choice
     if (form == VL1_FORM_SPLIT_I8 && (v & (kVarOneRow | kVarNoPhase))) continue;
     if ((v & kVarMorton) && !multi_box) continue;
+    float& same = order_ms[(v & kVarMorton) ? 1 : 0];
+    if (fold && same >= 0.f) {
+      if (times_ms) times_ms[v] = same;
+      continue;
+    }
     pl->forced_variant = v;
     rc = vl1_plan_contract(pl, form, n_rhs, y, ldy, opts, stream);  // warm (and schedule)
     if (rc != VL1_OK) break;
@@ -2905,6 +2914,7 @@ int vl1_plan_tune(vl1_plan* pl, int form, const double* f, int64_t ldf, int n_rh
     float ms = 0.f;
     if (e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
     ms /= reps;
+    same = ms;
     if (times_ms) times_ms[v] = ms;
     if (best < 0 || ms < best_ms) {
       best = v;

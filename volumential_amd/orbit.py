@@ -34,6 +34,7 @@ entry ids + values) map onto the same rows.
 
 from __future__ import annotations
 
+import itertools
 import math
 from dataclasses import dataclass
 from functools import lru_cache
@@ -210,18 +211,39 @@ def kernel_case_metadata(kernel, quad_order: int) -> ArithmeticCaseMetadata:
     return build_case_metadata(kernel.dim, quad_order, fixed, power)
 
 
+def _representatives_numpy(meta: ArithmeticCaseMetadata) -> np.ndarray:
+    q, dim = meta.quad_order, meta.dim
+    n, stride = q**dim, q ** np.arange(dim - 1, -1, -1)
+    out = []
+    for cid in meta.canonical_case_ids.tolist():
+        ids = np.array([cid * n * n], dtype=np.int64)
+        for gid in range(dim):  # the first group slowest
+            axes = np.flatnonzero(meta.case_axis_group[cid] == gid)
+            if axes.size:
+                alpha = group_alphabet(q, bool(np.any(meta.case_axis_sign[cid][axes] == 0)))
+                codes = np.array(list(itertools.combinations_with_replacement(range(alpha), axes.size)))
+                ids = np.add.outer(ids, (codes // q * n + codes % q) @ stride[axes]).ravel()
+        out.append(ids)
+    return np.concatenate(out)
+
+
 def enumerate_representatives(meta: ArithmeticCaseMetadata) -> np.ndarray:
     """Full entry ids of the canonical representatives in compact-row order.
 
-    ``orbit_arithmetic.py:748-790``.  Full id = ``case*n^2 + s*n + t``.
+    ``orbit_arithmetic.py:748-790``.  Full id = ``case*n^2 + s*n + t``.  Hosts
+    without the native library (tables are data there) take numpy.
     """
     from . import _capi
 
+    try:
+        L = _capi.lib()
+    except (RuntimeError, OSError):
+        return _representatives_numpy(meta)
     cases = np.ascontiguousarray(meta.canonical_case_ids, dtype=np.int32)
     sign = np.ascontiguousarray(meta.case_axis_sign[cases], dtype=np.int8)
     group = np.ascontiguousarray(meta.case_axis_group[cases], dtype=np.uint8)
     out = np.empty(meta.n_compact_entries, dtype=np.int64)
-    _capi.check(_capi.lib().vl1_orbit_representatives_host(
+    _capi.check(L.vl1_orbit_representatives_host(
         meta.dim, meta.quad_order, cases.size, cases.ctypes.data, sign.ctypes.data,
         group.ctypes.data, out.size, out.ctypes.data), "vl1_orbit_representatives_host")
     return out

@@ -35,7 +35,9 @@ constexpr bool fold_whole(int np, int nct, int g0, int g1, int g2, int g3) {
 // For a thread with outputs that came out infinite or NaN: each of its outputs
 // again, as the products of the densities' infinities and NaN with their entries
 // of the blocks, the signed infinity or NaN that the sum over sources has
-// (finite products do not matter).  Outputs without any keep what was written.
+// (finite products do not matter; a NaN ends the sum).  Outputs without any keep
+// what was written.  Slow and meant for few: 24 densities of 4096 boxes, 3D q = 6,
+// all NaN 1.6 ms (finite 1.2), all +inf 730.
 template <int NP>
 __device__ inline void fold_nonfinite(const FoldParams& p, const double* smem) {
   const int n_rc = (p.R + p.Rc - 1) / p.Rc;
@@ -53,12 +55,12 @@ __device__ inline void fold_nonfinite(const FoldParams& p, const double* smem) {
     double sum = 0.0;
     bool any = false;
     int64_t step = ti.step - 1;
-    for (int i = 0; i < ti.n_chunks; ++i) {
+    for (int i = 0; i < ti.n_chunks && sum == sum; ++i) {
       const uint32_t w = p.chunks[ti.chunk + i];
       if (!fold_chunk_first(w)) continue;
       ++step;
       const int z = fold_chunk_z(w), blk = f.rep_blk[fold_chunk_cls(w)] * f.n_rg;
-      for (int j = 0; j < 1 << fold_chunk_m(w); ++j) {
+      for (int j = 0; j < 1 << fold_chunk_m(w) && sum == sum; ++j) {
         const int src = p.step_src[(step * p.B + b) * NP + j];
         if (src == p.nb) continue;
         int J = 0;  // the slot's negative axes
@@ -67,7 +69,7 @@ __device__ inline void fold_nonfinite(const FoldParams& p, const double* smem) {
         const int t = row / p.nm * p.nm + reflect_node(f.dim, f.q, row % p.nm, J);
         const double* m = f.M + ((int64_t)(blk + t / f.rg_size) * f.MP + t % f.rg_size) * f.KP;
         const double eps = (__popc((unsigned)J & p.d.sp) & 1) ? -1.0 : 1.0;
-        for (int e = 0; e < 4 * p.d.kg; ++e) {
+        for (int e = 0; e < 4 * p.d.kg && sum == sum; ++e) {
           const double x = Xc[(((int64_t)src * p.d.kg + e / 4) * p.Rc + r) * 4 + e % 4];
           if (fabs(x) <= kFoldMax || (uint64_t)__double_as_longlong(x) == kFoldFinite) continue;
           const FoldSlot s = f.slots[e / 4 * 4 + ((e % 4) ^ ((e % 4) >> 1))];

@@ -162,9 +162,10 @@ struct FoldPlan {
   std::vector<int32_t> start, cls, src;  // src [entry][np], -1: none
 };
 
-// Folded basis of q^dim nodes (2 values per node if complex) for plans of n_tgt
-// target boxes; false: sizes the kernel does not take.
-bool fold_layout(FoldPlan& f, int dim, int q, int cplx, uint32_t sign_mask, int n_tgt);
+// Folded basis of q^dim nodes (2 values per node if complex); false: sizes the
+// kernel does not take.  `few_axes`: the basis with fewer folded axes that many
+// columns are faster in, false where there is none.
+bool fold_layout(FoldPlan& f, int dim, int q, int cplx, uint32_t sign_mask, bool few_axes = false);
 // Whether the tile kernel's 32-bit byte offsets reach all nb boxes and the zero
 // box at Rc densities per tile (a box holds kg K groups of 32 Rc bytes; a lane
 // reads up to one box past its own offset).

@@ -22,7 +22,7 @@ hipError_t fold_launch_2d(const FoldParams& p, int nct, const int g[4], hipStrea
     case 1 << 20 | fold_key(8, 8, 8, 8): return pick<1, 8, 8, 8, 8>(p, nct, s);  // 3D q = 3, unfolded
     case 2 << 20 | fold_key(1, 1, 1, 1): return pick<2, 1, 1, 1, 1>(p, nct, s);  // 2D q = 2 complex, 3D q = 2
     case 4 << 20 | fold_key(1, 1, 1, 1): return pick<4, 1, 1, 1, 1>(p, nct, s);  // 2D q = 3, 4; 3D q = 2 complex
-    case 4 << 20 | fold_key(4, 2, 1, 1): return pick<4, 4, 2, 1, 1>(p, nct, s);  // 2D q = 5; 3D q = 3
+    case 4 << 20 | fold_key(4, 2, 1, 1): return pick<4, 4, 2, 1, 1>(p, nct, s);  // 2D q = 5
     case 4 << 20 | fold_key(4, 4, 4, 4): return pick<4, 4, 4, 4, 4>(p, nct, s);  // 2D q = 6, 7, 8
     case 4 << 20 | fold_key(6, 4, 2, 2): return pick<4, 6, 4, 2, 2>(p, nct, s);  // 3D q = 3 complex
     default: return fold_launch_2dc(p, nct, g, s);

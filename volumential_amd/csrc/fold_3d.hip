@@ -1,4 +1,5 @@
-// Instances of the folded tile kernel with eight parities, even orders.
+// Instances of the folded tile kernel with eight parities, even orders (and
+// order 3).
 #include "fold_kernel.h"
 
 namespace vl1 {
@@ -17,6 +18,7 @@ hipError_t pick(const FoldParams& p, int nct, hipStream_t s) {
 
 hipError_t fold_launch_3d(const FoldParams& p, int nct, const int g[4], hipStream_t s) {
   switch (p.d.np << 20 | fold_key(g[0], g[1], g[2], g[3])) {
+    case 8 << 20 | fold_key(2, 1, 1, 1): return pick<8, 2, 1, 1, 1>(p, nct, s);  // q = 3
     case 8 << 20 | fold_key(2, 2, 2, 2): return pick<8, 2, 2, 2, 2>(p, nct, s);  // q = 4
     case 8 << 20 | fold_key(8, 8, 8, 8): return pick<8, 8, 8, 8, 8>(p, nct, s);  // q = 6
     case 8 << 20 | fold_key(16, 16, 16, 16): return pick<8, 16, 16, 16, 16>(p, nct, s);  // q = 8

@@ -30,7 +30,7 @@ int parity_groups(int dim, int q, int vw, int nf, int p) {
 
 }  // namespace
 
-bool fold_layout(FoldPlan& f, int dim, int q, int cplx, uint32_t sign_mask, int n_tgt) {
+bool fold_layout(FoldPlan& f, int dim, int q, int cplx, uint32_t sign_mask, bool few_axes) {
   const int vw = cplx ? 2 : 1;
   // fold as many axes as pay: the products of a class whose nonzero axes are
   // all folded (2^m sums, each with the blocks p -> p ^ s) against one fold
@@ -52,13 +52,11 @@ bool fold_layout(FoldPlan& f, int dim, int q, int cplx, uint32_t sign_mask, int 
   for (int k = 1; k <= dim; ++k)
     if (cost(k) < cost(nf)) nf = k;
   // 3D q = 3: all axes folded leave parities of 8 to 1 entries, so that most of
-  // a chunk's waves and loads serve padding.  Many tiles are bound by that
-  // work: fewer folds, more products.  us at 3 / 2 / 0 folded axes, real, 64
-  // densities: 32768 boxes 4283 / 3209 / 2131 (the digit kernel at 5 slices 2663),
-  // 4096 boxes 526 / 404 / 301; one density 83 / 78 / 90 and 28 / 29 / 41, a tile's
-  // chain being longer.  Complex at 3 / 2: 32768 boxes 7168 / 6069 and 133 / 124,
-  // 4096 boxes 865 / 736 and 40 / 45.
-  if (dim == 3 && q == 3) nf = n_tgt >= 16384 ? (cplx ? 2 : 0) : (cplx ? 3 : 2);
+  // a chunk's waves and loads serve padding (plan_fold says what it costs)
+  if (few_axes) {
+    if (dim != 3 || q != 3) return false;
+    nf = cplx ? 2 : 0;
+  }
   FoldDims d;
   d.nf = nf;
   d.np = 1 << nf;

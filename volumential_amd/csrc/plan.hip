@@ -1264,7 +1264,8 @@ struct vl1_plan {
   bool stream_colmax = false;
   std::map<int, TileSchedule*> schedules;  // by 2 Rc + (Morton-only order)
   FoldPlan* fold = nullptr;                // folded FP64 form (null: the dense one)
-  std::map<int, FoldSchedule*> fold_schedules;  // by 2 B + (Morton-only order)
+  FoldPlan* fold_many = nullptr;           // ... for many columns (null: none)
+  std::map<int, FoldSchedule*> fold_schedules;  // by 4 B + 2 (Morton-only order) + (fold_many)
   uint32_t fold_ready = 0;  // fold_bit of the calls prepared on it
   int max_sources = 0;      // list-1 sources of a target
   bool unfolded = false;    // a call ran on the general kernels
@@ -1283,6 +1284,7 @@ struct vl1_plan {
     for (auto& kv : schedules) delete kv.second;
     for (auto& kv : fold_schedules) delete kv.second;
     delete fold;
+    delete fold_many;
     for (auto& kv : A_by_slices) delete kv.second;
     for (auto& kv : A8_by_slices) delete kv.second;
     for (DevBuf* b : retired) delete b;
@@ -1424,8 +1426,7 @@ static int build_schedule(vl1_plan* pl, int Rc, bool morton_only, TileSchedule**
 
 // Each target's classes; a repeated source of one class slot counts once, as
 // in the dense form's schedule.
-static void fold_targets(vl1_plan* pl) {
-  FoldPlan& f = *pl->fold;
+static void fold_targets(vl1_plan* pl, FoldPlan& f) {
   if (!f.start.empty()) return;
   const int np = f.d.np;
   std::vector<std::pair<int, int64_t>> ent;  // (class x np + slot, pair)
@@ -1460,16 +1461,20 @@ static void fold_targets(vl1_plan* pl) {
 // with the lists in hash order.  Tiles are then dealt out longest first, runs of
 // equal length in eighths to the XCDs (workgroup i runs on XCD i % 8), which
 // keeps neighbours in one L2.
-static int build_fold_schedule(vl1_plan* pl, int B, bool morton_only, FoldSchedule** out,
-                               hipStream_t s) {
-  const int key = B * 2 + (morton_only ? 1 : 0);
+static int fold_key_of(const vl1_plan* pl, const FoldPlan* f, int B, bool morton_only) {
+  return B * 4 + (morton_only ? 2 : 0) + (f == pl->fold_many ? 1 : 0);
+}
+
+static int build_fold_schedule(vl1_plan* pl, FoldPlan* f, int B, bool morton_only,
+                               FoldSchedule** out, hipStream_t s) {
+  const int key = fold_key_of(pl, f, B, morton_only);
   auto it = pl->fold_schedules.find(key);
   if (it != pl->fold_schedules.end()) {
     *out = it->second;
     return VL1_OK;
   }
-  fold_targets(pl);
-  const FoldPlan& fp = *pl->fold;
+  fold_targets(pl, *f);
+  const FoldPlan& fp = *f;
   const int np = fp.d.np;
   std::vector<int> rank(pl->n_tgt, 0);  // of a target's class list among the different ones
   if (B > 1 && !morton_only) {
@@ -1768,10 +1773,12 @@ static hipError_t expand_plan_blocks(const vl1_payload* pay, const vl1_plan* pl,
 // appended to `keys`.  Null for boxes the tile kernel does not take and trees
 // beyond its 32-bit byte offsets at one density per tile: the dense form runs.
 static std::unique_ptr<FoldPlan> fold_classes(const vl1_plan* pl, const vl1_payload* pay, bool split,
-                                              const std::vector<int64_t>& key_vid, BlockList& keys) {
+                                              const std::vector<int64_t>& key_vid, BlockList& keys,
+                                              bool few_axes) {
   const int dim = pl->dim;
   auto f = std::unique_ptr<FoldPlan>(new FoldPlan());
-  if (!fold_layout(*f, dim, pay->q, pl->cplx, (uint32_t)pay->sign_mask, pl->n_tgt)) return nullptr;
+  if (!fold_layout(*f, dim, pay->q, pl->cplx, (uint32_t)pay->sign_mask, few_axes))
+    return nullptr;
   if (!fold_fits(f->d, pl->nboxes, 1)) return nullptr;
   // blocks of a level: the table level, or the split's source level
   auto level_key = [&](int k) {
@@ -1827,11 +1834,12 @@ static std::unique_ptr<FoldPlan> fold_classes(const vl1_plan* pl, const vl1_payl
 // representative or a representative not its own along an axis where its case
 // vector is zero (descriptors without the reflection symmetry of a list-1
 // table, middle-node values of a derivative table).
-static hipError_t fold_tables(vl1_plan* pl, std::unique_ptr<FoldPlan> f, int q, hipStream_t s) {
+static hipError_t fold_tables(vl1_plan* pl, std::unique_ptr<FoldPlan> f, int q, FoldPlan** out,
+                              hipStream_t s) {
   int32_t flag = 0;
   const hipError_t e = fold_build_launch(*f, pl->dim, q, pl->M.as<double>(), pl->MP, pl->KP, pl->n_rg,
                                          pl->rg_size, &flag, s);
-  if (e == hipSuccess && !flag) pl->fold = f.release();
+  if (e == hipSuccess && !flag) *out = f.release();
   return e;
 }
 
@@ -2172,10 +2180,13 @@ static int plan_create(vl1_plan** out, const vl1_payload* pay, const vl1_plan_de
   if (e == hipSuccess) e = upload(pl->box_disp, bdisp.data(), bdisp.size() * 8, s);
   if (e == hipSuccess && pl->n_blocks > 0) {
     BlockList keys{pl->blk_case, pl->blk_lev, pl->blk_alpha, pl->blk_disp, pl->blk_h};
-    std::unique_ptr<FoldPlan> fold;
-    if (one_vid && !pay->dense_kind) fold = fold_classes(pl, pay, split, key_vid, keys);
+    std::unique_ptr<FoldPlan> fold, many;
+    if (one_vid && !pay->dense_kind) fold = fold_classes(pl, pay, split, key_vid, keys, false);
+    if (fold) many = fold_classes(pl, pay, split, key_vid, keys, true);
     e = expand_plan_blocks(pay, pl, sp, H, keys, pl->MP, pl->KP, pl->n_rg, pl->rg_size, pl->M, s);
-    if (e == hipSuccess && fold) e = fold_tables(pl, std::move(fold), pay->q, s);
+    if (e == hipSuccess && fold) e = fold_tables(pl, std::move(fold), pay->q, &pl->fold, s);
+    if (e == hipSuccess && pl->fold && many)
+      e = fold_tables(pl, std::move(many), pay->q, &pl->fold_many, s);
     if (e == hipSuccess && !pl->fold) e = pl->MF.alloc(pl->M.bytes);
     if (e == hipSuccess && !pl->fold) {
       const int64_t total = (int64_t)pl->n_blocks * pl->MP * pl->KP;
@@ -2308,6 +2319,7 @@ static int i8_check_range(const vl1_plan* pl, const TileSchedule* sch, int S) {
 struct Prepared {
   int S = 0;
   TileSchedule* sch = nullptr;
+  FoldPlan* form = nullptr;  // the folded basis (with `fold`)
   FoldSchedule* fold = nullptr;
   FoldTile tile;
 };
@@ -2332,8 +2344,24 @@ static bool uses_fold(const vl1_plan* pl, int form, int S, int n_rhs) {
   return form != VL1_FORM_SPLIT_I8 || i8_sums_fit(steps, pl->KP, S);
 }
 
-static FoldTile plan_tile(const vl1_plan* pl, int n_rhs, int nct = 0) {
-  return fold_tile(pl->fold->d, pl->nboxes, pl->n_tgt, n_rhs, nct);
+// The folded basis of a call.  In 3D order 3 the one with all axes folded pads so
+// much that split calls of many columns (target boxes x densities) were slower
+// than the digit kernels; they take the one with fewer, whose rounding errors
+// are up to twice as large (9e-16 against 4e-16; the digits' 1e-11), so that FP64
+// calls do not.  us, 5 int8 slices / all axes / fewer: real (none folded), uniform
+// trees, 32768 boxes, 64 densities 2663 / 4283 / 2104, one 101 / 83 / 90; 4096 boxes, 64
+// densities 346 / 506 / 301, 8 densities 82 / 82 / 75, 4 59 / 45 / 66; graded, 14246
+// boxes, one density - / 84 / 157, 4 - / 195 / 169.  Complex (two folded): 4096
+// boxes, 64 densities 624 / 865 / 736, 4 100 / 70 / 77.
+constexpr int64_t kManyColumns = 49152;
+static FoldPlan* plan_fold(const vl1_plan* pl, int form, int n_rhs) {
+  const bool many = pl->fold_many && form != VL1_FORM_F64 &&
+                    (int64_t)pl->n_tgt * std::min(n_rhs, kCols) >= kManyColumns;
+  return many ? pl->fold_many : pl->fold;
+}
+
+static FoldTile plan_tile(const vl1_plan* pl, const FoldPlan* f, int n_rhs, int nct = 0) {
+  return fold_tile(f->d, pl->nboxes, pl->n_tgt, n_rhs, nct);
 }
 
 // Checks, then builds (allocating) the slice set and tile schedule this
@@ -2356,23 +2384,29 @@ static int plan_prepare(vl1_plan* pl, int form, int n_rhs, const vl1_split_opts*
   }
   if (fold) {
     pl->fold_ready |= fold_bit(form, S);
-    out->tile = plan_tile(pl, n_rhs);
+    out->form = plan_fold(pl, form, n_rhs);
+    out->tile = plan_tile(pl, out->form, n_rhs);
     if (pl->fold_schedules.empty()) pl->fold_rc = Rc;
-    rc = build_fold_schedule(pl, out->tile.B, morton, &out->fold, s);
+    rc = build_fold_schedule(pl, out->form, out->tile.B, morton, &out->fold, s);
   } else {
     pl->unfolded = true;
     rc = build_schedule(pl, Rc, morton, &out->sch, s);
     if (rc == VL1_OK && form == VL1_FORM_SPLIT_I8) rc = i8_check_range(pl, out->sch, S);
   }
-  // a plan that serves both kernels keeps the tiles of every density count for
-  // both: an allocation-free call takes any prepared form at any prepared count
+  // a plan that serves several kernels or bases keeps the tiles of every
+  // density count for all of them: an allocation-free call takes any prepared
+  // form at any prepared count
   pl->prepared_rhs.insert(Rc);
-  if (rc != VL1_OK || !pl->fold || !pl->unfolded) return rc;
+  if (rc != VL1_OK || !pl->fold) return rc;
+  const bool many = pl->fold_many && (pl->fold_ready & ~fold_bit(VL1_FORM_F64, 0)) != 0;
+  if (!pl->unfolded && !many) return rc;
   for (int R : pl->prepared_rhs) {
     FoldSchedule* fs = nullptr;
     TileSchedule* ts = nullptr;
-    rc = build_fold_schedule(pl, plan_tile(pl, R).B, false, &fs, s);
-    if (rc == VL1_OK) rc = build_schedule(pl, R, false, &ts, s);
+    rc = build_fold_schedule(pl, pl->fold, plan_tile(pl, pl->fold, R).B, false, &fs, s);
+    if (rc == VL1_OK && many)
+      rc = build_fold_schedule(pl, pl->fold_many, plan_tile(pl, pl->fold_many, R).B, false, &fs, s);
+    if (rc == VL1_OK && pl->unfolded) rc = build_schedule(pl, R, false, &ts, s);
     if (rc != VL1_OK) return rc;
   }
   return VL1_OK;
@@ -2392,18 +2426,18 @@ struct Staging {
 
 // Bytes of staging for (form, S, R) laid out in one region, each part
 // 256-byte aligned: split X | colscale | nmdot, FP64 XF | nmdot (folded: X | dl
-// with `tile`).
+// with the basis and tile of `folded`).
 static size_t staging_layout(const vl1_plan* pl, int form, int S, int R, int n_tiles, char* base,
-                             Staging* st, const FoldTile* tile = nullptr) {
+                             Staging* st, const Prepared* folded = nullptr) {
   auto al = [](size_t b) { return (b + 255) / 256 * 256; };
   const size_t cols = (size_t)pl->nboxes * R;
   size_t off = 0;
   Staging t;
-  if (tile) {
+  if (folded) {
     t.XF = reinterpret_cast<double*>(base);
-    off = al(fold_x_size(pl->fold->d, *tile, pl->nboxes, R) * 8);
+    off = al(fold_x_size(folded->form->d, folded->tile, pl->nboxes, R) * 8);
     t.nmdot = reinterpret_cast<double*>(base + off);
-    off += al(fold_dl_size(*tile, pl->nboxes, R) * 8);
+    off += al(fold_dl_size(folded->tile, pl->nboxes, R) * 8);
     if (st) *st = t;
     return off;
   }
@@ -2431,10 +2465,10 @@ static size_t staging_layout(const vl1_plan* pl, int form, int S, int R, int n_t
   return off;
 }
 
-static int fold_stage(vl1_plan* pl, const FoldTile& tile, const double* f, int64_t ldf, int R,
+static int fold_stage(vl1_plan* pl, const Prepared& pr, const double* f, int64_t ldf, int R,
                       const Staging& st, hipStream_t s) {
   const hipError_t e = fold_stage_launch(
-      *pl->fold, tile, pl->nboxes, R, f, ldf, pl->mode_point.as<int32_t>(),
+      *pr.form, pr.tile, pl->nboxes, R, f, ldf, pl->mode_point.as<int32_t>(),
       pl->box_starts.as<int32_t>(), pl->box_alpha.as<double>(), pl->box_disp.as<double>(),
       pl->payload->nmlz.as<double>(), pl->log_disp, st.XF, st.nmdot, s);
   if (e != hipSuccess) return fail(VL1_E_HIP, std::string("staging launch: ") + hipGetErrorString(e));
@@ -2450,7 +2484,7 @@ constexpr int64_t kMaxThreads = 0xffffffff;  // of one launch
 
 static int fold_contract(vl1_plan* pl, const Prepared& pr, int R, double* y, int64_t ldy,
                          const Staging& st, hipStream_t s, double* est) {
-  const FoldPlan& f = *pl->fold;
+  const FoldPlan& f = *pr.form;
   FoldParams p{};
   p.d = f.d;
   p.B = pr.tile.B;
@@ -2696,7 +2730,7 @@ int vl1_plan_stage(vl1_plan* pl, int form, const double* f, int64_t ldf, int n_r
   // the largest buffer first: a failed allocation then leaves the others
   // untouched
   if (pr.fold) {
-    e = pl->grow(pl->XF, fold_x_size(pl->fold->d, pr.tile, pl->nboxes, R) * 8);
+    e = pl->grow(pl->XF, fold_x_size(pr.form->d, pr.tile, pl->nboxes, R) * 8);
     if (e == hipSuccess && pl->log_disp)
       e = pl->grow(pl->nmdot, fold_dl_size(pr.tile, pl->nboxes, R) * 8);
   } else if (form == VL1_FORM_SPLIT_I8) {
@@ -2715,7 +2749,7 @@ int vl1_plan_stage(vl1_plan* pl, int form, const double* f, int64_t ldf, int n_r
   }
   if (e != hipSuccess) return fail(VL1_E_HIP, std::string("vl1_plan_stage alloc: ") + hipGetErrorString(e));
   const Staging st = plan_staging(pl);
-  rc = pr.fold ? fold_stage(pl, pr.tile, f, ldf, R, st, s)
+  rc = pr.fold ? fold_stage(pl, pr, f, ldf, R, st, s)
                : stage_launch(pl, form, S, f, ldf, R, st, s);
   if (rc != VL1_OK) return rc;
   pl->staged_form = form;
@@ -2799,10 +2833,11 @@ int vl1_plan_eval_noalloc(vl1_plan* pl, int form, const double* f, int64_t ldf, 
   if (fold) {
     // either tile width serves: a count prepared at another multiple of 64
     // may have taken the other one
-    pr.tile = plan_tile(pl, n_rhs);
+    pr.form = plan_fold(pl, form, n_rhs);
+    pr.tile = plan_tile(pl, pr.form, n_rhs);
     for (int k = 0; k < 2 && !pr.fold; ++k) {
-      if (k) pr.tile = plan_tile(pl, n_rhs, 3 - pr.tile.nct);
-      auto it = pl->fold_schedules.find(pr.tile.B * 2 + (morton ? 1 : 0));
+      if (k) pr.tile = plan_tile(pl, pr.form, n_rhs, 3 - pr.tile.nct);
+      auto it = pl->fold_schedules.find(fold_key_of(pl, pr.form, pr.tile.B, morton));
       if (it != pl->fold_schedules.end()) pr.fold = it->second;
     }
   } else {
@@ -2836,13 +2871,13 @@ int vl1_plan_eval_noalloc(vl1_plan* pl, int form, const double* f, int64_t ldf, 
     // as many densities at a time as the array holds (all of them but for
     // trees of a few boxes with very many densities)
     int step = n_rhs;
-    while (step > 64 && staging_layout(pl, form, S, step, 0, nullptr, nullptr, &pr.tile) > kScratchArray)
+    while (step > 64 && staging_layout(pl, form, S, step, 0, nullptr, nullptr, &pr) > kScratchArray)
       step = (step / 2 + 63) / 64 * 64;
-    if (staging_layout(pl, form, S, step, 0, static_cast<char*>(base), &st, &pr.tile) > kScratchArray)
+    if (staging_layout(pl, form, S, step, 0, static_cast<char*>(base), &st, &pr) > kScratchArray)
       return fail(VL1_E_UNSUPPORTED, "vl1_plan_eval_noalloc: staging exceeds the scratch array");
     for (int r = 0; r < n_rhs && rc == VL1_OK; r += step) {
       const int nr = std::min(step, n_rhs - r);
-      rc = fold_stage(pl, pr.tile, f + r * ldf, ldf, nr, st, s);
+      rc = fold_stage(pl, pr, f + r * ldf, ldf, nr, st, s);
       if (rc == VL1_OK) rc = fold_contract(pl, pr, nr, y + r * ldy, ldy, st, s, est ? est + 2 * r : est);
     }
     return rc;
@@ -2967,7 +3002,7 @@ int vl1_plan_fold_tile_host(int dim, int q, int is_complex, int64_t n_boxes, int
     return fail(VL1_E_ARG, "vl1_plan_fold_tile_host: bad argument");
   for (int k = 0; k < 5; ++k) out5[k] = 0;
   FoldPlan f;
-  if (!fold_layout(f, dim, q, is_complex != 0, 0, (int)n_tgt_boxes) || !fold_fits(f.d, (int)n_boxes, 1)) return VL1_OK;
+  if (!fold_layout(f, dim, q, is_complex != 0, 0) || !fold_fits(f.d, (int)n_boxes, 1)) return VL1_OK;
   const FoldTile t = fold_tile(f.d, (int)n_boxes, (int)n_tgt_boxes, n_rhs);
   out5[0] = 1;
   out5[1] = 16 * t.nct;
@@ -2998,7 +3033,8 @@ int vl1_plan_stats(const vl1_plan* pl, int64_t* out5) {
   out5[3] = pl->n_keys;
   int64_t bytes = (int64_t)(pl->M.bytes + pl->MF.bytes + pl->rowscale.bytes + pl->X.bytes +
                             pl->XF.bytes + pl->colscale.bytes + pl->nmdot.bytes +
-                            pl->mode_point.bytes + (pl->fold ? pl->fold->A.bytes : 0));
+                            pl->mode_point.bytes + (pl->fold ? pl->fold->A.bytes : 0) +
+                            (pl->fold_many ? pl->fold_many->A.bytes : 0));
   for (auto& kv : pl->A_by_slices) bytes += (int64_t)kv.second->bytes;
   for (const DevBuf* b : pl->retired) bytes += (int64_t)b->bytes;
   out5[4] = bytes;

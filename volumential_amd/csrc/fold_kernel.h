@@ -39,9 +39,9 @@ constexpr bool fold_whole(int np, int nct, int g0, int g1, int g2, int g3) {
 // what was written.  Slow and meant for few: 24 densities of 4096 boxes, 3D q = 6,
 // all NaN 1.6 ms (finite 1.2), all +inf 730.
 template <int NP>
-__device__ inline void fold_nonfinite(const FoldParams& p, const double* smem) {
+__device__ inline void fold_nonfinite(const FoldParams& p, const double* smem, int wg) {
   const int n_rc = (p.R + p.Rc - 1) / p.Rc;
-  const int i8 = (int)(blockIdx.x / 8), bt = i8 / n_rc * 8 + (int)(blockIdx.x % 8), rcx = i8 % n_rc;
+  const int i8 = wg / 8, bt = i8 / n_rc * 8 + wg % 8, rcx = i8 % n_rc;
   const FoldTileInfo& ti = p.tiles[bt];
   const double* log_sums = smem + p.slot_doubles + 32 * NP * 2 + 64 * NP;
   const FoldBlocks& f = *p.blocks;
@@ -466,6 +466,10 @@ __global__ void __launch_bounds__(64 * NP, G0 <= 8 ? 4 : 2) fold_f64_kernel(cons
   const int n_rc = (p.R + p.Rc - 1) / p.Rc;
   const int i = (int)(blockIdx.x / 8), bt = i / n_rc * 8 + (int)(blockIdx.x % 8), rcx = i % n_rc;
   if (bt >= p.n_box_tiles) return;  // uniform over the workgroup
+  if (threadIdx.x == 0) {           // for the end of the kernel, out of the registers
+    reinterpret_cast<uint64_t*>(fold_smem)[0] = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+    reinterpret_cast<int*>(fold_smem)[2] = (int)blockIdx.x;
+  }
   // waves 0-3 and 4-7 pair large with small parities on a SIMD (odd orders)
   const int pout = NP == 8 ? (0x35674210 >> (4 * wave)) & 7 : wave;
   int grow = 0;  // groups before this parity
@@ -474,27 +478,29 @@ __global__ void __launch_bounds__(64 * NP, G0 <= 8 ? 4 : 2) fold_f64_kernel(cons
   constexpr bool WHOLE = fold_whole(NP, NCT, G0, G1, G2, G3);
   double finite;
   if constexpr (G0 == G1 && G1 == G2 && G2 == G3) {
-    finite = fold_run<NP, NCT, G0, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
+    finite = fold_run<NP, NCT, G0, G0, WHOLE>(p, fold_smem + 2, bt, rcx, pout, grow);
   } else {
     // the loops hold the same barriers, so waves may run different ones
     const int odd = __popc(pout);
-    if (odd == 0) finite = fold_run<NP, NCT, G0, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
-    else if (odd == 1) finite = fold_run<NP, NCT, G1, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
-    else if (odd == 2) finite = fold_run<NP, NCT, G2, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
-    else if constexpr (NP == 8) finite = fold_run<NP, NCT, G3, G0, WHOLE>(p, fold_smem, bt, rcx, pout, grow);
+    if (odd == 0) finite = fold_run<NP, NCT, G0, G0, WHOLE>(p, fold_smem + 2, bt, rcx, pout, grow);
+    else if (odd == 1) finite = fold_run<NP, NCT, G1, G0, WHOLE>(p, fold_smem + 2, bt, rcx, pout, grow);
+    else if (odd == 2) finite = fold_run<NP, NCT, G2, G0, WHOLE>(p, fold_smem + 2, bt, rcx, pout, grow);
+    else if constexpr (NP == 8) finite = fold_run<NP, NCT, G3, G0, WHOLE>(p, fold_smem + 2, bt, rcx, pout, grow);
   }
   if (finite != 0.0) {
     // the arguments read again: kept in registers for this they spill others of
     // the loop (4 to 10 % slower)
-    auto args = (uintptr_t)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(args));
+    const auto* at = reinterpret_cast<const int*>(fold_smem);
+    const int lo = __builtin_amdgcn_readfirstlane(at[0]), hi = __builtin_amdgcn_readfirstlane(at[1]);
+    const uint64_t args = (uint64_t)(unsigned)hi << 32 | (unsigned)lo;
     typedef const __attribute__((address_space(4))) uint32_t* scalar_ptr;
     struct Words {
       uint32_t w[sizeof(FoldParams) / 4];
     } words;
 #pragma unroll
     for (size_t k = 0; k < sizeof(FoldParams) / 4; ++k) words.w[k] = ((scalar_ptr)args)[k];
-    fold_nonfinite<NP>(__builtin_bit_cast(FoldParams, words), fold_smem);
+    fold_nonfinite<NP>(__builtin_bit_cast(FoldParams, words), fold_smem + 2,
+                       __builtin_amdgcn_readfirstlane(at[2]));
   }
 }
 
@@ -514,7 +520,7 @@ hipError_t launch_fold(const FoldParams& p, hipStream_t s) {
   FoldParams q = p;
   const int out_cols = fold_whole(NP, NCT, G0, G1, G2, G3) ? 16 * NCT : 16;
   q.slot_doubles = std::max(kFoldUnits * NP * NCT * 64, p.d.rows4 * (out_cols + 1));
-  const size_t doubles = (size_t)q.slot_doubles + 32 * NP * 2 + 64 * NP + 3 * 16 * NCT;
+  const size_t doubles = 2 + (size_t)q.slot_doubles + 32 * NP * 2 + 64 * NP + 3 * 16 * NCT;
   const int grid = (p.n_box_tiles + 7) / 8 * 8 * ((p.R + p.Rc - 1) / p.Rc);
   hipLaunchKernelGGL(fn, dim3(grid), dim3(64 * NP), doubles * sizeof(double), s, q);
   return hipGetLastError();

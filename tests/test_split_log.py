@@ -59,7 +59,7 @@ def test_relative_error(split_logs, what):
     elif what == "closest to 1":
         x = 1.0 + 10.0 ** rng.uniform(-15, -2, n) * rng.choice([-1, 1], n)
     else:  # ends of the table's intervals and of the octave
-        ends = np.concatenate([0.5 + np.arange(129) / 256, [np.sqrt(0.5)]])
+        ends = np.concatenate([0.5 + np.arange(129) / 256, 1 + np.arange(129) / 128, [np.sqrt(0.5)]])
         x = np.concatenate([ends * s for s in (1, 2, 4, 0.125)])
         x = np.concatenate([x, np.nextafter(x, 0), np.nextafter(x, 9)])
     y, ref = split_logs(x), np.log(x.astype(np.longdouble))

@@ -23,7 +23,7 @@
 // number.  The series coefficients are kernel arguments, so that a term is one
 // instruction with a scalar operand; from LDS each wave took 32 bytes per lane
 // and term, and the LDS return path (128 bytes per clock and CU) was the bound:
-// 2D, 4096 boxes of 36 points, k = 40, one density 509 us, 141 us so
+// 2D, 4096 boxes of 36 points, k = 40, one density 509 us, 138 us so
 // (251 us with the library's log).
 // A lane takes four sources at a time for the same coefficient.  Where the
 // imaginary parts are a quarter of the real log series (real k, order 1), that

@@ -2330,7 +2330,7 @@ struct Prepared {
 // Measured at S = 5, split against folded, us per call: int8 3D q = 6, 32768
 // boxes, 64 densities 31225 / 22010; int8 2D q = 6 complex per-level, 12919
 // boxes, 16 densities 1313 / 441; int8 fused Helmholtz split, 16384 boxes, 16
-// densities 604 / 491; BF16 3D q = 4, 4096 boxes, 20 densities 1157 / 217.
+// densities 604 / 491; BF16 3D q = 4, 4096 boxes, 20 densities 1157 / 209.
 // Below 5 slices a caller asks for the split itself, its error included.
 // Calls whose int8 sums might leave int32 stay with the int8 form, which
 // refuses them by its own schedule (i8_check_range).
